@@ -60,11 +60,60 @@ __device__ __forceinline__ void wave_lds_sync()
 }
 
 // ---- deterministic reductions ---------------------------------------------
+// One step of a butterfly sum: v plus the v of lane ^ OFF, the steps taken from
+// 32 down to 1.  The exchanges stay inside the vector unit (half and row swaps,
+// rotations of a 16-lane row, quad permutations) instead of passing through the
+// LDS crossbar; once the larger offsets are summed v repeats every 2 * OFF
+// lanes, so a rotation by OFF reaches the partner's value.
+template <int OFF>
+__device__ __forceinline__ void butterfly_pair(unsigned v, unsigned& a, unsigned& b)
+{
+    if constexpr (OFF == 32 || OFF == 16)
+    {
+        const auto both = OFF == 32 ? __builtin_amdgcn_permlane32_swap(v, v, false, false)
+                                    : __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        a = both[0];
+        b = both[1];
+    }
+    else
+    {
+        constexpr int ctrl = OFF == 8 ? 0x128 : OFF == 4 ? 0x124 : OFF == 2 ? 0x4e : 0xb1;
+        a = v;
+        b = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), ctrl, 0xf, 0xf, false));
+    }
+}
+
+template <int OFF, typename T>
+__device__ __forceinline__ T butterfly_add(T v)
+{
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "butterfly word");
+    if constexpr (sizeof(T) == 4)
+    {
+        unsigned a, b;
+        butterfly_pair<OFF>(__builtin_bit_cast(unsigned, v), a, b);
+        return __builtin_bit_cast(T, a) + __builtin_bit_cast(T, b);
+    }
+    else
+    {
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+        unsigned al, bl, ah, bh;
+        butterfly_pair<OFF>(static_cast<unsigned>(u), al, bl);
+        butterfly_pair<OFF>(static_cast<unsigned>(u >> 32), ah, bh);
+        return __builtin_bit_cast(T, (static_cast<unsigned long long>(ah) << 32) | al) +
+               __builtin_bit_cast(T, (static_cast<unsigned long long>(bh) << 32) | bl);
+    }
+}
+
+// Sum over the wavefront in every lane, offsets 32, 16, ... 1 in turn.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)
 {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+    v = butterfly_add<32>(v);
+    v = butterfly_add<16>(v);
+    v = butterfly_add<8>(v);
+    v = butterfly_add<4>(v);
+    v = butterfly_add<2>(v);
+    v = butterfly_add<1>(v);
     return v;
 }
 
