@@ -29,7 +29,9 @@
 #include <deque>
 #include <string>
 
+#include "cg_rules.hpp"
 #include "dia.hpp"
+#include "persist.hpp"
 #include "plan_cache.hpp"
 #include "solver_internal.hpp"
 #include "spmv_kernels.hpp"
@@ -838,9 +840,6 @@ __global__ __launch_bounds__(kBlock) void k_factor_upper_dia(int64_t rows, DiaAr
 // an odd iteration (every chunk of iterations ends on one) a solve can
 // continue in that form.
 
-constexpr int kCounterRestart = 0;  // SolverState::counters slot: a single-reduction restart happened
-constexpr int kCgValues = 4;        // r.r, r.u, w.u, u.s
-
 __host__ __device__ inline double* cg_region(double* partials, int par)
 {
     return partials + kPartialsRes + (par == 1 ? 0 : kCgValues * kMaxPartials);
@@ -871,61 +870,30 @@ __device__ __forceinline__ int cg_decision(SolverState* st, const double* in, in
     const double delta = red[NV - 2];
     const double us = red[NV - 1];
     const int completed = st->iter[1 - par] + 1;
-    const double tol = completed != 0   ? st->tol
-                       : st->tol_rule   ? st->abs_tol + st->rel_tol * sqrt(rr)
-                                        : fmax(st->abs_tol, st->rel_tol * sqrt(rr));
-    int code = kRunning;
-    beta = 0.0;
-    alpha = 0.0;
-    double den = delta;
-    if (!isfinite(rr) || rr < 0.0) code = completed == 0 ? kInitNonFinite : kNonFinite;
-    else if (sqrt(rr) <= tol) code = kConverged;
-    else if (completed == 0 && st->bad_row != ~0ull) code = kBadDiagonal;
-    else if (completed >= st->max_iterations) code = kIterationLimit;
-    else
-    {
-        if (completed > 0)
-        {
-            const double gamma_prev = st->rho[1 - par];
-            if (gamma_prev == 0.0 && gamma == 0.0) beta = 0.0;
-            else if (isfinite(gamma_prev) && isfinite(gamma) && gamma_prev > 0.0 && gamma > 0.0)
-            {
-                beta = gamma / gamma_prev;
-                if (!isfinite(beta) || !isfinite(static_cast<S>(beta))) code = kBreakdown;
-            }
-            else code = kBreakdown;
-            // u.s exists only after a completed step
-            if (code == kRunning && beta != 0.0) den = delta + beta * (2.0 * us + beta * st->den[1 - par]);
-            // a non-positive p.Ap of the new direction restarts the step from
-            // u (beta = 0, p.Ap = u.Au = delta); only a non-positive delta is
-            // a breakdown of A itself
-            if (code == kRunning && !(den > 0.0 && isfinite(den)))
-            {
-                beta = 0.0;
-                den = delta;
-                // tells the host to continue in the three-kernel form, which
-                // forms p.Ap from a fresh product every iteration
-                if (blockIdx.x == 0 && threadIdx.x == 0) st->counters[kCounterRestart] = 1u;
-            }
-        }
-        if (code == kRunning && !step_length<S>(gamma, den, alpha)) code = kBreakdown;
-    }
+    const CgHistory h{st->max_iterations, st->tol_rule,     st->rel_tol,      st->abs_tol, st->tol,
+                      st->rho[1 - par],   st->den[1 - par], st->bad_row != ~0ull};
+    const CgDecision d = cg_rules<S>(h, completed, rr, gamma, delta, us);
+    alpha = d.alpha;
+    beta = d.beta;
     if (blockIdx.x == 0 && threadIdx.x == 0)
     {
+        // a restart tells the host to continue in the three-kernel form, which
+        // forms p.Ap from a fresh product every iteration
+        if (d.restart) st->counters[kCounterRestart] = 1u;
         st->rr = rr;
         st->iteration = completed;
         st->iter[par] = completed;
         st->rho[par] = gamma;
-        st->den[par] = den;
+        st->den[par] = d.den;
         st->alpha = alpha;
         if (completed == 0)
         {
             st->rr0 = rr;
-            st->tol = tol;
+            st->tol = d.tol;
         }
-        if (code != kRunning) st->done = code;
+        if (d.code != kRunning) st->done = d.code;
     }
-    return code;
+    return d.code;
 }
 
 // Vectors of single-reduction iteration t: iteration t's r, u, w and s_{t-1}
@@ -2140,8 +2108,7 @@ struct Policy
 // of an LM step ran 27 iterations of early-exit kernels with two chunks of 16
 // in flight), long launch-bound ones cross the host less often (65,536-row
 // FP64 Poisson, 767 iterations: 7.91 ms with chunks of 16, 7.54 ms with 64).
-constexpr int kFirstGrownChunk = 4;
-constexpr int kMaxGrownChunk = 64;
+constexpr int kFirstGrownChunk = 4;  // kMaxGrownChunk in persist.hpp
 
 // By default a chunk of iterations is replayed as a HIP graph below
 // kDirectLaunchRows rows, where the kernels are short enough for the launch
@@ -2281,10 +2248,13 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
         if (report) *report = rep;
         return PM_OK;
     }
-    hipLaunchKernelGGL(k_state_init, dim3(1), dim3(1), 0, stream, pb.st, options->max_iterations,
-                       options->relative_tolerance, options->absolute_tolerance, tol_rule);
-    PM_HIP(hipGetLastError());
-    PM_TRY(get_plan<S>(ws, pb, 0, 0, 0, 0)->run(stream, false));
+    auto initialise = [&]() -> int {
+        hipLaunchKernelGGL(k_state_init, dim3(1), dim3(1), 0, stream, pb.st, options->max_iterations,
+                           options->relative_tolerance, options->absolute_tolerance, tol_rule);
+        PM_HIP(hipGetLastError());
+        return get_plan<S>(ws, pb, 0, 0, 0, 0)->run(stream, false);
+    };
+    PM_TRY(initialise());
 
     // iteration t = max_iterations must run its first kernel to record the
     // final decision, so chunks cover iterations [0, max_iterations].
@@ -2295,6 +2265,54 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     std::deque<int64_t> inflight;
     int64_t launched = 0;
     int64_t chunk_id = 0;
+    if (pb.cg_fused && !pb.cg_factored)
+    {
+        // the one-kernel iteration of a matrix whose rows fit the register
+        // files runs as one launch for the whole solve
+        PersistProblem pp{};
+        pp.rows = a->rows;
+        pp.dtype = a->dtype;
+        pp.dia = &pb.dia;
+        pp.jacobi = pb.pre == kPreJacobi;
+        pp.rhs = rhs;
+        pp.x = x;
+        pp.r = pb.r;
+        pp.u = pb.z;
+        pp.w = pb.q;
+        pp.p = pb.p0;
+        pp.s = pb.p1;
+        pp.inv = pb.inv;
+        pp.x_out = pb.r2;
+        pp.st = pb.st;
+        pp.region = cg_region(pb.partials, 1);
+        pp.count = pb.grid_units;
+        pp.refresh = policy.refresh;
+        pp.chunk = policy.chunk;
+        pp.grow = policy.grow;
+        if (persist_wanted(pp, ws->device))
+        {
+            int outcome = 0;
+            int64_t next = 0;
+            PM_TRY(persist_run(ws, pp, options->max_iterations, stream, &outcome, &next, &fin));
+            if (outcome == kPersistStopped)
+            {
+                PM_HIP(hipEventRecord(ws->done_event, stream));
+                return finish_report(fin, options, report);
+            }
+            if (outcome == kPersistAbandoned) PM_TRY(initialise());
+            else
+            {
+                // a restart: the three-kernel form from iteration `next` on,
+                // with the chunks the schedule has there
+                pb.single_reduction = pb.cg_fused = false;
+                while (launched < next)
+                {
+                    launched += K;
+                    K = next_chunk(++chunk_id, K, policy.grow, kMaxGrownChunk);
+                }
+            }
+        }
+    }
     auto issue = [&]() -> int {
         const int64_t phase = policy.refresh > 0 ? launched % policy.refresh : 0;
         Plan* plan = get_plan<S>(ws, pb, 1, phase, K, policy.refresh);
@@ -2311,7 +2329,7 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
         launched += K;
         // the first two chunks go out together; later ones follow a
         // completed chunk that did not stop the solve
-        if (policy.grow && chunk_id >= 2 && K < kMaxGrownChunk) K *= 2;
+        K = next_chunk(chunk_id, K, policy.grow, kMaxGrownChunk);
         return PM_OK;
     };
     PM_TRY(issue());

@@ -1,0 +1,944 @@
+// A whole single-reduction CG / Jacobi-PCG solve in one cooperative launch,
+// for matrices on the diagonal layout.
+//
+// The per-kernel iteration streams every vector and the matrix through the
+// caches once per iteration and pays a kernel boundary (64 Ki rows: 9.9 us per
+// iteration, all latency; 2.1 M rows: 27.9 us for 113 MB).  Here a workgroup
+// keeps its rows for the whole solve: p, s, x, r, w and the rows' matrix values
+// live in registers (the chip's register files hold 128 MB), with a few words
+// per row in LDS for the largest systems.  Per iteration only u crosses
+// workgroups, and one reduction.
+//
+// Work split.  The per-kernel iteration sums its dot products in `count`
+// workgroups of four wavefronts over contiguous 64-row chunks; a workgroup here
+// takes four consecutive ones of those (1,024 threads), each wavefront the rows
+// of the wavefront it stands for, and every sum runs in the same order.  A solve
+// is therefore bitwise the per-kernel solve.
+//
+// Exchange.  Every word that crosses workgroups is a 64-bit relaxed atomic at
+// agent scope that carries 32 bits of data and the iteration's tag, so a reader
+// polls the data itself: no flags, fences or ordering between words.  (An
+// agent-scope fence writes back or drops the XCD's L2: with fences a 65,536-row
+// iteration took 27 us, with these words 5.)  A word is rewritten only after
+// every reader of its old value has contributed to a reduction that the writer
+// waited for; the partial sums, which several workgroups read, alternate
+// between two sets.
+//
+// Rows near a workgroup's ends are copied into LDS halos; the outermost
+// diagonals of a 3-D stencil reach whole pieces away, and their words are read
+// by the lane that needs them.
+//
+// Waits are bounded: a workgroup that sees no progress for kWaitSeconds (or
+// another one's notice of that) leaves, the new x is not committed, and the
+// host runs the solve in the per-kernel form instead.
+//
+// Measured, solve time per-kernel / persistent: 65,536-row FP64 2-D Laplacian
+// (767 iterations, one row per lane) 7.67 / 4.48 ms, 5.7 us per iteration, two
+// exchange latencies; 2,097,152-row FP32 3-D diffusion (753 iterations, eight
+// rows per lane) 20.4 / 15.4 ms, 18.6 us per iteration.
+#include "persist.hpp"
+
+#include <algorithm>
+#include <cstdlib>
+#include <type_traits>
+
+#include "cg_rules.hpp"
+#include "spmv_kernels.hpp"
+
+namespace pm
+{
+namespace
+{
+
+using word = unsigned long long;
+
+constexpr int kPersistThreads = 1024;
+constexpr int kPersistWaves = kPersistThreads / kWave;
+constexpr int kPersistGroups = kPersistThreads / kBlock;  // per-kernel workgroups one workgroup stands for
+constexpr int kPersistBlocks = kSolverGrid / kPersistGroups;
+constexpr int kRedEntries = kSolverGrid - kBlock;
+constexpr int kDecWords = 16;        // one 128-byte line per workgroup
+constexpr int kHandOver = 100;       // decision code: leave without deciding
+constexpr int kWaitSeconds = 4;
+constexpr int64_t kSegment = 8192;   // iterations per launch
+constexpr int kCounterOutcome = 1;   // SolverState::counters slot: 1 committed
+constexpr int kCounterNext = 2;      // ... iteration the launch handed over at
+
+struct PersistControl
+{
+    unsigned abort;
+    unsigned finished;
+    unsigned pad[62];
+    word part[2][kCgValues][2][kSolverGrid];  // parity, value, half, per-kernel workgroup
+    word dec[kPersistBlocks][kDecWords];
+};
+
+// What thread 0 of a leading workgroup keeps between decisions (in LDS: as
+// registers it would take some from every lane).
+struct PersistHistory
+{
+    CgHistory h;
+    double rr, rr0, alpha;
+    int completed, t_stop, restarted;
+};
+
+template <typename S>
+struct PersistArgs
+{
+    int rows;
+    DiaArgs dia;
+    const S* dv;
+    const uint16_t* mask;
+    const S* x_in;
+    S* x_out;
+    S *p, *r, *s, *w, *u;
+    const S* inv;
+    const S* rhs;
+    SolverState* st;
+    double* region;
+    PersistControl* ctl;
+    word* xu;  // u words: low halves (FP32: the value), then high halves
+    word* xx;  // x words of a residual refresh
+    unsigned tag;  // tags of this launch are above it
+    int count, per, halo, leaders, refresh;
+    int t0, t_end;
+    int chunk, grow, most;
+    int span;  // local rows that the LDS arrays hold
+    int priv, red;  // bytes of LDS before x and the inner diagonals, and before the leaders' reduction
+};
+
+__device__ __forceinline__ word load_word(const word* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_word(word* p, unsigned v, unsigned tag)
+{
+    __hip_atomic_store(p, (static_cast<word>(tag) << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Word i of an exchange array (fewer than 2^29 words: a 32-bit byte offset from
+// a uniform base).
+__device__ __forceinline__ word* word_at(word* b, unsigned i)
+{
+    return reinterpret_cast<word*>(reinterpret_cast<char*>(b) + i * 8u);
+}
+__device__ __forceinline__ const word* word_at(const word* b, unsigned i)
+{
+    return reinterpret_cast<const word*>(reinterpret_cast<const char*>(b) + i * 8u);
+}
+__device__ __forceinline__ bool word_ready(word v, unsigned tag) { return static_cast<unsigned>(v >> 32) == tag; }
+
+// A value of the exchange: one word for FP32, two for FP64 (half planes).
+template <typename S>
+struct Exchange;
+template <>
+struct Exchange<float>
+{
+    static constexpr int kWords = 1;
+    __device__ static __forceinline__ void put(word* b, int, unsigned i, float v, unsigned tag)
+    {
+        store_word(word_at(b, i), __float_as_uint(v), tag);
+    }
+    __device__ static __forceinline__ void issue(const word* b, int, unsigned i, word (&w)[1])
+    {
+        w[0] = load_word(word_at(b, i));
+    }
+    __device__ static __forceinline__ float value(const word (&w)[1]) { return __uint_as_float(static_cast<unsigned>(w[0])); }
+};
+template <>
+struct Exchange<double>
+{
+    static constexpr int kWords = 2;
+    __device__ static __forceinline__ void put(word* b, int plane, unsigned i, double v, unsigned tag)
+    {
+        const word bits = static_cast<word>(__double_as_longlong(v));
+        store_word(word_at(b, i), static_cast<unsigned>(bits), tag);
+        store_word(word_at(b + plane, i), static_cast<unsigned>(bits >> 32), tag);
+    }
+    __device__ static __forceinline__ void issue(const word* b, int plane, unsigned i, word (&w)[2])
+    {
+        w[0] = load_word(word_at(b, i));
+        w[1] = load_word(word_at(b + plane, i));
+    }
+    __device__ static __forceinline__ double value(const word (&w)[2])
+    {
+        return __longlong_as_double(static_cast<long long>((w[1] << 32) | (w[0] & 0xffffffffull)));
+    }
+};
+template <typename S>
+__device__ __forceinline__ bool ready(const word (&w)[Exchange<S>::kWords], unsigned tag)
+{
+    bool ok = word_ready(w[0], tag);
+    if constexpr (Exchange<S>::kWords == 2) ok = ok && word_ready(w[1], tag);
+    return ok;
+}
+
+// The workgroup of the per-kernel iteration that owns logical block lb (the
+// inverse of xcd_logical_block).
+__device__ __forceinline__ int physical_block(int lb, int nb)
+{
+    const int q = nb / kXcds, r = nb % kXcds;
+    const int head = r * (q + 1);
+    const int xcd = lb < head ? lb / (q + 1) : r + (lb - head) / (q > 0 ? q : 1);
+    const int idx = lb < head ? lb % (q + 1) : (lb - head) % (q > 0 ? q : 1);
+    return idx * kXcds + xcd;
+}
+
+// Waits for words that other workgroups write: `poll` loads them and says
+// whether all carry their tag.  The whole wavefront polls together.
+template <typename Poll>
+__device__ __forceinline__ bool wait_for(PersistControl* ctl, Poll poll)
+{
+    unsigned polls = 0;
+    long long start = 0;
+    while (!__all(poll()))
+    {
+        // the bound of the wait: every 256 polls look at the clock (100 MHz)
+        // and at another workgroup's notice that it gave up
+        if ((++polls & 255u) != 0u) continue;
+        const long long now = wall_clock64();
+        if (start == 0) start = now;
+        if (__hip_atomic_load(&ctl->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ||
+            now - start > kWaitSeconds * 100000000ll)
+        {
+            __hip_atomic_store(&ctl->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+    }
+    return true;
+}
+
+// ND diagonals with symmetric offsets (ND / 2 is the main diagonal), R rows per
+// lane.  UNIT: an unpreconditioned solve whose main diagonal is all ones (u is
+// r); else the main diagonal is stored and u = inv r (inv of ones without a
+// preconditioner, which gives the same bits).  FAR: the outermost diagonals
+// reach past the halos.  An absent entry has the value 0 and some finite
+// partner, which leaves the row sums' bits alone.
+//
+// Registers: p, s, r, w, the two outermost diagonals (and inv, diagonal) per
+// row, with x and the inner diagonals as long as a lane's rows stay below 32
+// bytes per vector.  From there on x and the inner upper diagonals sit in LDS
+// (a symmetric matrix: row l's lower value is row l - off's upper one).
+template <typename S, int ND, int R, bool UNIT, bool FAR>
+__global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a)
+{
+    using X = Exchange<S>;
+    constexpr int M = ND / 2;
+    constexpr bool kLds = sizeof(S) * R >= 32;
+    constexpr int NV = UNIT ? 3 : 4;
+    // far words in flight per lane: FB rows of two
+    constexpr int FB = R < 8 / (2 * X::kWords) ? R : 8 / (2 * X::kWords);
+    extern __shared__ char lds_raw[];
+    __shared__ double lds_p[kCgValues][kPersistWaves];   // partial sums of the wavefronts
+    __shared__ double lds_w[kCgValues][kBlock / kWave];  // the decision's reduction
+    __shared__ S sh_alpha, sh_beta;
+    __shared__ int sh_code, sh_fail;
+    __shared__ PersistHistory hs;
+
+    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    const int blocks = gridDim.x, bid = blockIdx.x;
+    const int g = static_cast<int>(xcd_logical_block(bid, blocks));
+    const int rows = a.rows, H = a.halo;
+    const int piece = kPersistGroups * a.per * kChunkRows;  // rows of a full piece
+    const int base = g * piece;
+    int size = rows - base;  // rows of this piece
+    size = size < 0 ? 0 : (size > piece ? piece : size);
+    S* us = reinterpret_cast<S*>(lds_raw) + H;         // u of rows [-H, span + H) of the piece
+    S* xs = reinterpret_cast<S*>(lds_raw + a.priv);    // kLds: x, [R][kPersistThreads]
+    S* vs = xs + R * kPersistThreads + H;              // kLds: inner upper diagonals of rows [-H, piece)
+    const int vstride = a.span + H;
+    double* red = reinterpret_cast<double*>(lds_raw + a.red);  // leaders: entries from kBlock on, [value][entry]
+
+    // rows of the lane: local row l0 + k * kBlock for k < slots
+    const int grp = tid / kBlock, gwave = wave % kWavesPerBlock;
+    const int l0 = (grp * a.per + gwave) * kChunkRows + lane;
+    const int slots = (a.per - gwave + kWavesPerBlock - 1) / kWavesPerBlock;
+    const int limit = l0 + slots * kBlock < size ? l0 + slots * kBlock : size;  // local rows below it are the lane's
+
+    S p[R], s[R], x[R], r[R], w[R], val[R][ND], inv[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+    {
+        const int l = l0 + k * kBlock;
+        const bool ok = l < limit;
+        const int i = ok ? base + l : 0;
+        const unsigned m = ok ? a.mask[i] : 0u;
+        p[k] = ok ? a.p[i] : S(0);
+        s[k] = ok ? a.s[i] : S(0);
+        r[k] = ok ? a.r[i] : S(0);
+        w[k] = ok ? a.w[i] : S(0);
+        if constexpr (!UNIT) inv[k] = ok ? (a.inv != nullptr ? a.inv[i] : S(1)) : S(0);
+        const S xv = ok ? a.x_in[i] : S(0);
+        if constexpr (kLds) xs[k * kPersistThreads + tid] = xv;
+        else x[k] = xv;
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+        {
+            if ((UNIT && d == M) || (kLds && d != 0 && d != M && d != ND - 1)) continue;
+            val[k][d] = ((m >> d) & 1u)
+                            ? dia_value(static_cast<int64_t>(i), static_cast<int64_t>(rows), a.dia, a.dv, d)
+                            : S(0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (kLds)
+    {
+#pragma unroll
+        for (int d = M + 1; d < ND - 1; ++d)
+            for (int l = tid - H; l < a.span; l += kPersistThreads)
+            {
+                const int i = base + l;
+                vs[(d - M - 1) * vstride + l] =
+                    i >= 0 && l < size && ((a.mask[i] >> d) & 1u) ? a.dv[static_cast<int64_t>(a.dia.slot[d]) * rows + i] : S(0);
+            }
+    }
+    // halo rows past the matrix and the rows past a short piece stay 0
+    for (int l = tid - H; l < a.span + H; l += kPersistThreads) us[l] = S(0);
+    auto u_of = [&](int k) {
+        if constexpr (UNIT) return r[k];
+        else return inv[k] * r[k];
+    };
+    auto x_of = [&](int k) {
+        if constexpr (kLds) return xs[k * kPersistThreads + tid];
+        else return x[k];
+    };
+
+    // thread 0 of a leading workgroup holds the history of the decisions
+    const bool leader = bid < a.leaders;
+    if (leader && tid == 0)
+    {
+        hs.h = CgHistory{a.st->max_iterations, a.st->tol_rule, a.st->rel_tol, a.st->abs_tol,
+                         a.st->tol,            a.st->rho[1],   a.st->den[1],  a.st->bad_row != ~0ull};
+        hs.completed = a.st->iter[1] + 1;
+        hs.rr0 = a.st->rr0;
+        hs.rr = hs.alpha = 0.0;
+        hs.t_stop = a.t_end;
+        hs.restarted = 0;
+    }
+    if (tid == 0) sh_fail = 0;
+    __syncthreads();
+
+    // the lane's rows of a vector into LDS and, where another workgroup reads
+    // them, into the exchange
+    auto publish = [&](word* buf, unsigned tag, auto get) {
+        int l = l0;
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+        {
+            const int lr = l + k * kBlock;
+            if (lr < limit)
+            {
+                const S v = get(k);
+                us[lr] = v;
+                if (FAR || lr < H || lr >= size - H) X::put(buf, rows, base + lr, v, tag);
+            }
+        }
+    };
+
+    // acc[k] = row k of A v for the vector published last, entries in
+    // increasing column order; own(k) is the lane's own entry
+    auto product = [&](const word* buf, unsigned tag, auto own, auto* acc) {
+        using Acc = std::remove_reference_t<decltype(acc[0])>;
+        int l = l0;
+        asm volatile("" : "+v"(l));
+        word far_lo[FB][X::kWords], far_hi[FB][X::kWords];
+        // every row is published under FAR, so the word of a clamped row
+        // (absent entries, slots past the lane's rows) arrives too
+        auto issue = [&](int kb) {
+#pragma unroll
+            for (int j = 0; j < FB; ++j)
+            {
+                const int i = base + l + (kb + j) * kBlock;
+                int lo = i + a.dia.off[0], hi = i + a.dia.off[ND - 1];
+                lo = lo < 0 ? 0 : (lo >= rows ? rows - 1 : lo);
+                hi = hi < 0 ? 0 : (hi >= rows ? rows - 1 : hi);
+                X::issue(buf, rows, lo, far_lo[j]);
+                X::issue(buf, rows, hi, far_hi[j]);
+            }
+        };
+        auto arrived = [&]() {
+            bool ok = true;
+#pragma unroll
+            for (int j = 0; j < FB; ++j) ok = ok && ready<S>(far_lo[j], tag) && ready<S>(far_hi[j], tag);
+            return ok;
+        };
+        bool fine = true;
+        if constexpr (FAR) issue(0);
+        // halo rows of the neighbouring pieces
+        for (int h0 = 0; h0 < 2 * H; h0 += kPersistThreads)
+        {
+            const int h = h0 + tid;
+            const int q = h < H ? h - H : size + (h - H);
+            const int i = base + q;
+            if (h >= 2 * H || size == 0 || i < 0 || i >= rows) continue;
+            word hw[X::kWords];
+            fine = fine && wait_for(a.ctl, [&] {
+                       X::issue(buf, rows, i, hw);
+                       return ready<S>(hw, tag);
+                   });
+            us[q] = X::value(hw);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kb = 0; kb < R; kb += FB)
+        {
+            if constexpr (FAR)
+            {
+                if (!__all(arrived()))
+                    fine = fine && wait_for(a.ctl, [&] {
+                               issue(kb);
+                               return arrived();
+                           });
+            }
+#pragma unroll
+            for (int j = 0; j < FB; ++j)
+            {
+                const int k = kb + j;
+                // slots past the lane's rows compute on whatever the LDS behind
+                // the piece holds and are dropped
+                const int lr = l + k * kBlock;
+                Acc sum = Acc(0);
+#pragma unroll
+                for (int d = 0; d < ND; ++d)
+                {
+                    S v, e;
+                    if (d == M) e = own(k);
+                    else if (FAR && (d == 0 || d == ND - 1)) e = X::value(d == 0 ? far_lo[j] : far_hi[j]);
+                    else e = us[lr + a.dia.off[d]];
+                    if (d == M)
+                    {
+                        if constexpr (UNIT) v = S(1);
+                        else v = val[k][d];
+                    }
+                    else if (!kLds || d == 0 || d == ND - 1) v = val[k][d];
+                    else if (d < M) v = vs[(ND - 1 - d - M - 1) * vstride + lr + a.dia.off[d]];
+                    else v = vs[(d - M - 1) * vstride + lr];
+                    sum = fma_s<Acc>(static_cast<Acc>(v), static_cast<Acc>(e), sum);
+                }
+                acc[k] = l + k * kBlock < limit ? sum : Acc(0);
+                if (kLds) __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (FAR)
+                if (kb + FB < R) issue(kb + FB);
+        }
+        if (!fine) sh_fail = 1;
+    };
+
+    int code = kRunning;
+    for (int t = a.t0;; ++t)
+    {
+        // ---- decision: stop test, alpha, beta from the partials of t - 1 ----
+        const unsigned tag = a.tag + static_cast<unsigned>(t - a.t0) + 1u;
+        if (leader)
+        {
+            bool fine = true;
+            auto entry = [&](int e, double (&out)[NV]) {
+                if (t == a.t0)
+                {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) out[v] = a.region[(UNIT && v > 0 ? v + 1 : v) * kMaxPartials + e];
+                    return;
+                }
+                word hw[NV][2];
+                const word* at = &a.ctl->part[(t - 1) & 1][0][0][e];
+                fine = wait_for(a.ctl, [&] {
+                    bool ok = true;
+#pragma unroll
+                    for (int v = 0; v < NV; ++v)
+                    {
+                        hw[v][0] = load_word(at + (2 * v) * kSolverGrid);
+                        hw[v][1] = load_word(at + (2 * v + 1) * kSolverGrid);
+                    }
+#pragma unroll
+                    for (int v = 0; v < NV; ++v)
+                        ok = ok && word_ready(hw[v][0], tag - 1u) && word_ready(hw[v][1], tag - 1u);
+                    return ok;
+                });
+#pragma unroll
+                for (int v = 0; v < NV; ++v) out[v] = Exchange<double>::value(hw[v]);
+            };
+            double acc[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) acc[v] = 0.0;
+            if (a.count <= kBlock)
+            {
+                if (tid < a.count)
+                {
+                    double e[NV];
+                    entry(tid, e);
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) acc[v] += e[v];
+                }
+            }
+            else
+            {
+                double e[NV];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) e[v] = 0.0;
+                if (tid < a.count) entry(tid, e);
+                if (tid >= kBlock)
+                {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) red[v * kRedEntries + tid - kBlock] = e[v];
+                }
+                __syncthreads();
+                if (tid < kBlock)
+                {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v)
+                    {
+                        acc[v] += e[v];
+#pragma unroll
+                        for (int j = 0; j < kRedEntries / kBlock; ++j) acc[v] += red[v * kRedEntries + tid + j * kBlock];
+                    }
+                }
+            }
+            if (tid < kBlock)
+            {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) acc[v] = wave_sum(acc[v]);
+                if (lane == 0)
+                {
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) lds_w[v][wave] = acc[v];
+                }
+            }
+            if (!fine) sh_fail = 1;
+            __syncthreads();
+            if (tid == 0)
+            {
+                double tot[NV];
+#pragma unroll
+                for (int v = 0; v < NV; ++v)
+                {
+                    double q = 0.0;
+#pragma unroll
+                    for (int z = 0; z < kBlock / kWave; ++z) q += lds_w[v][z];
+                    tot[v] = q;
+                }
+                int c = kHandOver;
+                if (t < hs.t_stop)
+                {
+                    const CgDecision d =
+                        cg_rules<S>(hs.h, hs.completed, tot[0], tot[UNIT ? 0 : 1], tot[NV - 2], tot[NV - 1]);
+                    c = d.code;
+                    sh_alpha = static_cast<S>(d.alpha);
+                    sh_beta = static_cast<S>(d.beta);
+                    hs.rr = tot[0];
+                    hs.alpha = d.alpha;
+                    if (hs.completed == 0) hs.rr0 = tot[0];
+                    hs.h.tol = d.tol;
+                    hs.h.gamma_prev = tot[UNIT ? 0 : 1];
+                    hs.h.den_prev = d.den;
+                    if (d.restart && hs.restarted == 0)
+                    {
+                        hs.restarted = 1;
+                        const int64_t over = hand_over_iteration(t, a.chunk, a.grow != 0, a.most);
+                        if (over < hs.t_stop) hs.t_stop = static_cast<int>(over);
+                    }
+                    ++hs.completed;
+                }
+                sh_code = c;
+            }
+            __syncthreads();
+            // the workgroups this leader answers to: bid + leaders, ...
+            const int who = bid + (tid + 1) * a.leaders;
+            if (who < blocks && sh_fail == 0)
+            {
+                word* line = a.ctl->dec[who];
+                X::put(line, kDecWords / 2, 0, sh_alpha, tag);
+                X::put(line, kDecWords / 2, 1, sh_beta, tag);
+                store_word(line + 2, static_cast<unsigned>(sh_code), tag);
+            }
+        }
+        else
+        {
+            if (wave == 0)
+            {
+                // alpha, beta, code by lanes 0, 1, 2 (the other lanes repeat 2)
+                const word* line = a.ctl->dec[bid] + (lane < 2 ? lane : 2);
+                word hw[X::kWords];
+                const bool fine = wait_for(a.ctl, [&] {
+                    hw[0] = load_word(line);
+                    bool ok = word_ready(hw[0], tag);
+                    if constexpr (X::kWords == 2)
+                    {
+                        hw[1] = load_word(line + (lane < 2 ? kDecWords / 2 : 0));
+                        ok = ok && word_ready(hw[1], tag);
+                    }
+                    return ok;
+                });
+                if (!fine) sh_fail = 1;
+                if (lane == 0) sh_alpha = X::value(hw);
+                else if (lane == 1) sh_beta = X::value(hw);
+                else if (lane == 2) sh_code = static_cast<int>(hw[0]);
+            }
+            __syncthreads();
+        }
+        if (sh_fail != 0) return;
+        code = sh_code;
+        if (code != kRunning) break;
+        const S al = sh_alpha, be = sh_beta;
+
+        // ---- step, then w = A u of the new u ----
+        const bool refresh = a.refresh > 0 && (t + 1) % a.refresh == 0;
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+        {
+            p[k] = fma_s(be, p[k], u_of(k));
+            s[k] = fma_s(be, s[k], w[k]);
+            const S xn = fma_s(al, p[k], x_of(k));
+            if constexpr (kLds) xs[k * kPersistThreads + tid] = xn;
+            else x[k] = xn;
+            if (!refresh) r[k] = fma_s(-al, s[k], r[k]);
+        }
+        if (refresh)
+        {
+            // r = b - A x with FP64 accumulation
+            publish(a.xx, tag, x_of);
+            double ax[R];
+            product(a.xx, tag, x_of, ax);
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+            {
+                const int l = l0 + k * kBlock;
+                if (l < limit) r[k] = static_cast<S>(static_cast<double>(a.rhs[base + l]) - ax[k]);
+            }
+            __syncthreads();
+        }
+        publish(a.xu, tag, u_of);
+        product(a.xu, tag, u_of, w);
+
+        // ---- partial sums per workgroup of the per-kernel iteration ----
+        double part[kCgValues] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+        {
+            const double rv = static_cast<double>(r[k]);
+            const double uv = static_cast<double>(u_of(k));
+            part[0] = __builtin_fma(rv, rv, part[0]);
+            if (!UNIT) part[1] = __builtin_fma(rv, uv, part[1]);
+            part[NV - 2] = __builtin_fma(static_cast<double>(w[k]), uv, part[NV - 2]);
+            part[NV - 1] = __builtin_fma(uv, static_cast<double>(s[k]), part[NV - 1]);
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) part[v] = wave_sum(part[v]);
+        if (lane == 0)
+        {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) lds_p[v][wave] = part[v];
+        }
+        __syncthreads();
+        if (sh_fail != 0) return;
+        if (tid < NV * kPersistGroups)
+        {
+            const int v = tid / kPersistGroups, q = tid % kPersistGroups;
+            const int lb = g * kPersistGroups + q;
+            if (lb < a.count)
+            {
+                double sum = 0.0;
+#pragma unroll
+                for (int z = 0; z < kWavesPerBlock; ++z) sum += lds_p[v][q * kWavesPerBlock + z];
+                const int vb = physical_block(lb, a.count);
+                Exchange<double>::put(&a.ctl->part[t & 1][v][0][vb], kSolverGrid, 0, sum, tag);
+            }
+        }
+    }
+
+    // ---- the end: x, and for a hand-over everything the next form reads ----
+    const bool over = code == kHandOver;
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+    {
+        const int l = l0 + k * kBlock;
+        if (l >= limit) continue;
+        const int i = base + l;
+        a.x_out[i] = x_of(k);
+        if (!over) continue;
+        a.p[i] = p[k];
+        a.s[i] = s[k];
+        a.r[i] = r[k];
+        a.w[i] = w[k];
+        if (!UNIT && a.inv != nullptr) a.u[i] = u_of(k);
+    }
+    if (over && tid < kPersistGroups && g * kPersistGroups + tid < a.count)
+    {
+        // t0 and the hand-over iteration are even: the last partials are of an
+        // odd iteration, region 1
+        const int vb = physical_block(g * kPersistGroups + tid, a.count);
+        double vals[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+        {
+            word hw[2] = {load_word(&a.ctl->part[1][v][0][vb]), load_word(&a.ctl->part[1][v][1][vb])};
+            vals[v] = Exchange<double>::value(hw);
+        }
+        a.region[vb] = vals[0];
+        a.region[kMaxPartials + vb] = vals[UNIT ? 0 : 1];
+        a.region[2 * kMaxPartials + vb] = vals[NV - 2];
+        a.region[3 * kMaxPartials + vb] = vals[NV - 1];
+    }
+    if (bid == 0 && tid == 0)
+    {
+        // completed counts the decisions: the last one saw completed - 1 updates
+        const int seen = hs.completed - 1, par = seen & 1;
+        SolverState* st = a.st;
+        st->rr = hs.rr;
+        st->rr0 = hs.rr0;
+        st->tol = hs.h.tol;
+        st->iteration = seen;
+        st->iter[par] = seen;
+        st->rho[par] = hs.h.gamma_prev;
+        st->den[par] = hs.h.den_prev;
+        st->alpha = hs.alpha;
+        if (hs.restarted) st->counters[kCounterRestart] = 1u;
+        st->counters[kCounterNext] = static_cast<unsigned>(hs.completed);
+        if (!over) st->done = code;
+    }
+    __syncthreads();
+    if (tid == 0) __hip_atomic_fetch_add(&a.ctl->finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void k_persist_reset(PersistControl* ctl, SolverState* st)
+{
+    ctl->abort = 0u;
+    ctl->finished = 0u;
+    st->counters[kCounterOutcome] = 0u;
+}
+
+__global__ void k_persist_clear(word* p, int64_t n)
+{
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+        p[i] = 0ull;
+}
+
+// Copies the new x when every workgroup of the solve reached its end and this
+// was the last launch of it, and tells the host.
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_persist_commit(int64_t rows, const S* __restrict__ from, S* __restrict__ x,
+                                                           const PersistControl* ctl, unsigned blocks, SolverState* st)
+{
+    if (ctl->finished != blocks) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->counters[kCounterOutcome] = 1u;
+    if (st->done == kRunning && st->counters[kCounterRestart] == 0u) return;  // the next launch continues from `from`
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < rows;
+         i += static_cast<int64_t>(gridDim.x) * kBlock)
+        x[i] = from[i];
+}
+
+struct PersistShape
+{
+    int nd, rows_per_lane, per, blocks, halo, span;
+    bool unit, far;
+    size_t shared, red;  // LDS before x and the inner diagonals, before the leaders' reduction
+    size_t lds;
+};
+
+constexpr size_t kPersistLds = 160 * 1024 - 2048;  // LDS of a CU less the static part
+
+bool persist_shape(const PersistProblem& p, PersistShape* out)
+{
+    const DiaLayout& d = *p.dia;
+    const int nd = d.args.ndiag;
+    if (!d.active || (nd != 5 && nd != 7) || p.rows <= 0) return false;
+    for (int k = 0; k < nd; ++k)
+        if (d.args.off[k] != -d.args.off[nd - 1 - k]) return false;
+    PersistShape s{};
+    s.nd = nd;
+    s.unit = !p.jacobi && d.args.slot[nd / 2] < 0;
+    const int64_t chunks = chunk_count(p.rows);
+    s.per = static_cast<int>(ceil_div(chunks, static_cast<int64_t>(p.count)));
+    const int need = (s.per + kWavesPerBlock - 1) / kWavesPerBlock;
+    s.rows_per_lane = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
+    const int es = p.dtype == PM_F64 ? 8 : 4;
+    if (need > 8 || s.rows_per_lane * es > 32) return false;
+    const bool in_lds = s.rows_per_lane * es == 32;  // x and the inner upper diagonals in LDS
+    for (int k = 0; in_lds && k < nd / 2; ++k)
+        if (d.args.slot[k] != d.args.slot[nd - 1 - k] || d.args.slot[k] < 0) return false;  // not mirrored
+    s.blocks = static_cast<int>(ceil_div(static_cast<int64_t>(p.count), static_cast<int64_t>(kPersistGroups)));
+    const int64_t piece = static_cast<int64_t>(kPersistGroups) * s.per * kChunkRows;
+    const int inner_arrays = nd / 2 - 1;
+    // the last local row any lane's R slots address
+    s.span = ((kPersistGroups - 1) * s.per + kWavesPerBlock) * kChunkRows + (s.rows_per_lane - 1) * kBlock;
+    s.span = std::max(s.span, static_cast<int>(piece));
+    // the piece's u with its halos, x and the inner upper diagonals, and the
+    // leaders' reduction of more than kBlock partials
+    auto shared = [&](int64_t halo) { return (static_cast<size_t>(s.span + 2 * halo) * es + 15) & ~size_t(15); };
+    auto reduction = [&](int64_t halo) {
+        const size_t kept = in_lds ? (static_cast<size_t>(s.rows_per_lane) * kPersistThreads +
+                                      static_cast<size_t>(inner_arrays) * (s.span + halo)) *
+                                         es
+                                   : 0;
+        return (shared(halo) + kept + 15) & ~size_t(15);
+    };
+    auto total = [&](int64_t halo) {
+        return reduction(halo) + (p.count > kBlock ? sizeof(double) * (s.unit ? 3 : 4) * kRedEntries : size_t(0));
+    };
+    // halos of the widest offset that a piece and the LDS can hold; only the
+    // outermost diagonals may reach past it
+    const int64_t outer = d.args.off[nd - 1], inner = d.args.off[nd - 2];
+    int64_t halo = outer;
+    if (halo > piece || halo > 2 * kPersistThreads || total(halo) > kPersistLds)
+    {
+        halo = inner;
+        s.far = true;
+        if (halo > piece || total(halo) > kPersistLds) return false;
+    }
+    s.halo = static_cast<int>(halo);
+    s.shared = shared(halo);
+    s.red = reduction(halo);
+    s.lds = total(halo);
+    *out = s;
+    return true;
+}
+
+template <typename S, int ND, int R>
+const void* persist_instance(const PersistShape& s)
+{
+    if (s.unit)
+        return s.far ? reinterpret_cast<const void*>(k_cg_persist<S, ND, R, true, true>)
+                     : reinterpret_cast<const void*>(k_cg_persist<S, ND, R, true, false>);
+    return s.far ? reinterpret_cast<const void*>(k_cg_persist<S, ND, R, false, true>)
+                 : reinterpret_cast<const void*>(k_cg_persist<S, ND, R, false, false>);
+}
+
+template <typename S, int ND>
+const void* persist_kernel(const PersistShape& s)
+{
+    switch (s.rows_per_lane)
+    {
+    case 1: return persist_instance<S, ND, 1>(s);
+    case 2: return persist_instance<S, ND, 2>(s);
+    case 4: return persist_instance<S, ND, 4>(s);
+    default: break;
+    }
+    if constexpr (sizeof(S) == 4) return persist_instance<S, ND, 8>(s);
+    return nullptr;
+}
+
+template <typename S>
+int persist_run_t(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream, int* outcome,
+                  int64_t* next, SolverState* state)
+{
+    PersistShape shape{};
+    *outcome = kPersistAbandoned;
+    if (!persist_shape(p, &shape)) return PM_OK;
+    const void* kernel = shape.nd == 5 ? persist_kernel<S, 5>(shape) : persist_kernel<S, 7>(shape);
+    if (kernel == nullptr) return PM_OK;
+    PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(shape.lds)));
+    const size_t words = static_cast<size_t>(p.rows) * Exchange<S>::kWords;
+    const size_t control = (sizeof(PersistControl) + 255) & ~size_t(255);
+    const size_t need = control + 2 * words * sizeof(word);
+    const bool grown = need > ws->persist.bytes;
+    PM_TRY(ws->persist.reserve(need));
+    if (grown || ws->persist_tag > 0xf0000000u)
+    {
+        // no word may carry a tag that is still to come
+        hipLaunchKernelGGL(k_persist_clear, dim3(1024), dim3(kBlock), 0, stream, ws->persist.as<word>(),
+                           static_cast<int64_t>(ws->persist.bytes / sizeof(word)));
+        PM_HIP(hipGetLastError());
+        ws->persist_tag = 0;
+    }
+    PersistArgs<S> a{};
+    a.rows = static_cast<int>(p.rows);
+    a.dia = p.dia->args;
+    a.dv = static_cast<const S*>(p.dia->values);
+    a.mask = p.dia->mask;
+    a.x_in = static_cast<const S*>(p.x);
+    a.x_out = static_cast<S*>(p.x_out);
+    a.p = static_cast<S*>(p.p);
+    a.r = static_cast<S*>(p.r);
+    a.s = static_cast<S*>(p.s);
+    a.w = static_cast<S*>(p.w);
+    a.u = static_cast<S*>(p.u);
+    a.inv = p.jacobi ? static_cast<const S*>(p.inv) : nullptr;
+    a.rhs = static_cast<const S*>(p.rhs);
+    a.st = p.st;
+    a.region = p.region;
+    a.ctl = ws->persist.as<PersistControl>();
+    a.xu = reinterpret_cast<word*>(ws->persist.as<char>() + control);
+    a.xx = a.xu + words;
+    a.count = p.count;
+    a.per = shape.per;
+    a.halo = shape.halo;
+    a.priv = static_cast<int>(shape.shared);
+    a.red = static_cast<int>(shape.red);
+    a.span = shape.span;
+    // every workgroup decides for itself, or eight decide and answer the rest
+    a.leaders = shape.blocks <= 64 ? shape.blocks : kXcds;
+    a.refresh = p.refresh;
+    a.chunk = p.chunk;
+    a.grow = p.grow ? 1 : 0;
+    a.most = kMaxGrownChunk;
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(p.rows, kBlock), 2048));
+    for (int64_t t = 0;; )
+    {
+        // an even number of iterations, the last one's decision included
+        const int64_t left = max_iterations + 2 - t;
+        const int64_t count = std::min<int64_t>(kSegment, left + (left & 1));
+        a.t0 = static_cast<int>(t);
+        a.t_end = static_cast<int>(t + count);
+        if (t > 0) a.x_in = a.x_out;
+        a.tag = ws->persist_tag;
+        ws->persist_tag += static_cast<uint32_t>(count) + 2u;
+        hipLaunchKernelGGL(k_persist_reset, dim3(1), dim3(1), 0, stream, a.ctl, p.st);
+        PM_HIP(hipGetLastError());
+        void* args[] = {&a};
+        const hipError_t err = hipLaunchCooperativeKernel(kernel, dim3(shape.blocks), dim3(kPersistThreads), args,
+                                                          static_cast<unsigned>(shape.lds), stream);
+        if (err == hipErrorCooperativeLaunchTooLarge || err == hipErrorNotSupported)
+        {
+            (void)hipGetLastError();
+            return PM_OK;
+        }
+        PM_HIP(err);
+        hipLaunchKernelGGL(k_persist_commit<S>, dim3(grid), dim3(kBlock), 0, stream, p.rows,
+                           static_cast<const S*>(p.x_out), static_cast<S*>(p.x), a.ctl,
+                           static_cast<unsigned>(shape.blocks), p.st);
+        PM_HIP(hipGetLastError());
+        PM_HIP(hipMemcpyAsync(ws->host_state, p.st, sizeof(SolverState), hipMemcpyDeviceToHost, stream));
+        PM_HIP(hipStreamSynchronize(stream));
+        *state = ws->host_state[0];
+        if (state->counters[kCounterOutcome] != 1u) return PM_OK;
+        if (state->done != kRunning)
+        {
+            *outcome = kPersistStopped;
+            return PM_OK;
+        }
+        t = static_cast<int64_t>(state->counters[kCounterNext]);
+        if (state->counters[kCounterRestart] != 0u)
+        {
+            *outcome = kPersistHandOver;
+            *next = t;
+            return PM_OK;
+        }
+    }
+}
+
+} // namespace
+
+bool persist_wanted(const PersistProblem& p, int device)
+{
+    const char* env = std::getenv("PLAMATRIX_AMD_PERSISTENT");
+    if (env != nullptr && env[0] == '0') return false;
+    PersistShape s{};
+    if (!persist_shape(p, &s)) return false;
+    int coop = 0, cus = 0;
+    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    return coop != 0 && s.blocks <= cus;
+}
+
+int persist_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream, int* outcome,
+                int64_t* next, SolverState* state)
+{
+    if (p.dtype == PM_F64) return persist_run_t<double>(ws, p, max_iterations, stream, outcome, next, state);
+    return persist_run_t<float>(ws, p, max_iterations, stream, outcome, next, state);
+}
+
+} // namespace pm

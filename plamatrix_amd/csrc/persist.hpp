@@ -1,0 +1,75 @@
+// Persistent single-reduction CG / Jacobi-PCG on the diagonal layout: one
+// cooperative launch runs a whole solve (persist.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "dia.hpp"
+#include "workspace.hpp"
+
+namespace pm
+{
+
+// Largest chunk of iterations a solve's schedule grows to (adaptive_solve).
+constexpr int kMaxGrownChunk = 64;
+
+// A solve on the diagonal layout whose vectors sit where the per-kernel
+// iteration keeps them between chunks: r, u (z; Jacobi only), w (q), p (p0)
+// and s (p1), the partials of the initialisation in region 1.
+struct PersistProblem
+{
+    int64_t rows;
+    int32_t dtype;
+    const DiaLayout* dia;
+    bool jacobi;
+    const void* rhs;
+    void* x;
+    void *r, *u, *w, *p, *s;
+    const void* inv;
+    void* x_out;       // scratch vector the new x is written to before it is committed to x
+    SolverState* st;
+    double* region;    // partials of iteration t0 - 1 (t0 even)
+    int count;         // workgroups of the per-kernel iteration (its partial sums)
+    int refresh;       // residual refresh interval, 0: never
+    int chunk;         // the host's chunk schedule: first chunk, and whether chunks grow
+    bool grow;
+};
+
+enum PersistOutcome : int
+{
+    kPersistStopped = 1,   // the state record holds the end of the solve
+    kPersistHandOver = 2,  // after a restart: continue at iteration *next in the three-kernel form
+    kPersistAbandoned = 3, // nothing was committed: x is as before, start again in another form
+};
+
+// Whether the persistent iteration takes this solve.
+bool persist_wanted(const PersistProblem& p, int device);
+
+// Runs the solve and waits for it.  *state receives the final state record.
+int persist_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream, int* outcome,
+                int64_t* next, SolverState* state);
+
+// The chunk schedule of an adaptive solve: chunk c covers iterations
+// [end(c - 1), end(c)).  Both forms of a solve must leave the single-reduction
+// form at the same iteration after a restart.
+__host__ __device__ inline int64_t next_chunk(int64_t issued, int64_t size, bool grow, int64_t most)
+{
+    return grow && issued >= 2 && size < most ? size * 2 : size;
+}
+
+// The iteration a restart at iteration t hands over at: the chunk that holds t
+// and the one after it are already in flight when the host reads the flag.
+__host__ __device__ inline int64_t hand_over_iteration(int64_t t, int64_t first, bool grow, int64_t most)
+{
+    int64_t end = 0, size = first, issued = 0;
+    do
+    {
+        end += size;
+        size = next_chunk(++issued, size, grow, most);
+    } while (end <= t);
+    return end + size;
+}
+
+} // namespace pm

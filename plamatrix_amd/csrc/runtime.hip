@@ -173,6 +173,8 @@ pm_workspace::~pm_workspace()
     dia.release();
     dia_g.release();
     dia_gt.release();
+    blocks.release();
+    persist.release();
     for (hipEvent_t& e : events)
         if (e) (void)hipEventDestroy(e);
     if (done_event) (void)hipEventDestroy(done_event);
@@ -237,6 +239,8 @@ int pm_workspace_close(pm_workspace* ws)
     ws->dia.release();
     ws->dia_g.release();
     ws->dia_gt.release();
+    ws->blocks.release();
+    ws->persist.release();
     ws->capacity_rows = 0;
     ws->bound = false;
     ws->stream = nullptr;
@@ -249,7 +253,7 @@ size_t pm_workspace_capacity_bytes(const pm_workspace* ws)
     if (!ws) return 0;
     return ws->vectors.bytes + ws->partials.bytes + ws->state.bytes + ws->scratch.bytes + ws->sort.bytes +
            ws->refine.bytes + ws->batch.bytes + ws->dense.bytes +
-           ws->dia.bytes + ws->dia_g.bytes + ws->dia_gt.bytes;
+           ws->dia.bytes + ws->dia_g.bytes + ws->dia_gt.bytes + ws->blocks.bytes + ws->persist.bytes;
 }
 
 int64_t pm_workspace_capacity_rows(const pm_workspace* ws) { return ws ? ws->capacity_rows : 0; }

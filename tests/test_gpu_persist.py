@@ -1,0 +1,104 @@
+"""The persistent CG / Jacobi-PCG (plamatrix_amd/csrc/persist.hip): one launch per
+solve, rows kept in registers.  It sums in the per-kernel iteration's order, so
+a solve must be bitwise the one with PLAMATRIX_AMD_PERSISTENT=0: iterations,
+residual and solution, at every number of rows per lane, with and without
+diagonals that reach past the halos, with a short last piece, with refreshes
+and at iteration limits around the launch's first decisions.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+from plamatrix_amd import capi, generators  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    capi.lib()
+    return torch.device("cuda:0")
+
+
+def matrix(kind, dims, dtype):
+    if kind == "diffusion":  # unit diagonal: the unpreconditioned kernels
+        return generators.diffusion3d_box_csr(*dims, seed=5, dtype=dtype)
+    h = generators.laplacian2d_csr(*dims, dtype=dtype)  # diagonal 4: the Jacobi kernels
+    if kind == "varied":  # a diagonal that differs from row to row
+        rows = np.repeat(np.arange(h.rows), np.diff(h.row_offsets))
+        on = rows == h.col_indices
+        h.values[on] += np.random.default_rng(3).random(h.rows).astype(dtype)
+    return h
+
+
+def solve(a, b, monkeypatch, persistent, refresh, rel, most, solver=capi.pcg, x0=None):
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", persistent)
+    ws = capi.Workspace()
+    x = torch.zeros_like(b) if x0 is None else x0.clone()
+    out = []
+    for _ in range(2):  # the second solve meets the first one's exchange words
+        y = x.clone()
+        rep = solver(a, b, y, ws, capi.policy(refresh_interval=refresh), relative_tolerance=rel, max_iterations=most)
+        torch.cuda.synchronize()
+        out.append((rep.converged, rep.iterations, rep.initial_residual, rep.final_residual, y.cpu().numpy().tobytes()))
+    assert ws.solver_diagonals > 0 and ws.solver_form == 1
+    assert out[0] == out[1]
+    return out[0], ws.capacity_bytes
+
+
+CASES = [
+    # rows per lane 1: all neighbours in halos; the halo wider than the inner
+    # diagonal; outermost diagonals past the halos; a short last piece
+    ("laplace", (256, 256), np.float64, 0),
+    ("varied", (2100, 33), np.float64, 20),
+    ("laplace", (33, 2100), np.float32, 0),
+    ("diffusion", (41, 43, 40), np.float32, 50),
+    ("diffusion", (41, 43, 40), np.float64, 0),
+    # 2 and 4 rows per lane, uneven chunks per wavefront
+    ("laplace", (517, 601), np.float64, 0),
+    ("varied", (701, 760), np.float32, 50),
+    ("diffusion", (71, 70, 67), np.float32, 20),
+    ("laplace", (850, 830), np.float64, 50),
+    ("diffusion", (97, 89, 91), np.float32, 0),
+    # 8 (FP32): x and the inner diagonals in LDS
+    ("diffusion", (109, 107, 103), np.float32, 50),
+    ("laplace", (1200, 1001), np.float32, 20),
+]
+
+
+@pytest.mark.parametrize("kind,dims,dtype,refresh", CASES)
+def test_persistent_solve_is_bitwise(dev, monkeypatch, kind, dims, dtype, refresh):
+    a = capi.to_device_csr(matrix(kind, dims, dtype), compact=True)
+    b = torch.from_numpy(generators.rhs_normal(a.rows, seed=17).astype(dtype)).to(dev)
+    ref, without = solve(a, b, monkeypatch, "0", refresh, 1e-4, 400)
+    got, with_ = solve(a, b, monkeypatch, "1", refresh, 1e-4, 400)
+    assert with_ > without  # the exchange words were allocated: the persistent kernel ran
+    assert got == ref
+
+
+@pytest.mark.parametrize("most", [0, 1, 2, 3, 50])
+def test_iteration_limits(dev, monkeypatch, most):
+    a = capi.to_device_csr(matrix("laplace", (300, 290), np.float64), compact=False)
+    b = torch.from_numpy(generators.rhs_uniform(a.rows, seed=2)).to(dev)
+    x0 = torch.from_numpy(generators.rhs_uniform(a.rows, seed=3)).to(dev)
+    for solver in (capi.cg, capi.pcg):
+        ref, _ = solve(a, b, monkeypatch, "0", 0, 1e-10, most, solver, x0)
+        got, _ = solve(a, b, monkeypatch, "1", 0, 1e-10, most, solver, x0)
+        assert got == ref and got[1] == most and not got[0]
+
+
+def test_stops_at_the_start(dev, monkeypatch):
+    # the first decision already converges: x must come back as it was
+    a = capi.to_device_csr(matrix("laplace", (300, 290), np.float64), compact=True)
+    b = torch.zeros(a.rows, dtype=torch.float64, device=dev)
+    got, _ = solve(a, b, monkeypatch, "1", 0, 1e-8, 100)
+    assert got[0] and got[1] == 0 and not np.frombuffer(got[4], np.uint8).any()
+    # a NaN right-hand side is rejected with x untouched
+    b[7] = float("nan")
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "1")
+    x = torch.full_like(b, 2.0)
+    with pytest.raises(capi.PlamatrixError):
+        capi.pcg(a, b, x, capi.Workspace(), relative_tolerance=1e-8, max_iterations=100)
+    assert bool((x == 2.0).all())
