@@ -517,16 +517,32 @@ __global__ __launch_bounds__(kBlock) void k_gemm_wgrad(int64_t n, const __bf16* 
     for (int i = threadIdx.x; i < K * kHid; i += kBlock) part[static_cast<int64_t>(blockIdx.x) * K * kHid + i] = tile[i];
 }
 
-// out[i] = sum over b of part[b][i] in block order.
-__global__ __launch_bounds__(kBlock) void k_reduce_parts(const float* __restrict__ part, int blocks, int width,
-                                                         float* __restrict__ out)
+// out[i] = sum over b of part[b][i], in a fixed order: a workgroup takes 64
+// consecutive outputs with 16 wavefronts, wavefront g the partials g, g + 16,
+// ... (every load of a wavefront one 256-byte line, eight in flight), then the
+// 16 sums of an output are added in order.  The partials are read once, 13 MB
+// for a 128 x 64 weight at 13,200 rows; one thread per output walking all of
+// them was one load after the other on 32 workgroups, or on one (118 us
+// whatever the width, 1,060 us of a training step; 5 us now).
+constexpr int kReduceGroups = 16;
+__global__ __launch_bounds__(kWave* kReduceGroups) void k_reduce_parts(const float* __restrict__ part, int blocks,
+                                                                      int width, float* __restrict__ out)
 {
-    for (int64_t i = gid(); i < width; i += gstr())
+    __shared__ float sums[kReduceGroups][kWave];
+    const int lane = threadIdx.x % kWave, group = threadIdx.x / kWave;
+    const int i = static_cast<int>(blockIdx.x) * kWave + lane;
+    float s = 0.f;
+    if (i < width)
     {
-        float s = 0.f;
-        for (int b = 0; b < blocks; ++b) s += part[static_cast<int64_t>(b) * width + i];
-        out[i] = s;
+#pragma unroll 8
+        for (int b = group; b < blocks; b += kReduceGroups) s += part[static_cast<int64_t>(b) * width + i];
     }
+    sums[group][lane] = s;
+    __syncthreads();
+    if (group != 0 || i >= width) return;
+#pragma unroll
+    for (int g = 1; g < kReduceGroups; ++g) s += sums[g][lane];
+    out[i] = s;
 }
 
 // ---- graph kernels ----------------------------------------------------------------
@@ -786,22 +802,38 @@ __global__ __launch_bounds__(kBlock) void k_select_systems(int64_t systems, cons
     }
 }
 
-// loss and per-probe scale c_p = 1 / (P ||z_p||^2); stat[0] = loss.
-__global__ void k_loss(const double* __restrict__ part, int blocks, int probes, double* __restrict__ stat)
+// loss and per-probe scale c_p = 1 / (P ||z_p||^2); stat[0] = loss.  One
+// workgroup: thread (group, column) sums every 64th partial of its column (r.r
+// and z.z of each probe), the 64 sums of a column are added in order.  (One
+// thread walking all 512 x 16 partials took 398 us of a training step; 4 now.)
+constexpr int kLossGroups = 64;
+__global__ __launch_bounds__(kLossGroups * 2 * kMaxProbes) void k_loss(const double* __restrict__ part, int blocks,
+                                                                       int probes, double* __restrict__ stat)
 {
+    constexpr int kColumns = 2 * kMaxProbes;
+    __shared__ double sums[kLossGroups][kColumns];
+    __shared__ double total[kColumns];
+    const int column = threadIdx.x % kColumns, group = threadIdx.x / kColumns;
+    double s = 0.0;
+#pragma unroll 8
+    for (int b = group; b < blocks; b += kLossGroups) s += part[static_cast<int64_t>(b) * kColumns + column];
+    sums[group][column] = s;
+    __syncthreads();
+    if (group == 0)
+    {
+#pragma unroll
+        for (int g = 1; g < kLossGroups; ++g) s += sums[g][column];
+        total[column] = s;
+    }
+    __syncthreads();
     if (threadIdx.x != 0) return;
     double loss = 0.0;
     for (int p = 0; p < probes; ++p)
     {
-        double rr = 0.0, zz = 0.0;
-        for (int b = 0; b < blocks; ++b)
-        {
-            rr += part[static_cast<int64_t>(b) * 2 * kMaxProbes + p];
-            zz += part[static_cast<int64_t>(b) * 2 * kMaxProbes + kMaxProbes + p];
-        }
+        const double zz = total[kMaxProbes + p];
         const double c = zz > 0.0 ? 1.0 / (probes * zz) : 0.0;
         stat[1 + p] = c;
-        loss += rr * c;
+        loss += total[p] * c;
     }
     stat[0] = loss;
 }
@@ -1269,7 +1301,7 @@ int net_loss_grad(pm_fsai_net* net, pm_fsai_graph* gr, const Act& a, int probes,
     spmm(gr->lro, gr->lci, gr->g, true, a.v, a.w);       // w = G v
     double* dpart = reinterpret_cast<double*>(gr->parts.as<char>());
     hipLaunchKernelGGL(k_residual_probes, dim3(kPartBlocks), dim3(kBlock), 0, stream, n, probes, a.z, a.w, a.r, dpart);
-    hipLaunchKernelGGL(k_loss, dim3(1), dim3(64), 0, stream, dpart, kPartBlocks, probes, a.stat);
+    hipLaunchKernelGGL(k_loss, dim3(1), dim3(kLossGroups * 2 * kMaxProbes), 0, stream, dpart, kPartBlocks, probes, a.stat);
     hipLaunchKernelGGL(k_scale_probes, dim3(gn), dim3(kBlock), 0, stream, n, probes, a.stat, a.r);  // r := dL/dw
     spmm(gr->uro, gr->uci, gr->gt, true, a.r, a.q);      // q = G^T dL/dw = dL/dv
     spmm(gr->ro, gr->ci, gr->values, false, a.q, a.u);   // u := A q = dL/du
@@ -1283,19 +1315,22 @@ int net_loss_grad(pm_fsai_net* net, pm_fsai_graph* gr, const Act& a, int probes,
     const __bf16* w = net->w.as<__bf16>();
     const int gr_rows = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, 4), 16384)));
     const int gw = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(ceil_div(ceil_div(n, 16), 4), 8192)));
+    auto reduce = [&](int blocks, int width, float* out) {
+        hipLaunchKernelGGL(k_reduce_parts, dim3(static_cast<unsigned>(ceil_div(width, kWave))),
+                           dim3(kWave * kReduceGroups), 0, stream, part, blocks, width, out);
+    };
+    // workgroups of the weight gradients: no more than there are 32-row strips
+    const int strips = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, 32), kPartBlocks)));
     hipLaunchKernelGGL(k_decode_back, dim3(kPartBlocks), dim3(kBlock), 0, stream, n, gr->lro, gr->lci, gr->lsrc,
                        gr->uro, gr->uci, gr->uperm, gr->s, a.h[kLayers], P, a.dout, a.dh, part);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(1), dim3(kBlock), 0, stream, part, kPartBlocks, kDecParams,
-                       grad + kOffWoff);
+    reduce(kPartBlocks, kDecParams, grad + kOffWoff);
     for (int l = kLayers; l >= 1; --l)
     {
         hipLaunchKernelGGL(k_relu_back, dim3(kPartBlocks), dim3(kBlock), 0, stream, n, a.dh, a.h[l], a.dp, part);
-        hipLaunchKernelGGL(k_reduce_parts, dim3(1), dim3(kBlock), 0, stream, part, kPartBlocks, kHid,
-                           grad + kOffBl + (l - 1) * kHid);
-        hipLaunchKernelGGL(k_gemm_wgrad<2 * kHid>, dim3(kPartBlocks), dim3(kBlock), 0, stream, n, a.h[l - 1], a.m[l],
+        reduce(kPartBlocks, kHid, grad + kOffBl + (l - 1) * kHid);
+        hipLaunchKernelGGL(k_gemm_wgrad<2 * kHid>, dim3(strips), dim3(kBlock), 0, stream, n, a.h[l - 1], a.m[l],
                            a.dp, part);
-        hipLaunchKernelGGL(k_reduce_parts, dim3(grid_of(2 * kHid * kHid)), dim3(kBlock), 0, stream, part,
-                           kPartBlocks, 2 * kHid * kHid, grad + kOffWl + (l - 1) * 2 * kHid * kHid);
+        reduce(strips, 2 * kHid * kHid, grad + kOffWl + (l - 1) * 2 * kHid * kHid);
         // [dH, dM] = dP W_l^T: the GEMM's B^T operand is W_l itself (2kHid x kHid row-major)
         const __bf16* wl = w + kFeat * kHid + (l - 1) * 2 * kHid * kHid;
         hipLaunchKernelGGL((k_gemm<kHid, 2 * kHid>), dim3(gw), dim3(kBlock), 0, stream, n, a.dp, nullptr, wl, a.y);
@@ -1304,10 +1339,9 @@ int net_loss_grad(pm_fsai_net* net, pm_fsai_graph* gr, const Act& a, int probes,
                            a.dh);
     }
     hipLaunchKernelGGL(k_relu_back, dim3(kPartBlocks), dim3(kBlock), 0, stream, n, a.dh, a.h[0], a.dp, part);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(1), dim3(kBlock), 0, stream, part, kPartBlocks, kHid, grad + kOffBin);
-    hipLaunchKernelGGL(k_gemm_wgrad<kFeat>, dim3(kPartBlocks), dim3(kBlock), 0, stream, n, gr->x, nullptr, a.dp, part);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(grid_of(kFeat * kHid)), dim3(kBlock), 0, stream, part, kPartBlocks,
-                       kFeat * kHid, grad + kOffWin);
+    reduce(kPartBlocks, kHid, grad + kOffBin);
+    hipLaunchKernelGGL(k_gemm_wgrad<kFeat>, dim3(strips), dim3(kBlock), 0, stream, n, gr->x, nullptr, a.dp, part);
+    reduce(strips, kFeat * kHid, grad + kOffWin);
     PM_HIP(hipGetLastError());
     return PM_OK;
 }
