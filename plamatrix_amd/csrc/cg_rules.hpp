@@ -43,17 +43,21 @@ __device__ __forceinline__ CgDecision cg_rules(const CgHistory& h, int completed
 {
     CgDecision d;
     d.restart = false;
+    // independent of each other and of the branches below, so that their
+    // latencies overlap: this runs in one thread while the others wait
+    const double root = sqrt(rr);
+    const double ratio = gamma / h.gamma_prev;
     // the accelerated solvers' max(abs, rel ||r0||), or the reference CPU
     // Schur solver's abs + rel ||r0|| (block_schur_cpu_solver.h:34-35)
     d.tol = completed != 0 ? h.tol
-            : h.tol_rule   ? h.abs_tol + h.rel_tol * sqrt(rr)
-                           : fmax(h.abs_tol, h.rel_tol * sqrt(rr));
+            : h.tol_rule   ? h.abs_tol + h.rel_tol * root
+                           : fmax(h.abs_tol, h.rel_tol * root);
     d.code = kRunning;
     d.beta = 0.0;
     d.alpha = 0.0;
     d.den = delta;
     if (!isfinite(rr) || rr < 0.0) d.code = completed == 0 ? kInitNonFinite : kNonFinite;
-    else if (sqrt(rr) <= d.tol) d.code = kConverged;
+    else if (root <= d.tol) d.code = kConverged;
     else if (completed == 0 && h.bad_diagonal) d.code = kBadDiagonal;
     else if (completed >= h.max_iterations) d.code = kIterationLimit;
     else
@@ -64,7 +68,7 @@ __device__ __forceinline__ CgDecision cg_rules(const CgHistory& h, int completed
             if (h.gamma_prev == 0.0 && gamma == 0.0) d.beta = 0.0;
             else if (isfinite(h.gamma_prev) && isfinite(gamma) && h.gamma_prev > 0.0 && gamma > 0.0)
             {
-                d.beta = gamma / h.gamma_prev;
+                d.beta = ratio;
                 if (!isfinite(d.beta) || !isfinite(static_cast<S>(d.beta))) d.code = kBreakdown;
             }
             else d.code = kBreakdown;

@@ -2265,13 +2265,14 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     std::deque<int64_t> inflight;
     int64_t launched = 0;
     int64_t chunk_id = 0;
-    if (pb.cg_fused && !pb.cg_factored)
+    if (pb.single_reduction && !pb.cg_factored)
     {
-        // the one-kernel iteration of a matrix whose rows fit the register
-        // files runs as one launch for the whole solve
+        // a solve whose rows fit the register files runs as one launch: on the
+        // diagonal layout over all CUs, a small CSR matrix in one workgroup
         PersistProblem pp{};
         pp.rows = a->rows;
         pp.dtype = a->dtype;
+        pp.a = a;
         pp.dia = &pb.dia;
         pp.jacobi = pb.pre == kPreJacobi;
         pp.rhs = rhs;
@@ -2289,11 +2290,13 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
         pp.refresh = policy.refresh;
         pp.chunk = policy.chunk;
         pp.grow = policy.grow;
-        if (persist_wanted(pp, ws->device))
+        const bool wide = pb.cg_fused && persist_wanted(pp, ws->device);
+        if (wide || (!pb.dia.active && persist_small_wanted(pp)))
         {
             int outcome = 0;
             int64_t next = 0;
-            PM_TRY(persist_run(ws, pp, options->max_iterations, stream, &outcome, &next, &fin));
+            const auto run = wide ? persist_run : persist_small_run;
+            PM_TRY(run(ws, pp, options->max_iterations, stream, &outcome, &next, &fin));
             if (outcome == kPersistStopped)
             {
                 PM_HIP(hipEventRecord(ws->done_event, stream));

@@ -42,7 +42,7 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "cg_rules.hpp"
+#include "persist_history.hpp"
 #include "spmv_kernels.hpp"
 
 namespace pm
@@ -58,11 +58,8 @@ constexpr int kPersistGroups = kPersistThreads / kBlock;  // per-kernel workgrou
 constexpr int kPersistBlocks = kSolverGrid / kPersistGroups;
 constexpr int kRedEntries = kSolverGrid - kBlock;
 constexpr int kDecWords = 16;        // one 128-byte line per workgroup
-constexpr int kHandOver = 100;       // decision code: leave without deciding
 constexpr int kWaitSeconds = 4;
 constexpr int64_t kSegment = 8192;   // iterations per launch
-constexpr int kCounterOutcome = 1;   // SolverState::counters slot: 1 committed
-constexpr int kCounterNext = 2;      // ... iteration the launch handed over at
 
 struct PersistControl
 {
@@ -71,15 +68,6 @@ struct PersistControl
     unsigned pad[62];
     word part[2][kCgValues][2][kSolverGrid];  // parity, value, half, per-kernel workgroup
     word dec[kPersistBlocks][kDecWords];
-};
-
-// What thread 0 of a leading workgroup keeps between decisions (in LDS: as
-// registers it would take some from every lane).
-struct PersistHistory
-{
-    CgHistory h;
-    double rr, rr0, alpha;
-    int completed, t_stop, restarted;
 };
 
 template <typename S>
@@ -102,7 +90,7 @@ struct PersistArgs
     unsigned tag;  // tags of this launch are above it
     int count, per, halo, leaders, refresh;
     int t0, t_end;
-    int chunk, grow, most;
+    int chunk, grow;
     int span;  // local rows that the LDS arrays hold
     int priv, red;  // bytes of LDS before x and the inner diagonals, and before the leaders' reduction
 };
@@ -304,16 +292,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
 
     // thread 0 of a leading workgroup holds the history of the decisions
     const bool leader = bid < a.leaders;
-    if (leader && tid == 0)
-    {
-        hs.h = CgHistory{a.st->max_iterations, a.st->tol_rule, a.st->rel_tol, a.st->abs_tol,
-                         a.st->tol,            a.st->rho[1],   a.st->den[1],  a.st->bad_row != ~0ull};
-        hs.completed = a.st->iter[1] + 1;
-        hs.rr0 = a.st->rr0;
-        hs.rr = hs.alpha = 0.0;
-        hs.t_stop = a.t_end;
-        hs.restarted = 0;
-    }
+    if (leader && tid == 0) hs.begin(a.st, a.t_end);
     if (tid == 0) sh_fail = 0;
     __syncthreads();
 
@@ -495,13 +474,8 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
             }
             if (tid < kBlock)
             {
-#pragma unroll
-                for (int v = 0; v < NV; ++v) acc[v] = wave_sum(acc[v]);
-                if (lane == 0)
-                {
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) lds_w[v][wave] = acc[v];
-                }
+                const double sum = wave_sum4(acc[0], acc[1], acc[2], acc[NV - 1]);
+                if (lane % 16 == 0) lds_w[lane / 16][wave] = sum;
             }
             if (!fine) sh_fail = 1;
             __syncthreads();
@@ -516,29 +490,8 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
                     for (int z = 0; z < kBlock / kWave; ++z) q += lds_w[v][z];
                     tot[v] = q;
                 }
-                int c = kHandOver;
-                if (t < hs.t_stop)
-                {
-                    const CgDecision d =
-                        cg_rules<S>(hs.h, hs.completed, tot[0], tot[UNIT ? 0 : 1], tot[NV - 2], tot[NV - 1]);
-                    c = d.code;
-                    sh_alpha = static_cast<S>(d.alpha);
-                    sh_beta = static_cast<S>(d.beta);
-                    hs.rr = tot[0];
-                    hs.alpha = d.alpha;
-                    if (hs.completed == 0) hs.rr0 = tot[0];
-                    hs.h.tol = d.tol;
-                    hs.h.gamma_prev = tot[UNIT ? 0 : 1];
-                    hs.h.den_prev = d.den;
-                    if (d.restart && hs.restarted == 0)
-                    {
-                        hs.restarted = 1;
-                        const int64_t over = hand_over_iteration(t, a.chunk, a.grow != 0, a.most);
-                        if (over < hs.t_stop) hs.t_stop = static_cast<int>(over);
-                    }
-                    ++hs.completed;
-                }
-                sh_code = c;
+                sh_code = hs.decide<S>(t, tot[0], tot[UNIT ? 0 : 1], tot[NV - 2], tot[NV - 1], a.chunk, a.grow != 0,
+                                       sh_alpha, sh_beta);
             }
             __syncthreads();
             // the workgroups this leader answers to: bid + leaders, ...
@@ -621,13 +574,8 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
             part[NV - 2] = __builtin_fma(static_cast<double>(w[k]), uv, part[NV - 2]);
             part[NV - 1] = __builtin_fma(uv, static_cast<double>(s[k]), part[NV - 1]);
         }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) part[v] = wave_sum(part[v]);
-        if (lane == 0)
-        {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) lds_p[v][wave] = part[v];
-        }
+        const double sum = wave_sum4(part[0], part[1], part[2], part[NV - 1]);
+        if (lane % 16 == 0) lds_p[lane / 16][wave] = sum;
         __syncthreads();
         if (sh_fail != 0) return;
         if (tid < NV * kPersistGroups)
@@ -636,11 +584,11 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
             const int lb = g * kPersistGroups + q;
             if (lb < a.count)
             {
-                double sum = 0.0;
+                double group = 0.0;
 #pragma unroll
-                for (int z = 0; z < kWavesPerBlock; ++z) sum += lds_p[v][q * kWavesPerBlock + z];
+                for (int z = 0; z < kWavesPerBlock; ++z) group += lds_p[v][q * kWavesPerBlock + z];
                 const int vb = physical_block(lb, a.count);
-                Exchange<double>::put(&a.ctl->part[t & 1][v][0][vb], kSolverGrid, 0, sum, tag);
+                Exchange<double>::put(&a.ctl->part[t & 1][v][0][vb], kSolverGrid, 0, group, tag);
             }
         }
     }
@@ -678,23 +626,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
         a.region[2 * kMaxPartials + vb] = vals[NV - 2];
         a.region[3 * kMaxPartials + vb] = vals[NV - 1];
     }
-    if (bid == 0 && tid == 0)
-    {
-        // completed counts the decisions: the last one saw completed - 1 updates
-        const int seen = hs.completed - 1, par = seen & 1;
-        SolverState* st = a.st;
-        st->rr = hs.rr;
-        st->rr0 = hs.rr0;
-        st->tol = hs.h.tol;
-        st->iteration = seen;
-        st->iter[par] = seen;
-        st->rho[par] = hs.h.gamma_prev;
-        st->den[par] = hs.h.den_prev;
-        st->alpha = hs.alpha;
-        if (hs.restarted) st->counters[kCounterRestart] = 1u;
-        st->counters[kCounterNext] = static_cast<unsigned>(hs.completed);
-        if (!over) st->done = code;
-    }
+    if (bid == 0 && tid == 0) hs.record(a.st, code);
     __syncthreads();
     if (tid == 0) __hip_atomic_fetch_add(&a.ctl->finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -870,7 +802,6 @@ int persist_run_t(pm_workspace* ws, const PersistProblem& p, int64_t max_iterati
     a.refresh = p.refresh;
     a.chunk = p.chunk;
     a.grow = p.grow ? 1 : 0;
-    a.most = kMaxGrownChunk;
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(p.rows, kBlock), 2048));
     for (int64_t t = 0;; )
     {

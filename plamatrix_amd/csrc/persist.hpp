@@ -1,5 +1,6 @@
-// Persistent single-reduction CG / Jacobi-PCG on the diagonal layout: one
-// cooperative launch runs a whole solve (persist.hip).
+// Persistent single-reduction CG / Jacobi-PCG: one launch runs a whole solve,
+// cooperative on the diagonal layout (persist.hip), in one workgroup on small
+// CSR matrices (persist_small.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -15,13 +16,14 @@ namespace pm
 // Largest chunk of iterations a solve's schedule grows to (adaptive_solve).
 constexpr int kMaxGrownChunk = 64;
 
-// A solve on the diagonal layout whose vectors sit where the per-kernel
-// iteration keeps them between chunks: r, u (z; Jacobi only), w (q), p (p0)
-// and s (p1), the partials of the initialisation in region 1.
+// A solve whose vectors sit where the per-kernel iteration keeps them between
+// chunks: r, u (z; Jacobi only), w (q), p (p0) and s (p1), the partials of the
+// initialisation in region 1.
 struct PersistProblem
 {
     int64_t rows;
     int32_t dtype;
+    const pm_csr* a;
     const DiaLayout* dia;
     bool jacobi;
     const void* rhs;
@@ -44,12 +46,17 @@ enum PersistOutcome : int
     kPersistAbandoned = 3, // nothing was committed: x is as before, start again in another form
 };
 
-// Whether the persistent iteration takes this solve.
+// Whether the persistent iteration on the diagonal layout takes this solve.
 bool persist_wanted(const PersistProblem& p, int device);
 
 // Runs the solve and waits for it.  *state receives the final state record.
 int persist_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream, int* outcome,
                 int64_t* next, SolverState* state);
+
+// The same for the one-workgroup solve of a small CSR matrix.
+bool persist_small_wanted(const PersistProblem& p);
+int persist_small_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream,
+                      int* outcome, int64_t* next, SolverState* state);
 
 // The chunk schedule of an adaptive solve: chunk c covers iterations
 // [end(c - 1), end(c)).  Both forms of a solve must leave the single-reduction

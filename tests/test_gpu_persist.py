@@ -102,3 +102,77 @@ def test_stops_at_the_start(dev, monkeypatch):
     with pytest.raises(capi.PlamatrixError):
         capi.pcg(a, b, x, capi.Workspace(), relative_tolerance=1e-8, max_iterations=100)
     assert bool((x == 2.0).all())
+
+
+def ragged(n, seed, long_row=0, dtype=np.float64):
+    """SPD matrix with 1 to 14 entries a row and, if asked, one long row."""
+    import scipy.sparse as sp
+
+    rng = np.random.default_rng(seed)
+    k = rng.integers(0, 7, n)
+    i = np.repeat(np.arange(n), k)
+    j = rng.integers(0, n, len(i))
+    if long_row:
+        i = np.concatenate([i, np.full(long_row, n // 2)])
+        j = np.concatenate([j, rng.permutation(n)[:long_row]])
+    m = sp.csr_matrix((rng.standard_normal(len(i)), (i, j)), shape=(n, n))
+    m = (m + m.T).tocsr()
+    m = (m + sp.diags(np.asarray(abs(m).sum(axis=1)).ravel() * rng.uniform(1.0, 1.4, n) + 0.1)).tocsr()
+    m.sort_indices()
+    return generators.CSRHost(n, n, m.indptr.astype(np.int64), m.indices.astype(np.int64), m.data.astype(dtype))
+
+
+SMALL = [
+    (ragged(1, 1), 0), (ragged(63, 2), 4), (ragged(257, 3, dtype=np.float32), 0), (ragged(1025, 4), 20),
+    (ragged(1100, 5, long_row=900), 6), (ragged(2049, 6, dtype=np.float32), 20), (ragged(4096, 7), 0),
+    (ragged(3001, 8, long_row=2500, dtype=np.float32), 0),  # a chunk of more than 2,048 entries: the per-kernel solve
+    (generators.laplacian2d_csr(45, 37), 0), (generators.laplacian2d_csr(64, 64, dtype=np.float32), 50),
+]
+
+
+@pytest.mark.parametrize("index", range(len(SMALL)))
+@pytest.mark.parametrize("compact", [False, True])
+def test_one_workgroup_solve_is_bitwise(dev, monkeypatch, index, compact):
+    h, refresh = SMALL[index]
+    a = capi.to_device_csr(h, compact=compact)
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=19).astype(h.values.dtype)).to(dev)
+    rel = 1e-10 if h.values.dtype == np.float64 else 1e-5
+    for solver in (capi.pcg, capi.cg):
+        for most in (0, 1, 3, 4000):
+            out = {}
+            for flag in ("0", "1"):
+                monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+                ws = capi.Workspace()
+                x = torch.full_like(b, 0.25)
+                rep = solver(a, b, x, ws, capi.policy(refresh_interval=refresh), relative_tolerance=rel,
+                             max_iterations=most)
+                torch.cuda.synchronize()
+                assert ws.solver_form == 2
+                out[flag] = (rep.converged, rep.iterations, rep.initial_residual, rep.final_residual,
+                             x.cpu().numpy().tobytes())
+            assert out["0"] == out["1"], (solver.__name__, most)
+
+
+def test_one_workgroup_errors(dev, monkeypatch):
+    # a rejected diagonal, an indefinite matrix (restart, hand-over, breakdown):
+    # the per-kernel solve's errors
+    h = generators.laplacian2d_csr(30, 30)
+    rows = np.repeat(np.arange(h.rows), np.diff(h.row_offsets))
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=23).astype(np.float64)).to(dev)
+    for row, value in ((100, -1.0), (None, 1.5)):
+        v = h.values.copy()
+        on = (rows == h.col_indices) & ((rows == row) if row is not None else True)
+        v[on] = value
+        a = capi.to_device_csr(generators.CSRHost(h.rows, h.cols, h.row_offsets, h.col_indices, v), compact=True)
+        out = {}
+        for flag in ("0", "1"):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+            x = torch.zeros_like(b)
+            try:
+                rep = capi.pcg(a, b, x, capi.Workspace(), relative_tolerance=1e-9, max_iterations=500)
+                out[flag] = ("ok", rep.iterations, rep.final_residual, x.cpu().numpy().tobytes())
+            except capi.PlamatrixError as e:
+                out[flag] = (e.kind, str(e))
+        assert out["0"] == out["1"]
+        if row is not None:
+            assert "diagonal" in out["1"][1] and f"row {row}" in out["1"][1]
