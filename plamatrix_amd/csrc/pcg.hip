@@ -1541,6 +1541,7 @@ struct Problem
     bool long_rows;          // classic CSR SpMV with kLongLanes lanes per row (few long rows)
     // workspace vectors
     void *r, *z, *q, *p0, *p1, *inv;
+    void* spare;             // a seventh vector: where a persistent solve leaves x until it is committed (r2's storage)
     void *r2, *z2, *q2, *s2; // second buffers of r, u, w, s for the one-kernel iteration (or null)
     SolverState* st;
     double* partials;
@@ -1987,7 +1988,7 @@ int prepare(pm_workspace* ws, Problem& pb, hipStream_t stream)
     // a matrix the diagonal layout may take also gets the second buffers of
     // the one-kernel single-reduction iteration
     const bool second = dia_wanted(pb.a);
-    PM_TRY(ws->vectors.reserve(vec * (second ? 10 : 6)));
+    PM_TRY(ws->vectors.reserve(vec * (second ? 10 : 7)));
     if (n > ws->capacity_rows) ws->capacity_rows = n;
     PM_TRY(ws->partials.reserve(sizeof(double) * kPartialsDoubles));
     PM_TRY(ws->state.reserve(4096));
@@ -1998,6 +1999,7 @@ int prepare(pm_workspace* ws, Problem& pb, hipStream_t stream)
     pb.p0 = base + 3 * vec;
     pb.p1 = base + 4 * vec;
     pb.inv = base + 5 * vec;
+    pb.spare = base + 6 * vec;
     pb.r2 = second ? base + 6 * vec : nullptr;
     pb.z2 = second ? base + 7 * vec : nullptr;
     pb.q2 = second ? base + 8 * vec : nullptr;
@@ -2254,7 +2256,45 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
         PM_HIP(hipGetLastError());
         return get_plan<S>(ws, pb, 0, 0, 0, 0)->run(stream, false);
     };
+    // a solve whose rows fit the register files runs as one launch: on the
+    // diagonal layout over all CUs, a small CSR matrix in one workgroup, another
+    // of short local rows with a row per lane (the device looks at its rows
+    // ahead of the initialisation)
+    PersistProblem pp{};
+    pp.rows = a->rows;
+    pp.dtype = a->dtype;
+    pp.a = a;
+    pp.dia = &pb.dia;
+    pp.jacobi = pb.pre == kPreJacobi;
+    pp.rhs = rhs;
+    pp.x = x;
+    pp.r = pb.r;
+    pp.u = pb.z;
+    pp.w = pb.q;
+    pp.p = pb.p0;
+    pp.s = pb.p1;
+    pp.inv = pb.inv;
+    pp.x_out = pb.spare;
+    pp.st = pb.st;
+    pp.region = cg_region(pb.partials, 1);
+    pp.count = pb.grid_units;
+    pp.refresh = policy.refresh;
+    pp.chunk = policy.chunk;
+    pp.grow = policy.grow;
+    const bool one_launch = pb.single_reduction && !pb.cg_factored;
+    const bool csr = one_launch && !pb.dia.active;
+    auto run = one_launch && pb.cg_fused && persist_wanted(pp, ws->device) ? persist_run
+               : csr && persist_small_wanted(pp)                           ? persist_small_run
+                                                                           : nullptr;
+    const bool look = csr && run == nullptr && persist_csr_candidate(pp, ws->device);
+    if (look) PM_TRY(persist_csr_look(ws, pp, stream));
     PM_TRY(initialise());
+    if (look)
+    {
+        bool fits = false;
+        PM_TRY(persist_csr_fits(ws, &fits));
+        if (fits) run = persist_csr_run;
+    }
 
     // iteration t = max_iterations must run its first kernel to record the
     // final decision, so chunks cover iterations [0, max_iterations].
@@ -2265,54 +2305,26 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     std::deque<int64_t> inflight;
     int64_t launched = 0;
     int64_t chunk_id = 0;
-    if (pb.single_reduction && !pb.cg_factored)
+    if (run != nullptr)
     {
-        // a solve whose rows fit the register files runs as one launch: on the
-        // diagonal layout over all CUs, a small CSR matrix in one workgroup
-        PersistProblem pp{};
-        pp.rows = a->rows;
-        pp.dtype = a->dtype;
-        pp.a = a;
-        pp.dia = &pb.dia;
-        pp.jacobi = pb.pre == kPreJacobi;
-        pp.rhs = rhs;
-        pp.x = x;
-        pp.r = pb.r;
-        pp.u = pb.z;
-        pp.w = pb.q;
-        pp.p = pb.p0;
-        pp.s = pb.p1;
-        pp.inv = pb.inv;
-        pp.x_out = pb.r2;
-        pp.st = pb.st;
-        pp.region = cg_region(pb.partials, 1);
-        pp.count = pb.grid_units;
-        pp.refresh = policy.refresh;
-        pp.chunk = policy.chunk;
-        pp.grow = policy.grow;
-        const bool wide = pb.cg_fused && persist_wanted(pp, ws->device);
-        if (wide || (!pb.dia.active && persist_small_wanted(pp)))
+        int outcome = 0;
+        int64_t next = 0;
+        PM_TRY(run(ws, pp, options->max_iterations, stream, &outcome, &next, &fin));
+        if (outcome == kPersistStopped)
         {
-            int outcome = 0;
-            int64_t next = 0;
-            const auto run = wide ? persist_run : persist_small_run;
-            PM_TRY(run(ws, pp, options->max_iterations, stream, &outcome, &next, &fin));
-            if (outcome == kPersistStopped)
+            PM_HIP(hipEventRecord(ws->done_event, stream));
+            return finish_report(fin, options, report);
+        }
+        if (outcome == kPersistAbandoned) PM_TRY(initialise());
+        else
+        {
+            // a restart: the three-kernel form from iteration `next` on,
+            // with the chunks the schedule has there
+            pb.single_reduction = pb.cg_fused = false;
+            while (launched < next)
             {
-                PM_HIP(hipEventRecord(ws->done_event, stream));
-                return finish_report(fin, options, report);
-            }
-            if (outcome == kPersistAbandoned) PM_TRY(initialise());
-            else
-            {
-                // a restart: the three-kernel form from iteration `next` on,
-                // with the chunks the schedule has there
-                pb.single_reduction = pb.cg_fused = false;
-                while (launched < next)
-                {
-                    launched += K;
-                    K = next_chunk(++chunk_id, K, policy.grow, kMaxGrownChunk);
-                }
+                launched += K;
+                K = next_chunk(++chunk_id, K, policy.grow, kMaxGrownChunk);
             }
         }
     }

@@ -39,36 +39,15 @@
 #include "persist.hpp"
 
 #include <algorithm>
-#include <cstdlib>
 #include <type_traits>
 
-#include "persist_history.hpp"
+#include "persist_launch.hpp"
 #include "spmv_kernels.hpp"
 
 namespace pm
 {
 namespace
 {
-
-using word = unsigned long long;
-
-constexpr int kPersistThreads = 1024;
-constexpr int kPersistWaves = kPersistThreads / kWave;
-constexpr int kPersistGroups = kPersistThreads / kBlock;  // per-kernel workgroups one workgroup stands for
-constexpr int kPersistBlocks = kSolverGrid / kPersistGroups;
-constexpr int kRedEntries = kSolverGrid - kBlock;
-constexpr int kDecWords = 16;        // one 128-byte line per workgroup
-constexpr int kWaitSeconds = 4;
-constexpr int64_t kSegment = 8192;   // iterations per launch
-
-struct PersistControl
-{
-    unsigned abort;
-    unsigned finished;
-    unsigned pad[62];
-    word part[2][kCgValues][2][kSolverGrid];  // parity, value, half, per-kernel workgroup
-    word dec[kPersistBlocks][kDecWords];
-};
 
 template <typename S>
 struct PersistArgs
@@ -95,106 +74,6 @@ struct PersistArgs
     int priv, red;  // bytes of LDS before x and the inner diagonals, and before the leaders' reduction
 };
 
-__device__ __forceinline__ word load_word(const word* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void store_word(word* p, unsigned v, unsigned tag)
-{
-    __hip_atomic_store(p, (static_cast<word>(tag) << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Word i of an exchange array (fewer than 2^29 words: a 32-bit byte offset from
-// a uniform base).
-__device__ __forceinline__ word* word_at(word* b, unsigned i)
-{
-    return reinterpret_cast<word*>(reinterpret_cast<char*>(b) + i * 8u);
-}
-__device__ __forceinline__ const word* word_at(const word* b, unsigned i)
-{
-    return reinterpret_cast<const word*>(reinterpret_cast<const char*>(b) + i * 8u);
-}
-__device__ __forceinline__ bool word_ready(word v, unsigned tag) { return static_cast<unsigned>(v >> 32) == tag; }
-
-// A value of the exchange: one word for FP32, two for FP64 (half planes).
-template <typename S>
-struct Exchange;
-template <>
-struct Exchange<float>
-{
-    static constexpr int kWords = 1;
-    __device__ static __forceinline__ void put(word* b, int, unsigned i, float v, unsigned tag)
-    {
-        store_word(word_at(b, i), __float_as_uint(v), tag);
-    }
-    __device__ static __forceinline__ void issue(const word* b, int, unsigned i, word (&w)[1])
-    {
-        w[0] = load_word(word_at(b, i));
-    }
-    __device__ static __forceinline__ float value(const word (&w)[1]) { return __uint_as_float(static_cast<unsigned>(w[0])); }
-};
-template <>
-struct Exchange<double>
-{
-    static constexpr int kWords = 2;
-    __device__ static __forceinline__ void put(word* b, int plane, unsigned i, double v, unsigned tag)
-    {
-        const word bits = static_cast<word>(__double_as_longlong(v));
-        store_word(word_at(b, i), static_cast<unsigned>(bits), tag);
-        store_word(word_at(b + plane, i), static_cast<unsigned>(bits >> 32), tag);
-    }
-    __device__ static __forceinline__ void issue(const word* b, int plane, unsigned i, word (&w)[2])
-    {
-        w[0] = load_word(word_at(b, i));
-        w[1] = load_word(word_at(b + plane, i));
-    }
-    __device__ static __forceinline__ double value(const word (&w)[2])
-    {
-        return __longlong_as_double(static_cast<long long>((w[1] << 32) | (w[0] & 0xffffffffull)));
-    }
-};
-template <typename S>
-__device__ __forceinline__ bool ready(const word (&w)[Exchange<S>::kWords], unsigned tag)
-{
-    bool ok = word_ready(w[0], tag);
-    if constexpr (Exchange<S>::kWords == 2) ok = ok && word_ready(w[1], tag);
-    return ok;
-}
-
-// The workgroup of the per-kernel iteration that owns logical block lb (the
-// inverse of xcd_logical_block).
-__device__ __forceinline__ int physical_block(int lb, int nb)
-{
-    const int q = nb / kXcds, r = nb % kXcds;
-    const int head = r * (q + 1);
-    const int xcd = lb < head ? lb / (q + 1) : r + (lb - head) / (q > 0 ? q : 1);
-    const int idx = lb < head ? lb % (q + 1) : (lb - head) % (q > 0 ? q : 1);
-    return idx * kXcds + xcd;
-}
-
-// Waits for words that other workgroups write: `poll` loads them and says
-// whether all carry their tag.  The whole wavefront polls together.
-template <typename Poll>
-__device__ __forceinline__ bool wait_for(PersistControl* ctl, Poll poll)
-{
-    unsigned polls = 0;
-    long long start = 0;
-    while (!__all(poll()))
-    {
-        // the bound of the wait: every 256 polls look at the clock (100 MHz)
-        // and at another workgroup's notice that it gave up
-        if ((++polls & 255u) != 0u) continue;
-        const long long now = wall_clock64();
-        if (start == 0) start = now;
-        if (__hip_atomic_load(&ctl->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ||
-            now - start > kWaitSeconds * 100000000ll)
-        {
-            __hip_atomic_store(&ctl->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-    }
-    return true;
-}
-
 // ND diagonals with symmetric offsets (ND / 2 is the main diagonal), R rows per
 // lane.  UNIT: an unpreconditioned solve whose main diagonal is all ones (u is
 // r); else the main diagonal is stored and u = inv r (inv of ones without a
@@ -216,11 +95,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
     // far words in flight per lane: FB rows of two
     constexpr int FB = R < 8 / (2 * X::kWords) ? R : 8 / (2 * X::kWords);
     extern __shared__ char lds_raw[];
-    __shared__ double lds_p[kCgValues][kPersistWaves];   // partial sums of the wavefronts
-    __shared__ double lds_w[kCgValues][kBlock / kWave];  // the decision's reduction
-    __shared__ S sh_alpha, sh_beta;
-    __shared__ int sh_code, sh_fail;
-    __shared__ PersistHistory hs;
+    __shared__ PersistShared<S> sh;
 
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int blocks = gridDim.x, bid = blockIdx.x;
@@ -290,10 +165,12 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
         else return x[k];
     };
 
-    // thread 0 of a leading workgroup holds the history of the decisions
-    const bool leader = bid < a.leaders;
-    if (leader && tid == 0) hs.begin(a.st, a.t_end);
-    if (tid == 0) sh_fail = 0;
+    const PersistWhere at{a.ctl, a.region, bid, blocks, g, a.count, a.leaders, a.t0, a.chunk, a.grow};
+    if (tid == 0)
+    {
+        sh.hs.begin(a.st, a.t_end);
+        sh.fail = 0;
+    }
     __syncthreads();
 
     // the lane's rows of a vector into LDS and, where another workgroup reads
@@ -400,7 +277,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
             if constexpr (FAR)
                 if (kb + FB < R) issue(kb + FB);
         }
-        if (!fine) sh_fail = 1;
+        if (!fine) sh.fail = 1;
     };
 
     int code = kRunning;
@@ -408,130 +285,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
     {
         // ---- decision: stop test, alpha, beta from the partials of t - 1 ----
         const unsigned tag = a.tag + static_cast<unsigned>(t - a.t0) + 1u;
-        if (leader)
-        {
-            bool fine = true;
-            auto entry = [&](int e, double (&out)[NV]) {
-                if (t == a.t0)
-                {
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) out[v] = a.region[(UNIT && v > 0 ? v + 1 : v) * kMaxPartials + e];
-                    return;
-                }
-                word hw[NV][2];
-                const word* at = &a.ctl->part[(t - 1) & 1][0][0][e];
-                fine = wait_for(a.ctl, [&] {
-                    bool ok = true;
-#pragma unroll
-                    for (int v = 0; v < NV; ++v)
-                    {
-                        hw[v][0] = load_word(at + (2 * v) * kSolverGrid);
-                        hw[v][1] = load_word(at + (2 * v + 1) * kSolverGrid);
-                    }
-#pragma unroll
-                    for (int v = 0; v < NV; ++v)
-                        ok = ok && word_ready(hw[v][0], tag - 1u) && word_ready(hw[v][1], tag - 1u);
-                    return ok;
-                });
-#pragma unroll
-                for (int v = 0; v < NV; ++v) out[v] = Exchange<double>::value(hw[v]);
-            };
-            double acc[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-            if (a.count <= kBlock)
-            {
-                if (tid < a.count)
-                {
-                    double e[NV];
-                    entry(tid, e);
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) acc[v] += e[v];
-                }
-            }
-            else
-            {
-                double e[NV];
-#pragma unroll
-                for (int v = 0; v < NV; ++v) e[v] = 0.0;
-                if (tid < a.count) entry(tid, e);
-                if (tid >= kBlock)
-                {
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) red[v * kRedEntries + tid - kBlock] = e[v];
-                }
-                __syncthreads();
-                if (tid < kBlock)
-                {
-#pragma unroll
-                    for (int v = 0; v < NV; ++v)
-                    {
-                        acc[v] += e[v];
-#pragma unroll
-                        for (int j = 0; j < kRedEntries / kBlock; ++j) acc[v] += red[v * kRedEntries + tid + j * kBlock];
-                    }
-                }
-            }
-            if (tid < kBlock)
-            {
-                const double sum = wave_sum4(acc[0], acc[1], acc[2], acc[NV - 1]);
-                if (lane % 16 == 0) lds_w[lane / 16][wave] = sum;
-            }
-            if (!fine) sh_fail = 1;
-            __syncthreads();
-            if (tid == 0)
-            {
-                double tot[NV];
-#pragma unroll
-                for (int v = 0; v < NV; ++v)
-                {
-                    double q = 0.0;
-#pragma unroll
-                    for (int z = 0; z < kBlock / kWave; ++z) q += lds_w[v][z];
-                    tot[v] = q;
-                }
-                sh_code = hs.decide<S>(t, tot[0], tot[UNIT ? 0 : 1], tot[NV - 2], tot[NV - 1], a.chunk, a.grow != 0,
-                                       sh_alpha, sh_beta);
-            }
-            __syncthreads();
-            // the workgroups this leader answers to: bid + leaders, ...
-            const int who = bid + (tid + 1) * a.leaders;
-            if (who < blocks && sh_fail == 0)
-            {
-                word* line = a.ctl->dec[who];
-                X::put(line, kDecWords / 2, 0, sh_alpha, tag);
-                X::put(line, kDecWords / 2, 1, sh_beta, tag);
-                store_word(line + 2, static_cast<unsigned>(sh_code), tag);
-            }
-        }
-        else
-        {
-            if (wave == 0)
-            {
-                // alpha, beta, code by lanes 0, 1, 2 (the other lanes repeat 2)
-                const word* line = a.ctl->dec[bid] + (lane < 2 ? lane : 2);
-                word hw[X::kWords];
-                const bool fine = wait_for(a.ctl, [&] {
-                    hw[0] = load_word(line);
-                    bool ok = word_ready(hw[0], tag);
-                    if constexpr (X::kWords == 2)
-                    {
-                        hw[1] = load_word(line + (lane < 2 ? kDecWords / 2 : 0));
-                        ok = ok && word_ready(hw[1], tag);
-                    }
-                    return ok;
-                });
-                if (!fine) sh_fail = 1;
-                if (lane == 0) sh_alpha = X::value(hw);
-                else if (lane == 1) sh_beta = X::value(hw);
-                else if (lane == 2) sh_code = static_cast<int>(hw[0]);
-            }
-            __syncthreads();
-        }
-        if (sh_fail != 0) return;
-        code = sh_code;
+        if (!persist_decide<S, NV>(sh, at, t, tag, red)) return;
+        code = sh.code;
         if (code != kRunning) break;
-        const S al = sh_alpha, be = sh_beta;
+        const S al = sh.alpha, be = sh.beta;
 
         // ---- step, then w = A u of the new u ----
         const bool refresh = a.refresh > 0 && (t + 1) % a.refresh == 0;
@@ -574,23 +331,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
             part[NV - 2] = __builtin_fma(static_cast<double>(w[k]), uv, part[NV - 2]);
             part[NV - 1] = __builtin_fma(uv, static_cast<double>(s[k]), part[NV - 1]);
         }
-        const double sum = wave_sum4(part[0], part[1], part[2], part[NV - 1]);
-        if (lane % 16 == 0) lds_p[lane / 16][wave] = sum;
-        __syncthreads();
-        if (sh_fail != 0) return;
-        if (tid < NV * kPersistGroups)
-        {
-            const int v = tid / kPersistGroups, q = tid % kPersistGroups;
-            const int lb = g * kPersistGroups + q;
-            if (lb < a.count)
-            {
-                double group = 0.0;
-#pragma unroll
-                for (int z = 0; z < kWavesPerBlock; ++z) group += lds_p[v][q * kWavesPerBlock + z];
-                const int vb = physical_block(lb, a.count);
-                Exchange<double>::put(&a.ctl->part[t & 1][v][0][vb], kSolverGrid, 0, group, tag);
-            }
-        }
+        if (!persist_partials<S, NV>(sh, at, t, tag, part)) return;
     }
 
     // ---- the end: x, and for a hand-over everything the next form reads ----
@@ -609,54 +350,8 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
         a.w[i] = w[k];
         if (!UNIT && a.inv != nullptr) a.u[i] = u_of(k);
     }
-    if (over && tid < kPersistGroups && g * kPersistGroups + tid < a.count)
-    {
-        // t0 and the hand-over iteration are even: the last partials are of an
-        // odd iteration, region 1
-        const int vb = physical_block(g * kPersistGroups + tid, a.count);
-        double vals[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-        {
-            word hw[2] = {load_word(&a.ctl->part[1][v][0][vb]), load_word(&a.ctl->part[1][v][1][vb])};
-            vals[v] = Exchange<double>::value(hw);
-        }
-        a.region[vb] = vals[0];
-        a.region[kMaxPartials + vb] = vals[UNIT ? 0 : 1];
-        a.region[2 * kMaxPartials + vb] = vals[NV - 2];
-        a.region[3 * kMaxPartials + vb] = vals[NV - 1];
-    }
-    if (bid == 0 && tid == 0) hs.record(a.st, code);
-    __syncthreads();
-    if (tid == 0) __hip_atomic_fetch_add(&a.ctl->finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__global__ void k_persist_reset(PersistControl* ctl, SolverState* st)
-{
-    ctl->abort = 0u;
-    ctl->finished = 0u;
-    st->counters[kCounterOutcome] = 0u;
-}
-
-__global__ void k_persist_clear(word* p, int64_t n)
-{
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-        p[i] = 0ull;
-}
-
-// Copies the new x when every workgroup of the solve reached its end and this
-// was the last launch of it, and tells the host.
-template <typename S>
-__global__ __launch_bounds__(kBlock) void k_persist_commit(int64_t rows, const S* __restrict__ from, S* __restrict__ x,
-                                                           const PersistControl* ctl, unsigned blocks, SolverState* st)
-{
-    if (ctl->finished != blocks) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->counters[kCounterOutcome] = 1u;
-    if (st->done == kRunning && st->counters[kCounterRestart] == 0u) return;  // the next launch continues from `from`
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < rows;
-         i += static_cast<int64_t>(gridDim.x) * kBlock)
-        x[i] = from[i];
+    if (over) persist_leave_partials<NV>(at);
+    persist_end(sh, at, a.st, code);
 }
 
 struct PersistShape
@@ -758,20 +453,6 @@ int persist_run_t(pm_workspace* ws, const PersistProblem& p, int64_t max_iterati
     if (!persist_shape(p, &shape)) return PM_OK;
     const void* kernel = shape.nd == 5 ? persist_kernel<S, 5>(shape) : persist_kernel<S, 7>(shape);
     if (kernel == nullptr) return PM_OK;
-    PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(shape.lds)));
-    const size_t words = static_cast<size_t>(p.rows) * Exchange<S>::kWords;
-    const size_t control = (sizeof(PersistControl) + 255) & ~size_t(255);
-    const size_t need = control + 2 * words * sizeof(word);
-    const bool grown = need > ws->persist.bytes;
-    PM_TRY(ws->persist.reserve(need));
-    if (grown || ws->persist_tag > 0xf0000000u)
-    {
-        // no word may carry a tag that is still to come
-        hipLaunchKernelGGL(k_persist_clear, dim3(1024), dim3(kBlock), 0, stream, ws->persist.as<word>(),
-                           static_cast<int64_t>(ws->persist.bytes / sizeof(word)));
-        PM_HIP(hipGetLastError());
-        ws->persist_tag = 0;
-    }
     PersistArgs<S> a{};
     a.rows = static_cast<int>(p.rows);
     a.dia = p.dia->args;
@@ -788,9 +469,6 @@ int persist_run_t(pm_workspace* ws, const PersistProblem& p, int64_t max_iterati
     a.rhs = static_cast<const S*>(p.rhs);
     a.st = p.st;
     a.region = p.region;
-    a.ctl = ws->persist.as<PersistControl>();
-    a.xu = reinterpret_cast<word*>(ws->persist.as<char>() + control);
-    a.xx = a.xu + words;
     a.count = p.count;
     a.per = shape.per;
     a.halo = shape.halo;
@@ -802,67 +480,15 @@ int persist_run_t(pm_workspace* ws, const PersistProblem& p, int64_t max_iterati
     a.refresh = p.refresh;
     a.chunk = p.chunk;
     a.grow = p.grow ? 1 : 0;
-    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(p.rows, kBlock), 2048));
-    for (int64_t t = 0;; )
-    {
-        // an even number of iterations, the last one's decision included
-        const int64_t left = max_iterations + 2 - t;
-        const int64_t count = std::min<int64_t>(kSegment, left + (left & 1));
-        a.t0 = static_cast<int>(t);
-        a.t_end = static_cast<int>(t + count);
-        if (t > 0) a.x_in = a.x_out;
-        a.tag = ws->persist_tag;
-        ws->persist_tag += static_cast<uint32_t>(count) + 2u;
-        hipLaunchKernelGGL(k_persist_reset, dim3(1), dim3(1), 0, stream, a.ctl, p.st);
-        PM_HIP(hipGetLastError());
-        void* args[] = {&a};
-        const hipError_t err = hipLaunchCooperativeKernel(kernel, dim3(shape.blocks), dim3(kPersistThreads), args,
-                                                          static_cast<unsigned>(shape.lds), stream);
-        if (err == hipErrorCooperativeLaunchTooLarge || err == hipErrorNotSupported)
-        {
-            (void)hipGetLastError();
-            return PM_OK;
-        }
-        PM_HIP(err);
-        hipLaunchKernelGGL(k_persist_commit<S>, dim3(grid), dim3(kBlock), 0, stream, p.rows,
-                           static_cast<const S*>(p.x_out), static_cast<S*>(p.x), a.ctl,
-                           static_cast<unsigned>(shape.blocks), p.st);
-        PM_HIP(hipGetLastError());
-        PM_HIP(hipMemcpyAsync(ws->host_state, p.st, sizeof(SolverState), hipMemcpyDeviceToHost, stream));
-        PM_HIP(hipStreamSynchronize(stream));
-        *state = ws->host_state[0];
-        if (state->counters[kCounterOutcome] != 1u) return PM_OK;
-        if (state->done != kRunning)
-        {
-            *outcome = kPersistStopped;
-            return PM_OK;
-        }
-        t = static_cast<int64_t>(state->counters[kCounterNext]);
-        if (state->counters[kCounterRestart] != 0u)
-        {
-            *outcome = kPersistHandOver;
-            *next = t;
-            return PM_OK;
-        }
-    }
+    return persist_loop<S>(ws, p, a, kernel, shape.blocks, shape.lds, max_iterations, stream, outcome, next, state);
 }
 
 } // namespace
 
 bool persist_wanted(const PersistProblem& p, int device)
 {
-    const char* env = std::getenv("PLAMATRIX_AMD_PERSISTENT");
-    if (env != nullptr && env[0] == '0') return false;
     PersistShape s{};
-    if (!persist_shape(p, &s)) return false;
-    int coop = 0, cus = 0;
-    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
-    {
-        (void)hipGetLastError();
-        return false;
-    }
-    return coop != 0 && s.blocks <= cus;
+    return persist_enabled() && persist_shape(p, &s) && persist_resident(s.blocks, device);
 }
 
 int persist_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream, int* outcome,

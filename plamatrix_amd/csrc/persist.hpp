@@ -1,6 +1,7 @@
 // Persistent single-reduction CG / Jacobi-PCG: one launch runs a whole solve,
-// cooperative on the diagonal layout (persist.hip), in one workgroup on small
-// CSR matrices (persist_small.hip).
+// cooperative on the diagonal layout (persist.hip) and on CSR matrices of short
+// rows (persist_csr.hip), in one workgroup on small CSR matrices
+// (persist_small.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -57,6 +58,15 @@ int persist_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iteration
 bool persist_small_wanted(const PersistProblem& p);
 int persist_small_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream,
                       int* outcome, int64_t* next, SolverState* state);
+
+// The same for CSR matrices of short, mostly local rows: a candidate by its
+// sizes, the device's look at its rows (stream-ordered) and the answer (waits for
+// the look only).
+bool persist_csr_candidate(const PersistProblem& p, int device);
+int persist_csr_look(pm_workspace* ws, const PersistProblem& p, hipStream_t stream);
+int persist_csr_fits(pm_workspace* ws, bool* fits);
+int persist_csr_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream,
+                    int* outcome, int64_t* next, SolverState* state);
 
 // The chunk schedule of an adaptive solve: chunk c covers iterations
 // [end(c - 1), end(c)).  Both forms of a solve must leave the single-reduction

@@ -1,0 +1,133 @@
+// Host side of the persistent solves: exchange storage, tags, the cooperative
+// launches of a solve and the commit of its x.
+#pragma once
+
+#include <algorithm>
+#include <cstdlib>
+
+#include "persist_device.hpp"
+
+namespace pm
+{
+
+static __global__ void k_persist_reset(PersistControl* ctl, SolverState* st)
+{
+    ctl->abort = 0u;
+    ctl->finished = 0u;
+    st->counters[kCounterOutcome] = 0u;
+}
+
+static __global__ void k_persist_clear(word* p, int64_t n)
+{
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+        p[i] = 0ull;
+}
+
+// Copies the new x when every workgroup of the solve reached its end and this
+// was the last launch of it, and tells the host.
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_persist_commit(int64_t rows, const S* __restrict__ from, S* __restrict__ x,
+                                                           const PersistControl* ctl, unsigned blocks, SolverState* st)
+{
+    if (ctl->finished != blocks) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->counters[kCounterOutcome] = 1u;
+    if (st->done == kRunning && st->counters[kCounterRestart] == 0u) return;  // the next launch continues from `from`
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < rows;
+         i += static_cast<int64_t>(gridDim.x) * kBlock)
+        x[i] = from[i];
+}
+
+// PLAMATRIX_AMD_PERSISTENT=0 keeps every solve on the per-kernel iteration.
+inline bool persist_enabled()
+{
+    const char* env = std::getenv("PLAMATRIX_AMD_PERSISTENT");
+    return env == nullptr || env[0] != '0';
+}
+
+// Whether `blocks` workgroups of a CU each can run together.
+inline bool persist_resident(int blocks, int device)
+{
+    int coop = 0, cus = 0;
+    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    return coop != 0 && blocks <= cus;
+}
+
+// Every workgroup decides for itself, or eight decide and answer the rest.
+inline int persist_leaders(int blocks) { return blocks <= 64 ? blocks : kXcds; }
+
+// Runs the launches of a solve; `a` is complete but for the exchange storage,
+// x and the iteration range.
+template <typename S, typename Args>
+int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void* kernel, int blocks, size_t lds,
+                 int64_t max_iterations, hipStream_t stream, int* outcome, int64_t* next, SolverState* state)
+{
+    *outcome = kPersistAbandoned;
+    PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    const size_t words = static_cast<size_t>(p.rows) * Exchange<S>::kWords;
+    const size_t control = (sizeof(PersistControl) + 255) & ~size_t(255);
+    const size_t need = control + 2 * words * sizeof(word);
+    const bool grown = need > ws->persist.bytes;
+    PM_TRY(ws->persist.reserve(need));
+    if (grown || ws->persist_tag > 0xf0000000u)
+    {
+        // no word may carry a tag that is still to come
+        hipLaunchKernelGGL(k_persist_clear, dim3(1024), dim3(kBlock), 0, stream, ws->persist.as<word>(),
+                           static_cast<int64_t>(ws->persist.bytes / sizeof(word)));
+        PM_HIP(hipGetLastError());
+        ws->persist_tag = 0;
+    }
+    a.ctl = ws->persist.as<PersistControl>();
+    a.xu = reinterpret_cast<word*>(ws->persist.as<char>() + control);
+    a.xx = a.xu + words;
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(p.rows, kBlock), 2048));
+    for (int64_t t = 0;; )
+    {
+        // an even number of iterations, the last one's decision included
+        const int64_t left = max_iterations + 2 - t;
+        const int64_t count = std::min<int64_t>(kSegment, left + (left & 1));
+        a.t0 = static_cast<int>(t);
+        a.t_end = static_cast<int>(t + count);
+        if (t > 0) a.x_in = a.x_out;
+        a.tag = ws->persist_tag;
+        ws->persist_tag += static_cast<uint32_t>(count) + 2u;
+        hipLaunchKernelGGL(k_persist_reset, dim3(1), dim3(1), 0, stream, a.ctl, p.st);
+        PM_HIP(hipGetLastError());
+        void* args[] = {&a};
+        const hipError_t err = hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads), args,
+                                                          static_cast<unsigned>(lds), stream);
+        if (err == hipErrorCooperativeLaunchTooLarge || err == hipErrorNotSupported)
+        {
+            (void)hipGetLastError();
+            return PM_OK;
+        }
+        PM_HIP(err);
+        hipLaunchKernelGGL(k_persist_commit<S>, dim3(grid), dim3(kBlock), 0, stream, p.rows,
+                           static_cast<const S*>(p.x_out), static_cast<S*>(p.x), a.ctl,
+                           static_cast<unsigned>(blocks), p.st);
+        PM_HIP(hipGetLastError());
+        PM_HIP(hipMemcpyAsync(ws->host_state, p.st, sizeof(SolverState), hipMemcpyDeviceToHost, stream));
+        PM_HIP(hipStreamSynchronize(stream));
+        *state = ws->host_state[0];
+        if (state->counters[kCounterOutcome] != 1u) return PM_OK;
+        if (state->done != kRunning)
+        {
+            *outcome = kPersistStopped;
+            return PM_OK;
+        }
+        t = static_cast<int64_t>(state->counters[kCounterNext]);
+        if (state->counters[kCounterRestart] != 0u)
+        {
+            *outcome = kPersistHandOver;
+            *next = t;
+            return PM_OK;
+        }
+    }
+}
+
+} // namespace pm

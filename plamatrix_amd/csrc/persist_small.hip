@@ -16,10 +16,7 @@
 // chunk is left to it.
 #include "persist.hpp"
 
-#include <algorithm>
-#include <cstdlib>
-
-#include "persist_history.hpp"
+#include "persist_launch.hpp"
 #include "spmv_kernels.hpp"
 #include "tuning.hpp"
 
@@ -315,11 +312,9 @@ int small_run(pm_workspace* ws, const PersistProblem& p, const I* ro, const I* c
 
 bool persist_small_wanted(const PersistProblem& p)
 {
-    const char* env = std::getenv("PLAMATRIX_AMD_PERSISTENT");
-    if (env != nullptr && env[0] == '0') return false;
     // one row per lane and slot: the per-kernel workgroups hold at most four
     // chunks of 64 rows
-    return p.rows > 0 && p.rows <= kSmallRows && p.a->nnz <= kSmallEntries &&
+    return persist_enabled() && p.rows > 0 && p.rows <= kSmallRows && p.a->nnz <= kSmallEntries &&
            p.count <= 4 * kSmallGroups && ceil_div(chunk_count(p.rows), static_cast<int64_t>(p.count)) <= kWavesPerBlock;
 }
 

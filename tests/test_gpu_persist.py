@@ -104,14 +104,21 @@ def test_stops_at_the_start(dev, monkeypatch):
     assert bool((x == 2.0).all())
 
 
-def ragged(n, seed, long_row=0, dtype=np.float64):
-    """SPD matrix with 1 to 14 entries a row and, if asked, one long row."""
+def ragged(n, seed, long_row=0, dtype=np.float64, band=0):
+    """SPD matrix with 1 to 14 entries a row and, if asked, one long row; with
+    `band` 1 to 9 entries a row, columns within `band` of the row."""
     import scipy.sparse as sp
 
     rng = np.random.default_rng(seed)
-    k = rng.integers(0, 7, n)
-    i = np.repeat(np.arange(n), k)
-    j = rng.integers(0, n, len(i))
+    if band:
+        off = np.concatenate([[0], np.sort(rng.integers(1, band, 4))])
+        i = np.concatenate([np.nonzero(rng.random(n) < 0.7)[0] for _ in off])
+        i = i[(i + off[-1]) < n]
+        j = i + off[rng.integers(1, 5, len(i))]
+    else:
+        k = rng.integers(0, 7, n)
+        i = np.repeat(np.arange(n), k)
+        j = rng.integers(0, n, len(i))
     if long_row:
         i = np.concatenate([i, np.full(long_row, n // 2)])
         j = np.concatenate([j, rng.permutation(n)[:long_row]])
@@ -176,3 +183,66 @@ def test_one_workgroup_errors(dev, monkeypatch):
         assert out["0"] == out["1"]
         if row is not None:
             assert "diagonal" in out["1"][1] and f"row {row}" in out["1"][1]
+
+
+WIDE = [
+    ("stencil", (67, 62), np.float64, 0),      # 4,154 rows, 64-row chunks not a multiple of four
+    ("stencil", (23, 21, 19), np.float32, 50),  # 9,177 rows
+    ("stencil", (39, 40, 41), np.float64, 0),   # 63,960 rows: the last size below the diagonal layout
+    ("banded", 5003, np.float64, 20),
+    ("banded", 70001, np.float32, 0),           # more than 64 workgroups, no few diagonals
+    ("banded", 262144, np.float64, 6),          # the largest
+    ("ragged", 30011, np.float32, 0),           # most entries in other pieces: the per-kernel solve
+    ("long", 6007, np.float64, 6),              # a row past the kept entries: likewise
+]
+
+
+@pytest.mark.parametrize("kind,size,dtype,refresh", WIDE)
+def test_wide_csr_solve_is_bitwise(dev, monkeypatch, kind, size, dtype, refresh):
+    if kind == "stencil":
+        h = generators.laplacian2d_csr(*size, dtype=dtype) if len(size) == 2 else \
+            generators.diffusion3d_box_csr(*size, seed=3, dtype=dtype)
+    else:
+        h = ragged(size, 11, 700 if kind == "long" else 0, dtype, 300 if kind == "banded" else 0)
+    rel = 1e-10 if dtype == np.float64 else 1e-5
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=29).astype(dtype)).to(dev)
+    for solver, compact, most in ((capi.pcg, True, 600), (capi.cg, False, 600), (capi.pcg, False, 1), (capi.cg, True, 0)):
+        a = capi.to_device_csr(h, compact=compact)
+        out, storage = {}, {}
+        for flag in ("0", "1"):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+            ws = capi.Workspace()
+            for _ in range(2):  # the second solve meets the first one's exchange words
+                x = torch.full_like(b, 0.5)
+                rep = solver(a, b, x, ws, capi.policy(refresh_interval=refresh), relative_tolerance=rel,
+                             max_iterations=most)
+                torch.cuda.synchronize()
+                got = (rep.converged, rep.iterations, rep.initial_residual, rep.final_residual, x.cpu().numpy().tobytes())
+                assert out.setdefault(flag, got) == got
+            storage[flag] = ws.capacity_bytes
+        # the exchange words tell which kernel ran
+        assert (storage["1"] > storage["0"]) == (kind in ("stencil", "banded"))
+        assert out["0"] == out["1"], (solver.__name__, compact, most)
+
+
+def test_wide_csr_restart_hands_over(dev, monkeypatch):
+    # an indefinite matrix: restart, hand-over at the chunk schedule's
+    # iteration, the three-kernel form's breakdown
+    h = generators.laplacian2d_csr(90, 80)
+    rows = np.repeat(np.arange(h.rows), np.diff(h.row_offsets))
+    for shift in (3.9, 3.0, 0.05):
+        v = h.values - shift * (rows == h.col_indices)
+        a = capi.to_device_csr(generators.CSRHost(h.rows, h.cols, h.row_offsets, h.col_indices, v), compact=True)
+        b = torch.from_numpy(generators.rhs_normal(h.rows, seed=31).astype(np.float64)).to(dev)
+        out = {}
+        for flag in ("0", "1"):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+            x = torch.zeros_like(b)
+            try:
+                rep = capi.cg(a, b, x, capi.Workspace(), relative_tolerance=1e-9, max_iterations=400)
+                out[flag] = ("ok", rep.iterations, rep.final_residual)
+            except capi.PlamatrixError as e:
+                out[flag] = (e.kind, str(e))
+            torch.cuda.synchronize()
+            out[flag] += (x.cpu().numpy().tobytes(),)
+        assert out["0"] == out["1"], shift
