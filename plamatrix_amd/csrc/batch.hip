@@ -33,6 +33,7 @@
 #include <string>
 #include <vector>
 
+#include "persist_batch.hpp"
 #include "plan_cache.hpp"
 #include "solver_internal.hpp"
 #include "spmv_kernels.hpp"
@@ -43,20 +44,6 @@ namespace pm
 
 constexpr int kBatchWaves = kWavesPerBlock;  // 4 wavefronts per 256-thread workgroup
 constexpr int kBatchGrid = 2048;
-
-struct BatchState
-{
-    double rho;
-    double alpha;
-    double beta;
-    double rr;
-    double rr0;
-    double tol;
-    int32_t iteration;
-    int32_t done;
-    unsigned long long bad_row;
-    double den;  // single-reduction form: p.Ap of the last direction
-};
 
 // Chunks of the systems still running, as a device list with its length in
 // device memory (so replayed graphs follow every rebuild): a superset of the
@@ -1033,7 +1020,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_cg_reduce(int64_t systems, con
         const double rr = sum[0], gamma = sum[1], delta = sum[2], us = sum[3];
         BatchState w = st[s];
         int code = kRunning;
-        double beta = 0.0, den = delta, alpha = 0.0;
+        const double beta = 0.0, den = delta;
+        double alpha = 0.0;
         if (INIT)
         {
             w.rr = rr;
@@ -1047,34 +1035,16 @@ __global__ __launch_bounds__(kBlock) void k_batch_cg_reduce(int64_t systems, con
         }
         else
         {
-            w.iteration += 1;
-            w.rr = rr;
-            if (!isfinite(rr) || rr < 0.0) code = kNonFinite;
-            else if (sqrt(rr) <= w.tol) code = kConverged;
-            else if (w.iteration >= max_iterations) code = kIterationLimit;
-            else
-            {
-                const double rho_prev = w.rho;
-                if (rho_prev == 0.0 && gamma == 0.0) beta = 0.0;
-                else if (isfinite(rho_prev) && isfinite(gamma) && rho_prev > 0.0 && gamma > 0.0)
-                {
-                    beta = gamma / rho_prev;
-                    if (!isfinite(beta) || !isfinite(static_cast<S>(beta))) code = kBreakdown;
-                }
-                else code = kBreakdown;
-                if (code == kRunning && beta != 0.0) den = delta + beta * (2.0 * us + beta * w.den);
-                if (code == kRunning && !(den > 0.0 && isfinite(den)))
-                {
-                    beta = 0.0;
-                    den = delta;
-                }
-            }
+            code = w.advance<S>(rr, gamma, delta, us, max_iterations);
         }
-        if (code == kRunning && !step_length<S>(gamma, den, alpha)) code = kBreakdown;
-        w.beta = beta;
-        w.alpha = alpha;
-        w.rho = gamma;
-        w.den = den;
+        if (INIT)
+        {
+            if (code == kRunning && !step_length<S>(gamma, den, alpha)) code = kBreakdown;
+            w.beta = beta;
+            w.alpha = alpha;
+            w.rho = gamma;
+            w.den = den;
+        }
         if (code != kRunning)
         {
             w.done = code;
@@ -1129,6 +1099,9 @@ struct BatchProblem
     int bmax;
     void* binv;
     double* block_rows;               // the gathered diagonal-block rows (FP64, bmax per row)
+    std::vector<int64_t> begin, end;  // host: the systems' rows
+    std::vector<uint8_t> blocked;     // host: block-Jacobi systems
+    std::vector<BatchLook> look;      // what the device saw of their rows (empty: not looked yet)
     // the Jacobi and block inverses of this matrix are in place from an
     // earlier solve (the refinement loop's later inner solves)
     bool inverses_ready;
@@ -1603,6 +1576,40 @@ int batch_solve(BatchProblem& b, const BatchPolicy& policy, pm_batch_report* rep
     PM_HIP(hipMemcpyAsync(hs, b.done_count, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
     PM_HIP(hipStreamSynchronize(stream));
     bool finished = static_cast<int64_t>(hs[0]) >= b.systems;
+    if (!finished && needed > 0 && b.single_reduction && !b.g && !b.split)
+    {
+        // systems of short, banded rows run to their end on their own CUs; the
+        // loop below takes the rest
+        BatchTeams teams{};
+        teams.a = b.a;
+        teams.systems = b.systems;
+        teams.begin = b.begin.data();
+        teams.end = b.end.data();
+        teams.skip = b.blocked.data();
+        teams.chunk_sys = b.chunk_sys;
+        teams.chunks = b.chunks;
+        teams.sys_end = b.sys_end;
+        teams.sys_chunk0 = b.sys_chunk0;
+        teams.rhs = b.rhs;
+        teams.x = b.x;
+        teams.r = b.r;
+        teams.u = b.z;
+        teams.w = b.q;
+        teams.p = b.p0;
+        teams.s = b.p1;
+        teams.inv = b.jacobi ? b.inv : nullptr;
+        teams.x_out = b.t;
+        teams.st = b.st;
+        teams.done_count = b.done_count;
+        teams.max_iterations = b.max_iterations;
+        teams.refresh = policy.refresh;
+        if (b.look.empty()) PM_TRY(batch_teams_look(ws, teams, b.look, stream));
+        PM_TRY(batch_teams_run(ws, teams, b.look, stream));
+        PM_HIP(hipMemcpyAsync(hs, b.done_count, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
+        PM_HIP(hipStreamSynchronize(stream));
+        finished = static_cast<int64_t>(hs[0]) >= b.systems;
+        if (!finished) PM_TRY(batch_plan<S>(ws, b, 2, 0, 0, 0)->run(stream, false));
+    }
     unsigned long long listed_at = hs[0];  // stopped systems when the list was last built
     if (!finished && needed > 0)
     {
@@ -1704,6 +1711,9 @@ int batch_setup(const pm_csr* a, int64_t systems, const int64_t* row_begin, cons
     b.jacobi = options->use_jacobi != 0;
     b.systems = systems;
     b.chunks = chunks;
+    b.begin.assign(row_begin, row_begin + systems);
+    b.end.assign(row_end, row_end + systems);
+    b.blocked.assign(static_cast<size_t>(systems), 0);
     b.max_iterations = options->max_iterations;
     b.rel_tol = options->relative_tolerance;
     b.abs_tol = options->absolute_tolerance;
@@ -1779,6 +1789,7 @@ int batch_attach_blocks(BatchProblem& b, const int64_t* row_begin, const int64_t
             return fail(PM_INVALID_ARGUMENT, "batched block pcg: system %lld has %lld rows, not a multiple of %d",
                         static_cast<long long>(s), static_cast<long long>(row_end[s] - row_begin[s]), bs);
         bmax = std::max(bmax, bs);
+        b.blocked[static_cast<size_t>(s)] = bs > 1 ? 1 : 0;
     }
     b.jacobi = true;
     if (bmax == 1) return PM_OK;

@@ -2283,10 +2283,10 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     pp.grow = policy.grow;
     const bool one_launch = pb.single_reduction && !pb.cg_factored;
     const bool csr = one_launch && !pb.dia.active;
-    auto run = one_launch && pb.cg_fused && persist_wanted(pp, ws->device) ? persist_run
+    auto run = one_launch && pb.cg_fused && persist_wanted(pp, ws) ? persist_run
                : csr && persist_small_wanted(pp)                           ? persist_small_run
                                                                            : nullptr;
-    const bool look = csr && run == nullptr && persist_csr_candidate(pp, ws->device);
+    const bool look = csr && run == nullptr && persist_csr_candidate(pp, ws);
     if (look) PM_TRY(persist_csr_look(ws, pp, stream));
     PM_TRY(initialise());
     if (look)

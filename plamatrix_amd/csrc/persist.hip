@@ -485,10 +485,10 @@ int persist_run_t(pm_workspace* ws, const PersistProblem& p, int64_t max_iterati
 
 } // namespace
 
-bool persist_wanted(const PersistProblem& p, int device)
+bool persist_wanted(const PersistProblem& p, const pm_workspace* ws)
 {
     PersistShape s{};
-    return persist_enabled() && persist_shape(p, &s) && persist_resident(s.blocks, device);
+    return persist_enabled() && persist_shape(p, &s) && persist_resident(ws, s.blocks);
 }
 
 int persist_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream, int* outcome,

@@ -48,7 +48,7 @@ enum PersistOutcome : int
 };
 
 // Whether the persistent iteration on the diagonal layout takes this solve.
-bool persist_wanted(const PersistProblem& p, int device);
+bool persist_wanted(const PersistProblem& p, const pm_workspace* ws);
 
 // Runs the solve and waits for it.  *state receives the final state record.
 int persist_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream, int* outcome,
@@ -62,7 +62,7 @@ int persist_small_run(pm_workspace* ws, const PersistProblem& p, int64_t max_ite
 // The same for CSR matrices of short, mostly local rows: a candidate by its
 // sizes, the device's look at its rows (stream-ordered) and the answer (waits for
 // the look only).
-bool persist_csr_candidate(const PersistProblem& p, int device);
+bool persist_csr_candidate(const PersistProblem& p, const pm_workspace* ws);
 int persist_csr_look(pm_workspace* ws, const PersistProblem& p, hipStream_t stream);
 int persist_csr_fits(pm_workspace* ws, bool* fits);
 int persist_csr_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream,

@@ -1,0 +1,561 @@
+// Batched CG / Jacobi-PCG of systems with short, banded rows, each solved by a
+// team of workgroups that keeps it on the CUs from the first iteration to the
+// last.
+//
+// The per-kernel batch runs three kernels per iteration over all systems until
+// the slowest has converged: on 48 systems of 1,000 to 60,000 rows 730 iterations
+// of 20 us, launch latency and one wavefront per system deciding.  Here a system
+// of n rows gets ceil(n / piece) workgroups of 1,024 lanes with R rows each:
+// vectors and row entries in registers, u of the piece and of the `halo` rows on
+// either side in LDS.  A team exchanges u's rows near its pieces' ends and four
+// sums per iteration as tagged 64-bit words (persist.hip), every workgroup of it
+// decides alike, and teams never wait for each other, so a stopped system frees
+// its CUs' bandwidth at once.  Teams that do not fit the chip together run in
+// successive launches, largest systems first, so that a launch's systems are of
+// like length.
+//
+// The iteration is that of the per-kernel batch (BatchState::advance); its dot
+// products are summed per workgroup and then per team instead of per 64-row
+// chunk.
+#include "persist_batch.hpp"
+
+#include <algorithm>
+#include <numeric>
+#include <type_traits>
+
+#include "persist_launch.hpp"
+#include "tuning.hpp"
+
+namespace pm
+{
+namespace
+{
+
+constexpr int kTeamEntries = 8;    // row entries in registers
+constexpr int kTeamSlots = 256;    // workgroups of a launch at most
+constexpr int kTeamLargest = kWave; // workgroups of a team: one lane each in the decision
+constexpr int32_t kTeamIterations = 1 << 16;  // a launch runs a system to its end
+
+// One workgroup's part of a launch.
+struct TeamTask
+{
+    int32_t system, slot0, team, piece;  // its team's first workgroup and size, its piece
+    int32_t rows, halo;                  // of the system
+    int64_t begin;                       // the system's first row
+};
+
+struct TeamControl
+{
+    unsigned abort;
+    unsigned pad[63];
+    unsigned finished[kTeamSlots];       // workgroups of a team (by first slot) that reached the end
+    BatchState out[kTeamSlots];          // ... and its final state
+    TeamTask tasks[kTeamSlots];
+    word part[2][kCgValues][2][kTeamSlots];
+};
+
+template <typename S, typename I>
+struct TeamArgs
+{
+    const I* ro;
+    const I* ci;
+    const S* values;
+    const S* rhs;
+    const S* x;
+    S* x_out;
+    const S *p, *r, *s, *w;
+    const S* inv;
+    const BatchState* st;
+    TeamControl* ctl;
+    PersistControl* give_up;  // its abort notice alone is used: TeamControl starts with it
+    word* xu;                 // [slot][row of the piece]
+    word* xx;
+    int plane;                // words of a half plane
+    unsigned tag;
+    int32_t max_iterations;
+    int refresh;
+};
+
+template <typename S, typename I, int R>
+__global__ __launch_bounds__(kPersistThreads) void k_batch_team(TeamArgs<S, I> a)
+{
+    using X = Exchange<S>;
+    constexpr int E = kTeamEntries;
+    constexpr int kPiece = R * kPersistThreads;
+    extern __shared__ char lds_raw[];
+    __shared__ double lds_p[kCgValues][kPersistWaves];
+    __shared__ BatchState state;
+    __shared__ S sh_alpha, sh_beta;
+    __shared__ int sh_code, sh_fail;
+
+    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    const TeamTask job = a.ctl->tasks[blockIdx.x];
+    const int H = job.team > 1 ? job.halo : 0;
+    const int first = job.piece * kPiece;  // the piece's first row of the system
+    const int size = job.rows - first < kPiece ? job.rows - first : kPiece;
+    const int words0 = job.slot0 * kPiece;  // the system's rows in the exchange
+    S* us = reinterpret_cast<S*>(lds_raw);  // u of rows [first - H, first + kPiece + H)
+
+    S p[R], s[R], x[R], r[R], w[R], inv[R], val[R][E];
+    unsigned col[R][E / 2];  // two 16-bit places in us each
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+    {
+        const int l = k * kPersistThreads + tid;
+        const bool ok = l < size;
+        const int64_t i = job.begin + first + (ok ? l : 0);
+        p[k] = ok ? a.p[i] : S(0);
+        s[k] = ok ? a.s[i] : S(0);
+        x[k] = ok ? a.x[i] : S(0);
+        r[k] = ok ? a.r[i] : S(0);
+        w[k] = ok ? a.w[i] : S(0);
+        inv[k] = !ok ? S(0) : a.inv != nullptr ? a.inv[i] : S(1);
+        const int64_t b = static_cast<int64_t>(a.ro[i]);
+        const int n = ok ? static_cast<int>(static_cast<int64_t>(a.ro[i + 1]) - b) : 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+        {
+            // an absent entry is 0 times the row's own u
+            val[k][e] = e < n ? a.values[b + e] : S(0);
+            const int c = e < n ? static_cast<int>(static_cast<int64_t>(a.ci[b + e]) - job.begin) - first : (ok ? l : 0);
+            const unsigned at = static_cast<unsigned>(c + H);
+            if (e % 2 == 0) col[k][e / 2] = at;
+            else col[k][e / 2] |= at << 16;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // halo rows past the system stay 0
+    for (int q = tid; q < kPiece + 2 * H; q += kPersistThreads) us[q] = S(0);
+    if (tid == 0)
+    {
+        state = a.st[job.system];
+        sh_alpha = static_cast<S>(state.alpha);
+        sh_beta = static_cast<S>(state.beta);
+        sh_code = state.done;
+        sh_fail = 0;
+    }
+    __syncthreads();
+    auto u_of = [&](int k) { return inv[k] * r[k]; };
+
+    auto publish = [&](word* buf, unsigned tag, auto get) {
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+        {
+            const int l = k * kPersistThreads + tid;
+            if (l >= size) continue;
+            const S v = get(k);
+            us[H + l] = v;
+            if (l < H || l >= size - H) X::put(buf, a.plane, words0 + first + l, v, tag);
+        }
+    };
+    // acc[k] = row k of A v for the vector published last, entries left to right
+    auto product = [&](const word* buf, unsigned tag, auto* acc) {
+        using Acc = std::remove_reference_t<decltype(acc[0])>;
+        bool fine = true;
+        for (int h0 = 0; h0 < 2 * H; h0 += kPersistThreads)
+        {
+            const int h = h0 + tid;
+            const int q = h < H ? h - H : size + (h - H);
+            const int i = first + q;
+            if (h >= 2 * H || i < 0 || i >= job.rows) continue;
+            word hw[X::kWords];
+            fine = wait_for(a.give_up, [&] {
+                       X::issue(buf, a.plane, words0 + i, hw);
+                       return ready<S>(hw, tag);
+                   }) && fine;
+            us[H + q] = X::value(hw);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+        {
+            Acc sum = Acc(0);
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+            {
+                const unsigned at = e % 2 == 0 ? col[k][e / 2] & 0xffffu : col[k][e / 2] >> 16;
+                sum = fma_s<Acc>(static_cast<Acc>(val[k][e]), static_cast<Acc>(us[at]), sum);
+            }
+            acc[k] = k * kPersistThreads + tid < size ? sum : Acc(0);
+            if (R > 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        if (!fine) sh_fail = 1;
+    };
+
+    unsigned tag = a.tag;
+    for (int t = 0; sh_code == kRunning; ++t)
+    {
+        ++tag;
+        const S al = sh_alpha, be = sh_beta;
+        const bool refresh = a.refresh > 0 && (t + 1) % a.refresh == 0;
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+        {
+            p[k] = fma_s(be, p[k], u_of(k));
+            s[k] = fma_s(be, s[k], w[k]);
+            x[k] = fma_s(al, p[k], x[k]);
+            if (!refresh) r[k] = fma_s(-al, s[k], r[k]);
+        }
+        if (refresh)
+        {
+            // r = b - A x with FP64 accumulation
+            publish(a.xx, tag, [&](int k) { return x[k]; });
+            double ax[R];
+            product(a.xx, tag, ax);
+#pragma unroll
+            for (int k = 0; k < R; ++k)
+            {
+                const int l = k * kPersistThreads + tid;
+                if (l < size) r[k] = static_cast<S>(static_cast<double>(a.rhs[job.begin + first + l]) - ax[k]);
+            }
+            __syncthreads();
+        }
+        publish(a.xu, tag, u_of);
+        product(a.xu, tag, w);
+
+        double part[kCgValues] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+        {
+            const double rv = static_cast<double>(r[k]), uv = static_cast<double>(u_of(k));
+            part[0] = __builtin_fma(rv, rv, part[0]);
+            part[1] = __builtin_fma(rv, uv, part[1]);
+            part[2] = __builtin_fma(static_cast<double>(w[k]), uv, part[2]);
+            part[3] = __builtin_fma(uv, static_cast<double>(s[k]), part[3]);
+        }
+        const double wsum = wave_sum4(part[0], part[1], part[2], part[3]);
+        if (lane % 16 == 0) lds_p[lane / 16][wave] = wsum;
+        __syncthreads();
+        if (sh_fail != 0) return;
+        if (wave == 0)
+        {
+            // row v of the wavefront sums value v over the wavefronts
+            double mine = lds_p[lane / 16][lane % 16];
+            mine = butterfly_add<8>(mine);
+            mine = butterfly_add<4>(mine);
+            mine = butterfly_add<2>(mine);
+            mine = butterfly_add<1>(mine);
+            double tot[kCgValues];
+            bool fine = true;
+            if (job.team > 1)
+            {
+                if (lane % 16 == 0)
+                    Exchange<double>::put(&a.ctl->part[t & 1][lane / 16][0][blockIdx.x], kTeamSlots, 0, mine, tag);
+                double v[kCgValues] = {0.0, 0.0, 0.0, 0.0};
+                if (lane < job.team)
+                {
+                    const word* from = &a.ctl->part[t & 1][0][0][job.slot0 + lane];
+                    word hw[kCgValues][2];
+                    fine = wait_for(a.give_up, [&] {
+                        bool ok = true;
+#pragma unroll
+                        for (int q = 0; q < kCgValues; ++q)
+                        {
+                            hw[q][0] = load_word(from + (2 * q) * kTeamSlots);
+                            hw[q][1] = load_word(from + (2 * q + 1) * kTeamSlots);
+                        }
+#pragma unroll
+                        for (int q = 0; q < kCgValues; ++q)
+                            ok = ok && word_ready(hw[q][0], tag) && word_ready(hw[q][1], tag);
+                        return ok;
+                    });
+#pragma unroll
+                    for (int q = 0; q < kCgValues; ++q) v[q] = Exchange<double>::value(hw[q]);
+                }
+                mine = wave_sum4(v[0], v[1], v[2], v[3]);
+            }
+#pragma unroll
+            for (int q = 0; q < kCgValues; ++q) tot[q] = __shfl(mine, q * 16, kWave);
+            if (!fine) sh_fail = 1;
+            if (lane == 0)
+            {
+                sh_code = state.template advance<S>(tot[0], tot[1], tot[2], tot[3], a.max_iterations);
+                sh_alpha = static_cast<S>(state.alpha);
+                sh_beta = static_cast<S>(state.beta);
+            }
+        }
+        __syncthreads();
+        if (sh_fail != 0) return;
+    }
+
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+    {
+        const int l = k * kPersistThreads + tid;
+        if (l < size) a.x_out[job.begin + first + l] = x[k];
+    }
+    if (tid == 0 && job.piece == 0)
+    {
+        BatchState end = state;
+        end.done = sh_code;
+        a.ctl->out[job.slot0] = end;
+    }
+    __syncthreads();
+    if (tid == 0)
+        __hip_atomic_fetch_add(&a.ctl->finished[job.slot0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The x of every team whose workgroups all reached the end, then (in a kernel of
+// its own) its state.
+template <typename S>
+__global__ __launch_bounds__(kBlock) void k_team_commit(const TeamControl* ctl, int piece_rows,
+                                                        const S* __restrict__ from, S* __restrict__ x)
+{
+    const TeamTask job = ctl->tasks[blockIdx.x];
+    if (ctl->finished[job.slot0] != static_cast<unsigned>(job.team)) return;
+    const int first = job.piece * piece_rows;
+    const int size = job.rows - first < piece_rows ? job.rows - first : piece_rows;
+    for (int l = threadIdx.x; l < size; l += kBlock) x[job.begin + first + l] = from[job.begin + first + l];
+}
+
+__global__ void k_team_states(const TeamControl* ctl, int slots, BatchState* st, unsigned long long* done_count)
+{
+    const int slot = static_cast<int>(threadIdx.x);
+    if (slot >= slots) return;
+    const TeamTask job = ctl->tasks[slot];
+    if (job.piece != 0 || ctl->finished[slot] != static_cast<unsigned>(job.team)) return;
+    if (st[job.system].done != kRunning) return;  // stopped before the launch, and counted then
+    st[job.system] = ctl->out[slot];
+    atomicAdd(done_count, 1ull);
+}
+
+__global__ void k_team_reset(TeamControl* ctl)
+{
+    if (threadIdx.x == 0) ctl->abort = 0u;
+    if (threadIdx.x < kTeamSlots) ctl->finished[threadIdx.x] = 0u;
+}
+
+// Longest row and band per system, a wavefront per 64-row chunk.
+template <typename I>
+__global__ __launch_bounds__(kBlock) void k_team_look(int64_t chunks, const int32_t* __restrict__ chunk_sys,
+                                                      const int64_t* __restrict__ sys_end,
+                                                      const int64_t* __restrict__ sys_chunk0,
+                                                      const I* __restrict__ ro, const I* __restrict__ ci,
+                                                      BatchLook* look)
+{
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave;
+    if (c >= chunks) return;
+    const int32_t s = chunk_sys[c];
+    if (s < 0) return;
+    const int64_t row = c * kChunkRows + threadIdx.x % kWave;
+    int longest = 0, band = 0;
+    if (row < sys_end[s])
+    {
+        const int64_t b = static_cast<int64_t>(ro[row]), e = static_cast<int64_t>(ro[row + 1]);
+        longest = static_cast<int>(e - b);
+        if (longest <= kTeamEntries)
+            for (int64_t k = b; k < e; ++k)
+            {
+                const int64_t col = static_cast<int64_t>(ci[k]);
+                const int64_t far = col < row ? row - col : col - row;
+                band = far > band ? static_cast<int>(far > 0x3fffffff ? 0x3fffffff : far) : band;
+                // a column outside the system leaves it to the per-kernel form
+                if (col < sys_chunk0[s] * kChunkRows || col >= sys_end[s]) longest = kTeamEntries + 1;
+            }
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off /= 2)
+    {
+        longest = max(longest, __shfl_xor(longest, off, kWave));
+        band = max(band, __shfl_xor(band, off, kWave));
+    }
+    if (threadIdx.x % kWave == 0)
+    {
+        atomicMax(&look[s].longest, longest);
+        atomicMax(&look[s].band, band);
+    }
+}
+
+__global__ void k_look_reset(int64_t systems, BatchLook* look)
+{
+    for (int64_t s = threadIdx.x; s < systems; s += blockDim.x) look[s] = BatchLook{0, 0};
+}
+
+size_t team_lds(int es, int rows_per_lane, int halo)
+{
+    return static_cast<size_t>(es) * (static_cast<size_t>(rows_per_lane) * kPersistThreads + 2 * static_cast<size_t>(halo));
+}
+
+constexpr size_t kTeamLds = 160 * 1024 - 2048;  // LDS of a CU less the static part
+
+template <typename S, typename I>
+const void* team_kernel(int rows_per_lane)
+{
+    if (rows_per_lane == 1) return reinterpret_cast<const void*>(k_batch_team<S, I, 1>);
+    if (rows_per_lane == 2) return reinterpret_cast<const void*>(k_batch_team<S, I, 2>);
+    if constexpr (sizeof(S) == 4) return reinterpret_cast<const void*>(k_batch_team<S, I, 4>);
+    return nullptr;
+}
+
+template <typename S, typename I>
+int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook>& look, const I* ro, const I* ci,
+              hipStream_t stream)
+{
+    const int most = sizeof(S) == 4 ? 4 : 2;  // rows per lane that the registers hold
+    const int es = static_cast<int>(sizeof(S));
+    int cus = 0;
+    if (!persist_enabled() || !persist_resident(ws, 1) || b.max_iterations > kTeamIterations) return PM_OK;
+    PM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ws->device));
+    const int slots = std::min(cus, kTeamSlots);
+    std::vector<int> order;
+    int64_t total[3] = {0, 0, 0};  // workgroups with 1, 2, 4 rows per lane
+    for (int64_t s = 0; s < b.systems; ++s)
+    {
+        const int64_t n = b.end[s] - b.begin[s];
+        const BatchLook& l = look[static_cast<size_t>(s)];
+        const int64_t piece = static_cast<int64_t>(most) * kPersistThreads;
+        const int64_t team = ceil_div(n, piece);
+        if (n <= 0 || b.skip[s] || l.longest > kTeamEntries || team > std::min(kTeamLargest, slots)) continue;
+        if (team > 1 && (team_lds(es, most, l.band) > kTeamLds || piece + 2 * static_cast<int64_t>(l.band) > 65535)) continue;
+        order.push_back(static_cast<int>(s));
+        for (int k = 0; k < 3; ++k) total[k] += ceil_div(n, static_cast<int64_t>(kPersistThreads) << k);
+    }
+    if (order.empty()) return PM_OK;
+    // as few rows per lane as let all teams run together (and no team grow past
+    // its decision's lanes)
+    int rows_per_lane = most;
+    for (int k = 0; (1 << k) < most; ++k)
+    {
+        bool fits = total[k] <= slots;
+        for (int s : order)
+        {
+            const int64_t piece = static_cast<int64_t>(kPersistThreads) << k;
+            fits = fits && ceil_div(b.end[s] - b.begin[s], piece) <= kTeamLargest;
+        }
+        if (fits)
+        {
+            rows_per_lane = 1 << k;
+            break;
+        }
+    }
+    const int64_t piece = static_cast<int64_t>(rows_per_lane) * kPersistThreads;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int l, int r) { return b.end[l] - b.begin[l] > b.end[r] - b.begin[r]; });
+    // launches of at most `slots` workgroups
+    std::vector<std::vector<TeamTask>> launches;
+    std::vector<TeamTask> now;
+    auto add = [&](int s) {
+        const int64_t n = b.end[s] - b.begin[s];
+        const int team = static_cast<int>(ceil_div(n, piece));
+        if (static_cast<int>(now.size()) + team > slots) return false;
+        const int slot0 = static_cast<int>(now.size());
+        for (int q = 0; q < team; ++q)
+            now.push_back(TeamTask{s, slot0, team, q, static_cast<int32_t>(n), look[static_cast<size_t>(s)].band, b.begin[s]});
+        return true;
+    };
+    for (int s : order)
+    {
+        if (add(s)) continue;
+        launches.push_back(std::move(now));
+        now.clear();
+        (void)add(s);
+    }
+    if (!now.empty()) launches.push_back(std::move(now));
+
+    const size_t words = static_cast<size_t>(slots) * static_cast<size_t>(piece);
+    const size_t plane_words = words * Exchange<S>::kWords;
+    const size_t control = (sizeof(TeamControl) + 255) & ~size_t(255);
+    const size_t control_all = control * launches.size();
+    // the control blocks come after the words, whose places then only ever hold words
+    const size_t need = 2 * plane_words * sizeof(word) + control_all;
+    // (blocks in a place that earlier held words, or the other way round, are
+    // cleared with the whole buffer when the layout changes)
+    if (need > ws->teams.bytes || ws->teams_words != plane_words || ws->teams_tag > 0xf0000000u)
+    {
+        PM_TRY(ws->teams.reserve(need));
+        hipLaunchKernelGGL(k_persist_clear, dim3(1024), dim3(kBlock), 0, stream, ws->teams.as<word>(),
+                           static_cast<int64_t>(ws->teams.bytes / sizeof(word)));
+        PM_HIP(hipGetLastError());
+        ws->teams_words = plane_words;
+        ws->teams_tag = 0;
+    }
+    const void* kernel = team_kernel<S, I>(rows_per_lane);
+    TeamArgs<S, I> a{};
+    a.ro = ro;
+    a.ci = ci;
+    a.values = static_cast<const S*>(b.a->values);
+    a.rhs = static_cast<const S*>(b.rhs);
+    a.x = static_cast<const S*>(b.x);
+    a.x_out = static_cast<S*>(b.x_out);
+    a.p = static_cast<const S*>(b.p);
+    a.r = static_cast<const S*>(b.r);
+    a.s = static_cast<const S*>(b.s);
+    a.w = static_cast<const S*>(b.w);
+    a.inv = static_cast<const S*>(b.inv);
+    a.st = b.st;
+    a.xu = ws->teams.as<word>();
+    a.xx = a.xu + plane_words;
+    a.plane = static_cast<int>(words);
+    a.max_iterations = b.max_iterations;
+    a.refresh = b.refresh;
+    // the tasks of every launch in one synchronous copy (the host arrays go out of scope)
+    char* blocks0 = ws->teams.as<char>() + 2 * plane_words * sizeof(word);
+    for (size_t k = 0; k < launches.size(); ++k)
+    {
+        auto* ctl = reinterpret_cast<TeamControl*>(blocks0 + k * control);
+        PM_HIP(hipMemcpyAsync(ctl->tasks, launches[k].data(), sizeof(TeamTask) * launches[k].size(),
+                              hipMemcpyHostToDevice, stream));
+    }
+    for (size_t k = 0; k < launches.size(); ++k)
+    {
+        auto* ctl = reinterpret_cast<TeamControl*>(blocks0 + k * control);
+        const int grid = static_cast<int>(launches[k].size());
+        int halo = 0;
+        for (const TeamTask& t : launches[k]) halo = std::max(halo, t.team > 1 ? t.halo : 0);
+        const size_t lds = team_lds(es, rows_per_lane, halo);
+        PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        a.ctl = ctl;
+        a.give_up = reinterpret_cast<PersistControl*>(ctl);
+        a.tag = ws->teams_tag;
+        ws->teams_tag += static_cast<uint32_t>(b.max_iterations) + 2u;
+        hipLaunchKernelGGL(k_team_reset, dim3(1), dim3(kTeamSlots), 0, stream, ctl);
+        PM_HIP(hipGetLastError());
+        void* args[] = {&a};
+        const hipError_t err = hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(kPersistThreads), args,
+                                                          static_cast<unsigned>(lds), stream);
+        if (persist_refused(err, ws)) break;
+        PM_HIP(err);
+        hipLaunchKernelGGL(k_team_commit<S>, dim3(grid), dim3(kBlock), 0, stream, ctl, static_cast<int>(piece),
+                           static_cast<const S*>(b.x_out), static_cast<S*>(b.x));
+        hipLaunchKernelGGL(k_team_states, dim3(1), dim3(kTeamSlots), 0, stream, ctl, grid, b.st, b.done_count);
+        PM_HIP(hipGetLastError());
+    }
+    // the launches vector is the source of the copies above
+    PM_HIP(hipStreamSynchronize(stream));
+    return PM_OK;
+}
+
+} // namespace
+
+int batch_teams_look(pm_workspace* ws, const BatchTeams& b, std::vector<BatchLook>& look, hipStream_t stream)
+{
+    look.assign(static_cast<size_t>(b.systems), BatchLook{0, 0});
+    if (b.systems == 0 || b.chunks == 0 || !persist_enabled()) return PM_OK;
+    PM_TRY(ws->scratch.reserve(sizeof(BatchLook) * static_cast<size_t>(b.systems)));
+    auto* dev = ws->scratch.as<BatchLook>();
+    hipLaunchKernelGGL(k_look_reset, dim3(1), dim3(kBlock), 0, stream, b.systems, dev);
+    const dim3 grid(static_cast<unsigned>(ceil_div(b.chunks, kBlock / kWave)));
+    if (use_compact(b.a))
+        hipLaunchKernelGGL(k_team_look<int32_t>, grid, dim3(kBlock), 0, stream, b.chunks, b.chunk_sys, b.sys_end,
+                           b.sys_chunk0, b.a->row_offsets32, b.a->col_indices32, dev);
+    else
+        hipLaunchKernelGGL(k_team_look<int64_t>, grid, dim3(kBlock), 0, stream, b.chunks, b.chunk_sys, b.sys_end,
+                           b.sys_chunk0, b.a->row_offsets, b.a->col_indices, dev);
+    PM_HIP(hipGetLastError());
+    PM_HIP(hipMemcpyAsync(look.data(), dev, sizeof(BatchLook) * look.size(), hipMemcpyDeviceToHost, stream));
+    PM_HIP(hipStreamSynchronize(stream));
+    return PM_OK;
+}
+
+int batch_teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook>& look, hipStream_t stream)
+{
+    const pm_csr* m = b.a;
+    const bool compact = use_compact(m);
+    if (m->dtype == PM_F64)
+        return compact ? teams_run<double>(ws, b, look, m->row_offsets32, m->col_indices32, stream)
+                       : teams_run<double>(ws, b, look, m->row_offsets, m->col_indices, stream);
+    return compact ? teams_run<float>(ws, b, look, m->row_offsets32, m->col_indices32, stream)
+                   : teams_run<float>(ws, b, look, m->row_offsets, m->col_indices, stream);
+}
+
+} // namespace pm

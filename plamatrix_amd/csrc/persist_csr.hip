@@ -300,10 +300,10 @@ int csr_run(pm_workspace* ws, const PersistProblem& p, const I* ro, const I* ci,
 
 } // namespace
 
-bool persist_csr_candidate(const PersistProblem& p, int device)
+bool persist_csr_candidate(const PersistProblem& p, const pm_workspace* ws)
 {
     return persist_enabled() && p.rows > 0 && p.rows <= kCsrRows && p.a->nnz <= p.rows * kCsrEntries &&
-           csr_per(p) <= kWavesPerBlock && persist_resident(csr_blocks(p), device);
+           csr_per(p) <= kWavesPerBlock && persist_resident(ws, csr_blocks(p));
 }
 
 int persist_csr_look(pm_workspace* ws, const PersistProblem& p, hipStream_t stream)

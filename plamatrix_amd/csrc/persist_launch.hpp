@@ -46,8 +46,10 @@ inline bool persist_enabled()
 }
 
 // Whether `blocks` workgroups of a CU each can run together.
-inline bool persist_resident(int blocks, int device)
+inline bool persist_resident(const pm_workspace* ws, int blocks)
 {
+    if (ws->cooperative_refused) return false;
+    const int device = ws->device;
     int coop = 0, cus = 0;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
@@ -56,6 +58,19 @@ inline bool persist_resident(int blocks, int device)
         return false;
     }
     return coop != 0 && blocks <= cus;
+}
+
+// A cooperative launch that the runtime turned down, as it does for every
+// process but the first that holds a cooperative queue on the device
+// (hipErrorIllegalState): the workspace stays on the per-kernel forms from then
+// on, without an error.
+inline bool persist_refused(hipError_t err, pm_workspace* ws)
+{
+    if (err != hipErrorCooperativeLaunchTooLarge && err != hipErrorNotSupported && err != hipErrorIllegalState)
+        return false;
+    (void)hipGetLastError();
+    ws->cooperative_refused = true;
+    return true;
 }
 
 // Every workgroup decides for itself, or eight decide and answer the rest.
@@ -101,11 +116,7 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
         void* args[] = {&a};
         const hipError_t err = hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads), args,
                                                           static_cast<unsigned>(lds), stream);
-        if (err == hipErrorCooperativeLaunchTooLarge || err == hipErrorNotSupported)
-        {
-            (void)hipGetLastError();
-            return PM_OK;
-        }
+        if (persist_refused(err, ws)) return PM_OK;
         PM_HIP(err);
         hipLaunchKernelGGL(k_persist_commit<S>, dim3(grid), dim3(kBlock), 0, stream, p.rows,
                            static_cast<const S*>(p.x_out), static_cast<S*>(p.x), a.ctl,

@@ -175,6 +175,7 @@ pm_workspace::~pm_workspace()
     dia_gt.release();
     blocks.release();
     persist.release();
+    teams.release();
     for (hipEvent_t& e : events)
         if (e) (void)hipEventDestroy(e);
     if (done_event) (void)hipEventDestroy(done_event);
@@ -241,6 +242,7 @@ int pm_workspace_close(pm_workspace* ws)
     ws->dia_gt.release();
     ws->blocks.release();
     ws->persist.release();
+    ws->teams.release();
     ws->capacity_rows = 0;
     ws->bound = false;
     ws->stream = nullptr;
@@ -253,7 +255,7 @@ size_t pm_workspace_capacity_bytes(const pm_workspace* ws)
     if (!ws) return 0;
     return ws->vectors.bytes + ws->partials.bytes + ws->state.bytes + ws->scratch.bytes + ws->sort.bytes +
            ws->refine.bytes + ws->batch.bytes + ws->dense.bytes +
-           ws->dia.bytes + ws->dia_g.bytes + ws->dia_gt.bytes + ws->blocks.bytes + ws->persist.bytes;
+           ws->dia.bytes + ws->dia_g.bytes + ws->dia_gt.bytes + ws->blocks.bytes + ws->persist.bytes + ws->teams.bytes;
 }
 
 int64_t pm_workspace_capacity_rows(const pm_workspace* ws) { return ws ? ws->capacity_rows : 0; }

@@ -127,6 +127,10 @@ struct pm_workspace
     pm::DeviceBuffer dia_gt;    // ... and of G^T
     pm::DeviceBuffer persist;   // persistent solver: control block and exchange words
     uint32_t persist_tag = 0;   // last exchange tag used in it
+    bool cooperative_refused = false; // the runtime turned a cooperative launch down (another process has the queue)
+    pm::DeviceBuffer teams;     // persistent batch: exchange words and control blocks
+    size_t teams_words = 0;     // words before its control blocks
+    uint32_t teams_tag = 0;     // last exchange tag used in it
     int32_t last_diagonals = 0; // diagonals of the last solve's layout (0: CSR kernels)
     int32_t last_value_streams = 0; // value arrays its row sums read (fewer than the diagonals when mirrored)
     int32_t last_form = 0;      // kernels per iteration of the last solve's form (1, 2 or 3)

@@ -1,0 +1,119 @@
+"""The persistent batch (plamatrix_amd/csrc/persist_batch.hip): systems of short,
+banded rows solved by teams of workgroups, against the per-kernel batch
+(PLAMATRIX_AMD_PERSISTENT=0).  The dot products are summed in another order, so
+iteration counts may differ by a step or two and the solutions by what the stop
+rule leaves: both end at ||r|| <= rel ||b|| of the recursive residual, so their
+difference in the A-norm is of that size; with rel = 1e-10 (FP64) and matrices of
+condition below 1e4 that is 1e-6 of x, and 1e-5 * 1e3 = 1e-2 with rel = 1e-5
+(FP32, condition below 1e3).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+from plamatrix_amd import capi, generators  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    capi.lib()
+    return torch.device("cuda:0")
+
+
+def diag_system(n):
+    return generators.CSRHost(n, n, np.arange(n + 1, dtype=np.int64), np.arange(n, dtype=np.int64),
+                              np.linspace(1.0, 3.0, n))
+
+
+def long_rows(n, seed):
+    rng = np.random.default_rng(seed)
+    m = rng.standard_normal((n, n)) * 0.1
+    m = m @ m.T + np.eye(n) * n * 0.05
+    return generators.CSRHost(n, n, np.arange(n + 1, dtype=np.int64) * n, np.tile(np.arange(n, dtype=np.int64), n),
+                              m.reshape(-1))
+
+
+def members(kind):
+    lap, box = generators.laplacian2d_csr, generators.diffusion3d_box_csr
+    if kind == "edges":  # one workgroup and one row beyond, for 1, 2 and 4 rows per lane; tiny systems; long rows
+        return [diag_system(1), lap(8, 8), lap(32, 32), lap(25, 41), lap(64, 32), lap(2049, 1), lap(64, 64),
+                lap(17, 241), long_rows(60, 1), diag_system(63)]
+    if kind == "teams":  # halos narrower and wider than a piece
+        return [lap(150, 90), box(25, 24, 23, seed=1), lap(40, 400), box(60, 50, 4, seed=2), lap(3000, 5)]
+    # more workgroups than CUs at any rows per lane: several launches
+    return [lap(150, 140 + i % 7) for i in range(60)] + [box(30, 30, 30, seed=i) for i in range(6)]
+
+
+def batch(kind, dtype):
+    hosts = [generators.CSRHost(h.rows, h.cols, h.row_offsets, h.col_indices, h.values.astype(dtype)) for h in members(kind)]
+    h, begin, end = generators.block_diagonal(hosts, dtype=dtype)
+    return h, begin, end
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["edges", "teams", "launches"])
+def test_teams_match_the_per_kernel_batch(dev, monkeypatch, kind, dtype):
+    h, begin, end = batch(kind, dtype)
+    rel, bound = (1e-10, 1e-6) if dtype == np.float64 else (1e-5, 1e-2)
+    b = torch.zeros(h.rows, dtype=torch.float64)
+    for i, (s, e) in enumerate(zip(begin, end)):
+        b[s:e] = torch.from_numpy(generators.rhs_normal(e - s, seed=i).astype(np.float64))
+    b = b.to(torch.float32 if dtype == np.float32 else torch.float64).to(dev)
+    x0 = 0.1 * torch.ones_like(b)
+    for compact, jacobi, refresh, most in ((True, True, 50, 3000), (False, False, 0, 3000), (True, True, 10, 7)):
+        a = capi.to_device_csr(h, compact=compact)
+        out, storage = {}, {}
+        for flag in ("0", "1"):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+            ws = capi.Workspace()
+            for _ in range(2):  # the second solve meets the first one's exchange words
+                x = x0.clone()
+                reps = capi.batch_pcg(a, begin, end, b, x, ws, pol=capi.policy(refresh_interval=refresh),
+                                      use_jacobi=jacobi, relative_tolerance=rel, max_iterations=most)
+                torch.cuda.synchronize()
+                got = [(r.converged, r.iterations, r.status) for r in reps]
+                if flag == "1" and flag in out and kind != "edges":
+                    assert got == out[flag][0] and torch.equal(x, out[flag][1])  # every system in teams: deterministic
+                out[flag] = (got, x.clone(), reps)
+            storage[flag] = ws.capacity_bytes
+        assert storage["1"] > storage["0"]
+        for i, (s, e) in enumerate(zip(begin, end)):
+            (c0, n0, s0), (c1, n1, s1) = out["0"][0][i], out["1"][0][i]
+            assert (c0, s0) == (c1, s1) and abs(n0 - n1) <= max(2, 0.02 * n0), (i, n0, n1)
+            xa, xb = out["0"][1][s:e].double(), out["1"][1][s:e].double()
+            assert float((xa - xb).norm()) <= bound * float(xa.norm()), i
+            r0, r1 = out["0"][2][i], out["1"][2][i]
+            assert abs(r0.initial_residual - r1.initial_residual) <= 1e-12 * r0.initial_residual
+        gaps = torch.ones(h.rows, dtype=torch.bool)
+        for s, e in zip(begin, end):
+            gaps[s:e] = False
+        assert torch.equal(out["1"][1].cpu()[gaps], x0.cpu()[gaps])  # padding rows are not touched
+
+
+def test_stops_before_the_launch(dev, monkeypatch):
+    # a rejected diagonal, a zero right-hand side and an iteration limit of 0
+    # keep their states; the other systems go on
+    h, begin, end = batch("teams", np.float64)
+    v = h.values.copy()
+    row = int(begin[1]) + 5
+    k = slice(h.row_offsets[row], h.row_offsets[row + 1])
+    v[k][h.col_indices[k] == row] = -2.0
+    v[np.arange(h.row_offsets[row], h.row_offsets[row + 1])[h.col_indices[k] == row]] = -2.0
+    a = capi.to_device_csr(generators.CSRHost(h.rows, h.cols, h.row_offsets, h.col_indices, v), compact=True)
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=3).astype(np.float64)).to(dev)
+    b[int(begin[2]):int(end[2])] = 0.0
+    for most in (0, 2000):
+        out = {}
+        for flag in ("0", "1"):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+            x = torch.zeros_like(b)
+            reps = capi.batch_pcg(a, begin, end, b, x, capi.Workspace(), relative_tolerance=1e-9, max_iterations=most)
+            torch.cuda.synchronize()
+            out[flag] = [(r.converged, r.status, r.bad_row) for r in reps]
+            assert not bool(x[int(begin[1]):int(end[1])].any()) and not bool(x[int(begin[2]):int(end[2])].any())
+        assert out["0"] == out["1"]
+        assert out["1"][1][1] == 6 and out["1"][1][2] == row and out["1"][2][0]
