@@ -60,6 +60,12 @@ __global__ __launch_bounds__(kBlock) void k_dia_detect(int64_t rows, const I* __
     if (threadIdx.x == 0) flags = 0;
     __syncthreads();
     int my_flags = 0;
+    // the table's first offsets in registers: an offset among them needs no
+    // look into LDS (a slot that is set never changes)
+    constexpr int kKnown = 8;
+    int known[kKnown];
+#pragma unroll
+    for (int s = 0; s < kKnown; ++s) known[s] = kEmpty;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
     for (int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; r < rows; r += stride)
     {
@@ -72,7 +78,16 @@ __global__ __launch_bounds__(kBlock) void k_dia_detect(int64_t rows, const I* __
             const int64_t c = static_cast<int64_t>(ci[k]);
             if (c <= prev) my_flags |= 1;
             prev = c;
-            if (!dia_insert(local, static_cast<int>(c - r), true)) my_flags |= 2;
+            const int off = static_cast<int>(c - r);
+            bool seen = false;
+#pragma unroll
+            for (int s = 0; s < kKnown; ++s) seen = seen || known[s] == off;
+            if (!seen)
+            {
+                if (!dia_insert(local, off, true)) my_flags |= 2;
+#pragma unroll
+                for (int s = 0; s < kKnown; ++s) known[s] = __atomic_load_n(&local[s], __ATOMIC_RELAXED);
+            }
             if constexpr (UNIT)
             {
                 const double a = static_cast<double>(v[k]);
