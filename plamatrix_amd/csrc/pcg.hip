@@ -2167,11 +2167,21 @@ int finish_report(const SolverState& fin, const pm_solver_options* options, pm_s
     return PM_OK;
 }
 
+// The diagonal layouts of a solve's matrices, for a caller that solves with the
+// same arrays again before it returns (the passes of a refinement: nothing can
+// change them in between).
+struct SolveLayouts
+{
+    bool built = false;
+    bool unit = false;  // every Jacobi inverse is exactly 1
+    DiaLayout dia, dia_g, dia_gt;
+};
+
 template <typename S>
 int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_blocks, int64_t bsize, int pre,
                    const pm_solver_options* options, const pm_solve_policy* policy_in, pm_solver_report* report,
                    pm_workspace* ws, hipStream_t stream, const pm_csr* gf = nullptr, const pm_csr* gtf = nullptr,
-                   int tol_rule = 0)
+                   int tol_rule = 0, SolveLayouts* keep = nullptr)
 {
     const Policy policy = resolve_policy(policy_in, a->rows);
     Problem pb{};
@@ -2184,7 +2194,14 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     pb.bsize = pre == kPreBlock ? bsize : 1;
     pb.pre = pre;
     PM_TRY(prepare(ws, pb, stream));
-    if (dia_wanted(a))
+    if (keep != nullptr && keep->built)
+    {
+        pb.dia = keep->dia;
+        pb.dia_g = keep->dia_g;
+        pb.dia_gt = keep->dia_gt;
+        if (keep->unit) pb.pre = kPreNone;
+    }
+    else if (dia_wanted(a))
     {
         // Jacobi on a matrix whose every Jacobi inverse is exactly 1 is the
         // unpreconditioned iteration bit for bit (z = 1 * r = r): it then runs
@@ -2199,12 +2216,20 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
         const bool mirror = mirror_env == nullptr || mirror_env[0] != '0';
         PM_TRY(dia_build(ws->dia, a, &pb.dia, stream, check_unit ? &unit : nullptr, mirror));
         if (check_unit && unit) pb.pre = kPreNone;
+        if (keep != nullptr) keep->unit = check_unit && unit;
     }
-    if (pb.pre == kPreFactored && dia_wanted(gf) && dia_wanted(gtf))
+    if (!(keep != nullptr && keep->built) && pb.pre == kPreFactored && dia_wanted(gf) && dia_wanted(gtf))
     {
         PM_TRY(dia_build(ws->dia_g, gf, &pb.dia_g, stream));
         PM_TRY(dia_build(ws->dia_gt, gtf, &pb.dia_gt, stream));
         if (!pb.dia_g.active || !pb.dia_gt.active) pb.dia_g.active = pb.dia_gt.active = false;
+    }
+    if (keep != nullptr && !keep->built)
+    {
+        keep->built = true;
+        keep->dia = pb.dia;
+        keep->dia_g = pb.dia_g;
+        keep->dia_gt = pb.dia_gt;
     }
     pb.fuse_step = fuse_step_wanted(pb);
     pb.single_reduction = single_reduction_wanted(pb);
@@ -2228,16 +2253,16 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     // r.z partials with grid_rows workgroups
     pb.cg_factored = pb.single_reduction && pb.pre == kPreFactored;
     if (pb.cg_factored) pb.grid_rows = pb.grid_units;
+    const char* fused_env = std::getenv("PLAMATRIX_AMD_CG_FUSED");
+    const bool fused_wanted = fused_env == nullptr || fused_env[0] != '0';
     {
         // on the diagonal layout, one kernel per iteration; factored with a
         // four-diagonal G, G r and G^T t in one kernel (PLAMATRIX_AMD_CG_FUSED=0
         // keeps two, and three)
-        const char* env = std::getenv("PLAMATRIX_AMD_CG_FUSED");
         bool pair = pb.dia_g.active && pb.dia_g.args.ndiag == 4 && pb.dia_gt.args.ndiag == 4;
         for (int d = 0; pair && d < 4; ++d)
             pair = pb.dia_g.args.off[d] <= 0 && pb.dia_gt.args.off[3 - d] == -pb.dia_g.args.off[d];
-        pb.cg_fused = pb.single_reduction && (!pb.cg_factored || pair) && pb.dia.active && pb.r2 != nullptr &&
-                      (env == nullptr || env[0] != '0');
+        pb.cg_fused = pb.single_reduction && (!pb.cg_factored || pair) && pb.dia.active && pb.r2 != nullptr && fused_wanted;
     }
     ws->last_diagonals = pb.dia.active ? pb.dia.args.ndiag : 0;
     ws->last_value_streams = pb.dia.active ? pb.dia.streams : 0;
@@ -2265,6 +2290,8 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     pp.dtype = a->dtype;
     pp.a = a;
     pp.dia = &pb.dia;
+    pp.dia_g = &pb.dia_g;
+    pp.dia_gt = &pb.dia_gt;
     pp.jacobi = pb.pre == kPreJacobi;
     pp.rhs = rhs;
     pp.x = x;
@@ -2283,9 +2310,10 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     pp.grow = policy.grow;
     const bool one_launch = pb.single_reduction && !pb.cg_factored;
     const bool csr = one_launch && !pb.dia.active;
-    auto run = one_launch && pb.cg_fused && persist_wanted(pp, ws) ? persist_run
-               : csr && persist_small_wanted(pp)                           ? persist_small_run
-                                                                           : nullptr;
+    auto run = one_launch && pb.cg_fused && persist_wanted(pp, ws)  ? persist_run
+               : csr && persist_small_wanted(pp)                    ? persist_small_run
+               : pb.cg_factored && fused_wanted && persist_factored_wanted(pp, ws) ? persist_factored_run
+                                                                    : nullptr;
     const bool look = csr && run == nullptr && persist_csr_candidate(pp, ws);
     if (look) PM_TRY(persist_csr_look(ws, pp, stream));
     PM_TRY(initialise());
@@ -2320,7 +2348,7 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
         {
             // a restart: the three-kernel form from iteration `next` on,
             // with the chunks the schedule has there
-            pb.single_reduction = pb.cg_fused = false;
+            pb.single_reduction = pb.cg_fused = pb.cg_factored = false;
             while (launched < next)
             {
                 launched += K;
@@ -2641,6 +2669,7 @@ int refine(const pm_csr* a, const double* b, double* x, const pm_solver_options*
     in.require_convergence = 0;
     in.absolute_tolerance = 0.0;
     pm_refine_report rep{};
+    SolveLayouts layouts;
     for (int outer = 0;; ++outer)
     {
         hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, stream, counter);
@@ -2673,7 +2702,7 @@ int refine(const pm_csr* a, const double* b, double* x, const pm_solver_options*
         pm_solver_report inner_rep{};
         in.relative_tolerance = refine_pass_tolerance(inner->relative_tolerance, relres, target);
         const int pre = gf ? kPreFactored : (in.use_jacobi ? kPreJacobi : kPreNone);
-        PM_TRY(adaptive_solve<float>(a, rf, d, nullptr, 1, pre, &in, policy, &inner_rep, ws, stream, gf, gtf));
+        PM_TRY(adaptive_solve<float>(a, rf, d, nullptr, 1, pre, &in, policy, &inner_rep, ws, stream, gf, gtf, 0, &layouts));
         rep.inner_iterations += inner_rep.iterations;
         hipLaunchKernelGGL(k_accumulate, dim3(grid), dim3(kBlock), 0, stream, n, x, d, norm);
         PM_HIP(hipGetLastError());

@@ -18,14 +18,14 @@ namespace pm
 constexpr int kMaxGrownChunk = 64;
 
 // A solve whose vectors sit where the per-kernel iteration keeps them between
-// chunks: r, u (z; Jacobi only), w (q), p (p0) and s (p1), the partials of the
-// initialisation in region 1.
+// chunks: r, u (z; with a preconditioner), w (q), p (p0) and s (p1), the partials
+// of the initialisation in region 1.
 struct PersistProblem
 {
     int64_t rows;
     int32_t dtype;
     const pm_csr* a;
-    const DiaLayout* dia;
+    const DiaLayout *dia, *dia_g, *dia_gt;
     bool jacobi;
     const void* rhs;
     void* x;
@@ -67,6 +67,12 @@ int persist_csr_look(pm_workspace* ws, const PersistProblem& p, hipStream_t stre
 int persist_csr_fits(pm_workspace* ws, bool* fits);
 int persist_csr_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream,
                     int* outcome, int64_t* next, SolverState* state);
+
+// The same with a factored preconditioner, all three matrices on the diagonal
+// layout (persist_factored.hip).
+bool persist_factored_wanted(const PersistProblem& p, const pm_workspace* ws);
+int persist_factored_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream,
+                         int* outcome, int64_t* next, SolverState* state);
 
 // The chunk schedule of an adaptive solve: chunk c covers iterations
 // [end(c - 1), end(c)).  Both forms of a solve must leave the single-reduction

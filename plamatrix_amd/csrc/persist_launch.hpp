@@ -76,17 +76,18 @@ inline bool persist_refused(hipError_t err, pm_workspace* ws)
 // Every workgroup decides for itself, or eight decide and answer the rest.
 inline int persist_leaders(int blocks) { return blocks <= 64 ? blocks : kXcds; }
 
-// Runs the launches of a solve; `a` is complete but for the exchange storage,
-// x and the iteration range.
+// Runs the launches of a solve; `a` is complete but for the exchange storage (of
+// `vectors` vectors, xu and xx first) and the iteration range.
 template <typename S, typename Args>
 int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void* kernel, int blocks, size_t lds,
-                 int64_t max_iterations, hipStream_t stream, int* outcome, int64_t* next, SolverState* state)
+                 int64_t max_iterations, hipStream_t stream, int* outcome, int64_t* next, SolverState* state,
+                 int vectors = 2)
 {
     *outcome = kPersistAbandoned;
     PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
     const size_t words = static_cast<size_t>(p.rows) * Exchange<S>::kWords;
     const size_t control = (sizeof(PersistControl) + 255) & ~size_t(255);
-    const size_t need = control + 2 * words * sizeof(word);
+    const size_t need = control + static_cast<size_t>(vectors) * words * sizeof(word);
     const bool grown = need > ws->persist.bytes;
     PM_TRY(ws->persist.reserve(need));
     if (grown || ws->persist_tag > 0xf0000000u)

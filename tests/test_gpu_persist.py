@@ -246,3 +246,41 @@ def test_wide_csr_restart_hands_over(dev, monkeypatch):
             torch.cuda.synchronize()
             out[flag] += (x.cpu().numpy().tobytes(),)
         assert out["0"] == out["1"], shift
+
+
+FACTORED = [
+    ("diffusion", (41, 43, 40), np.float32, 0),   # far outermost diagonals, a short last piece
+    ("diffusion", (11, 13, 480), np.float32, 20),  # every neighbour in the halos
+    ("diffusion", (45, 41, 40), np.float64, 50),
+    ("diffusion", (71, 70, 67), np.float32, 20),  # two rows per lane
+    ("laplace", (260, 300), np.float64, 0),       # five diagonals
+    ("laplace", (2500, 31), np.float32, 20),
+]
+
+
+@pytest.mark.parametrize("kind,dims,dtype,refresh", FACTORED)
+def test_factored_solve_is_bitwise(dev, monkeypatch, kind, dims, dtype, refresh):
+    a = capi.to_device_csr(matrix(kind, dims, dtype), compact=True)
+    net = capi.FsaiNet(seed=0)
+    p = capi.fsai_initial_parameters(2)
+    p[-70:-1] += 0.03 * np.random.default_rng(4).standard_normal(69).astype(np.float32)
+    net.parameters = p
+    graph = capi.FsaiGraph(a)
+    capi.fsai_forward(net, graph)
+    b = torch.from_numpy(generators.rhs_normal(a.rows, seed=37).astype(dtype)).to(dev)
+    for most in (0, 1, 300):
+        out, storage = {}, {}
+        for flag in ("0", "1"):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+            ws = capi.Workspace()
+            for _ in range(2):  # the second solve meets the first one's exchange words
+                x = torch.full_like(b, 0.5)
+                rep = capi.pcg_factored(a, b, x, graph, ws, pol=capi.policy(refresh_interval=refresh),
+                                        relative_tolerance=1e-4, max_iterations=most)
+                torch.cuda.synchronize()
+                got = (rep.converged, rep.iterations, rep.initial_residual, rep.final_residual, x.cpu().numpy().tobytes())
+                assert out.setdefault(flag, got) == got
+            assert ws.solver_form in (4, 5)
+            storage[flag] = ws.capacity_bytes
+        assert storage["1"] > storage["0"]  # the exchange words: the persistent kernel ran
+        assert out["0"] == out["1"], most
