@@ -24,4 +24,27 @@ int64_t radix_hist_words(int64_t count);
 // Smallest b with 2^b >= n.
 int bits_for(int64_t n);
 
+// Rank of an active lane among the wavefront's earlier occurrences of its digit,
+// by ballots; `count`: the wavefront's running count per digit.  Lanes of a
+// wavefront run in step, so every lane reads the count before the first lane of
+// its digit raises it.
+__device__ __forceinline__ unsigned wave_rank(bool active, unsigned digit, int bits, unsigned short* count)
+{
+    unsigned long long peers = __ballot(active);
+    for (int bit = 0; bit < bits; ++bit)
+    {
+        const unsigned long long ones = __ballot((digit >> bit) & 1u);
+        peers &= ((digit >> bit) & 1u) ? ones : ~ones;
+    }
+    const unsigned below = static_cast<unsigned>(__popcll(peers & ((1ull << (threadIdx.x % kWave)) - 1ull)));
+    const unsigned before =
+        active ? __hip_atomic_load(count + digit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) : 0u;
+    __builtin_amdgcn_wave_barrier();
+    if (active && below == 0)
+        __hip_atomic_store(count + digit, static_cast<unsigned short>(before + __popcll(peers)), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WAVEFRONT);
+    __builtin_amdgcn_sched_barrier(0);  // one round's ballots at a time
+    return before + below;
+}
+
 } // namespace pm

@@ -58,6 +58,9 @@ struct CooStatus
     unsigned long long invalid_value;   // first triplet (or run) with a non-finite value / sum
     long long nnz;                      // combined nnz
     long long expected_nnz;             // caller's output nnz (-1 when unchecked)
+    unsigned long long unsorted;        // conversion by buckets: given up, the keys are only packed
+    unsigned long long most;            // ... triplets of its largest bucket
+    unsigned long long ticket;          // host copy: which conversion the record is of
 };
 
 // One recorded kernel launch: the function, its shape and a private copy of
@@ -151,6 +154,10 @@ struct pm_workspace
     int coo_key_bits = 0;
     const void* coo_values = nullptr;
     bool coo_prepared = false;
+    bool coo_buckets = false;               // by buckets (coo_bucket.hpp)
+    bool coo_resolved = false;              // ... and known to have been sorted
+    bool coo_publish = false;               // kernels leave the status record in host_coo (prepare / nnz / finish)
+    unsigned long long coo_ticket = 0;
     bool coo_pending_status = false;
     pm::CooStatus* host_coo = nullptr;      // pinned
     unsigned long long* host_batch = nullptr;  // pinned, 2 slots: stopped-system counts

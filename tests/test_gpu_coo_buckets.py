@@ -1,0 +1,124 @@
+"""COO -> CSR by row buckets against the LSD sort (the asynchronous call), bit for
+bit: sizes around a bucket's and a tile's edges, and shapes that leave the buckets."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from plamatrix_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    capi.lib()
+    return torch.device("cuda:0")
+
+
+def triplets(rows, cols, count, kind, dtype, seed):
+    rng = np.random.default_rng(seed)
+    r = rng.integers(0, rows, count)
+    c = rng.integers(0, cols, count)
+    if kind == "stencil":  # near the diagonal, most keys repeated
+        c = np.clip(r * cols // rows + rng.integers(-2, 3, count), 0, cols - 1)
+    elif kind == "arrow":  # half of the triplets in one row: its bucket overflows
+        r[rng.random(count) < 0.5] = rows // 3
+    elif kind == "one":  # one entry
+        r[:], c[:] = rows - 1, cols - 1
+    elif kind == "sorted":
+        order = np.lexsort((c, r))
+        r, c = r[order], c[order]
+    v = rng.standard_normal(count).astype(dtype)
+    return r, c, v
+
+
+CASES = [
+    (1, 1, 1, "uniform"), (1, 1, 5000, "uniform"), (3, 2, 64, "uniform"), (40, 7, 65, "one"),
+    (8192, 8192, 1025, "uniform"), (8193, 8192, 3000, "uniform"), (500, 500, 8192, "stencil"),
+    (5000, 5000, 8193, "stencil"), (2025, 2025, 10900, "stencil"), (5000, 900, 40000, "sorted"),
+    (70000, 70000, 262145, "stencil"), (300, 300, 300000, "uniform"), (100000, 100000, 50000, "uniform"),
+    (3, 1 << 29, 9000, "uniform"), (3, 1 << 33, 9000, "uniform"), (20000, 20000, 100000, "arrow"),
+    (30000, 30000, 60000, "one"), (5000000, 50, 300000, "uniform"), (190000, 190000, 1100000, "stencil"),
+]
+
+
+@pytest.mark.parametrize("index", range(len(CASES)))
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_buckets_are_the_lsd_sort(dev, index, dtype):
+    rows, cols, count, kind = CASES[index]
+    r, c, v = triplets(rows, cols, count, kind, dtype, index)
+    r, c, v = (torch.from_numpy(t).to(dev) for t in (r, c, v))
+    ws = capi.Workspace()
+    for _ in range(2):  # the second conversion meets the first one's tables
+        a = capi.coo_to_csr(rows, cols, r, c, v, ws)
+    out = capi.DeviceCSR(rows, cols, torch.empty_like(a.row_offsets), torch.empty_like(a.col_indices),
+                         torch.empty_like(a.values))
+    capi.coo_to_csr_async(rows, cols, r, c, v, out, ws)
+    torch.cuda.synchronize()
+    ws.check_status()
+    assert torch.equal(a.row_offsets, out.row_offsets)
+    assert torch.equal(a.col_indices, out.col_indices)
+    assert a.values.cpu().numpy().tobytes() == out.values.cpu().numpy().tobytes()
+
+
+@pytest.mark.parametrize("count", [500, 20000])
+def test_errors_name_the_first_offset(dev, count):
+    r, c, v = triplets(900, 900, count, "stencil", np.float64, 3)
+    bad = r.copy()
+    bad[[count - 1, 77]] = 900, -1
+    ws = capi.Workspace()
+    up = lambda *t: [torch.from_numpy(x).to(dev) for x in t]
+    with pytest.raises(Exception, match="out of range at source offset 77"):
+        capi.coo_to_csr(900, 900, *up(bad, c, v), ws)
+    w = v.copy()
+    w[[count - 1, 91]] = np.inf, np.nan
+    with pytest.raises(Exception, match="non-finite value at source offset 91"):
+        capi.coo_to_csr(900, 900, *up(r, c, w), ws)
+    # a sum that overflows is met by the fold
+    r[:2], c[:2], v[:2] = 5, 5, 1.7e308
+    with pytest.raises(Exception, match="non-finite value at source offset 1"):
+        capi.coo_to_csr(900, 900, *up(r, c, v), ws)
+    assert capi.coo_to_csr(900, 900, *up(r, c, np.ones(count)), ws).values.sum().item() == count
+
+
+@pytest.mark.parametrize("kind", ["stencil", "arrow"])
+@pytest.mark.parametrize("capture", [False, True])
+def test_finish_without_reading_the_nnz(dev, kind, capture):
+    """A caller that knows the nnz may finish right away, also into a graph."""
+    rows, count = 20000, 100000
+    r, c, v = triplets(rows, rows, count, kind, np.float64, 8)
+    r, c, v = (torch.from_numpy(t).to(dev) for t in (r, c, v))
+    want = capi.coo_to_csr(rows, rows, r, c, v, capi.Workspace())
+    ws = capi.Workspace()
+    got = [torch.zeros_like(t) for t in (want.row_offsets, want.col_indices, want.values)]
+    i64, p = ctypes.c_int64, lambda t: ctypes.c_void_p(t.data_ptr())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        stream = capi.current_stream()
+        capi.check(capi.lib().pm_coo_to_csr_prepare(i64(rows), i64(rows), i64(count), p(r), p(c), p(v),
+                                                    ctypes.c_int32(capi.dtype_code(v)),
+                                                    ctypes.c_int32(capi.PM_COO_CHECK_FINITE), ws.handle, stream))
+        finish = lambda: capi.check(capi.lib().pm_coo_to_csr_finish(
+            p(got[0]), p(got[1]), p(got[2]), i64(want.nnz), ws.handle, stream))
+        if not capture:
+            finish()
+    side.synchronize()
+    if capture:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            stream = capi.current_stream()
+            finish()
+        for _ in range(3):
+            for t in got:
+                t.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got[0], want.row_offsets) and torch.equal(got[1], want.col_indices)
+            assert torch.equal(got[2], want.values)
+    else:
+        assert torch.equal(got[0], want.row_offsets) and torch.equal(got[1], want.col_indices)
+        assert torch.equal(got[2], want.values)
