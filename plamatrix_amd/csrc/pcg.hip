@@ -219,6 +219,34 @@ __global__ __launch_bounds__(kDirBlock) void k_spmv_den(int64_t rows, const I* _
 constexpr int kLongLanes = 8;
 constexpr int64_t kLongRowEntries = 32;  // average entries per row from which the lanes kernel serves
 
+// A lane's share of a long row, gathered kLongAhead entries ahead of the ordered
+// multiply-adds (a row of 360 entries is 45 dependent gathers per lane otherwise).
+constexpr int kLongAhead = 8;
+template <typename S, typename I, typename Gather>
+__device__ __forceinline__ S long_row_share(int64_t k, int64_t e0, const I* __restrict__ ci, const S* __restrict__ v,
+                                            Gather gather)
+{
+    S acc = S(0);
+    for (; k < e0; k += kLongAhead * kLongLanes)
+    {
+        S a[kLongAhead], g[kLongAhead];
+        I c[kLongAhead];
+#pragma unroll
+        for (int j = 0; j < kLongAhead; ++j)
+        {
+            const bool in = k + j * kLongLanes < e0;
+            c[j] = in ? ci[k + j * kLongLanes] : I(0);
+            a[j] = in ? v[k + j * kLongLanes] : S(0);
+        }
+#pragma unroll
+        for (int j = 0; j < kLongAhead; ++j) g[j] = gather(c[j]);
+#pragma unroll
+        for (int j = 0; j < kLongAhead; ++j)
+            if (k + j * kLongLanes < e0) acc = fma_s(a[j], g[j], acc);
+    }
+    return group_sum<kLongLanes>(acc);
+}
+
 template <typename S, typename I>
 __global__ __launch_bounds__(kDirBlock) void k_spmv_den_lanes(int64_t rows, const I* __restrict__ ro,
                                                               const I* __restrict__ ci, const S* __restrict__ v,
@@ -235,13 +263,49 @@ __global__ __launch_bounds__(kDirBlock) void k_spmv_den_lanes(int64_t rows, cons
     for (int64_t row = begin + group; row < end; row += gpb)
     {
         const int64_t s0 = ro[row], e0 = ro[row + 1];
-        S acc = S(0);
-        for (int64_t k = s0 + lane; k < e0; k += kLongLanes) acc = fma_s(v[k], p[ci[k]], acc);
-        acc = group_sum<kLongLanes>(acc);
+        const S acc = long_row_share<S, I>(s0 + lane, e0, ci, v, [=](I c) { return p[c]; });
         if (lane == 0)
         {
             q[row] = acc;
             den = __builtin_fma(static_cast<double>(p[row]), static_cast<double>(acc), den);
+        }
+    }
+    double part[1] = {den};
+    publish_partials<1>(part, partials + kPartialsDen);
+}
+
+// k_direction and k_spmv_den_lanes in one kernel, p_new = z + beta p_old formed in
+// the gathers with k_direction's multiply-add: bitwise the two.  These systems'
+// vectors (under kDirectLaunchRows rows) sit in L2, so the second gather costs
+// less than the launch: 360 rows 2.3 + 3.4 us and a launch gap, now 4.3; 12,000 rows
+// 2.6 + 3.5, now 4.3.
+template <typename S, typename I>
+__global__ __launch_bounds__(kDirBlock) void k_dir_spmv_lanes(int64_t rows, const I* __restrict__ ro,
+                                                              const I* __restrict__ ci, const S* __restrict__ v,
+                                                              const S* __restrict__ z, const S* __restrict__ p_old,
+                                                              S* __restrict__ p_new, S* __restrict__ q,
+                                                              SolverState* st, double* partials, int par, int count_res)
+{
+    if (st->done != kRunning) return;
+    double beta = 0.0;
+    if (direction_decision<S>(st, partials, par, count_res, beta) != kRunning) return;
+    const S b = static_cast<S>(beta);
+    constexpr int64_t gpb = kDirBlock / kLongLanes;
+    const int group = threadIdx.x / kLongLanes;
+    const int lane = threadIdx.x % kLongLanes;
+    int64_t begin, end;
+    block_range(rows, gpb, begin, end);
+    double den = 0.0;
+    for (int64_t row = begin + group; row < end; row += gpb)
+    {
+        const int64_t s0 = ro[row], e0 = ro[row + 1];
+        const S acc = long_row_share<S, I>(s0 + lane, e0, ci, v, [=](I c) { return fma_s(b, p_old[c], z[c]); });
+        if (lane == 0)
+        {
+            const S pn = fma_s(b, p_old[row], z[row]);
+            p_new[row] = pn;
+            q[row] = acc;
+            den = __builtin_fma(static_cast<double>(pn), static_cast<double>(acc), den);
         }
     }
     double part[1] = {den};
@@ -267,8 +331,23 @@ __global__ __launch_bounds__(kBlock) void k_residual_lanes(int64_t rows, const I
     {
         const int64_t s0 = ro[row], e0 = ro[row + 1];
         double acc = 0.0;
-        for (int64_t k = s0 + lane; k < e0; k += kLongLanes)
-            acc = __builtin_fma(static_cast<double>(v[k]), static_cast<double>(x[ci[k]]), acc);
+        for (int64_t k = s0 + lane; k < e0; k += kLongAhead * kLongLanes)
+        {
+            S a[kLongAhead], g[kLongAhead];
+            I c[kLongAhead];
+#pragma unroll
+            for (int j = 0; j < kLongAhead; ++j)
+            {
+                const bool in = k + j * kLongLanes < e0;
+                c[j] = in ? ci[k + j * kLongLanes] : I(0);
+                a[j] = in ? v[k + j * kLongLanes] : S(0);
+            }
+#pragma unroll
+            for (int j = 0; j < kLongAhead; ++j) g[j] = x[c[j]];
+#pragma unroll
+            for (int j = 0; j < kLongAhead; ++j)
+                if (k + j * kLongLanes < e0) acc = __builtin_fma(static_cast<double>(a[j]), static_cast<double>(g[j]), acc);
+        }
         acc = group_sum<kLongLanes>(acc);
         if (lane == 0)
         {
@@ -1533,6 +1612,7 @@ struct Problem
     DiaLayout dia;           // diagonal layout of A for q = A p, when it pays
     DiaLayout dia_g, dia_gt; // ... of the factors G and G^T (both or neither)
     bool fuse_direction;     // on the diagonal layout: p_new formed inside the SpMV
+    bool fuse_lanes;         // long_rows: likewise
     bool fuse_step;          // factored: the step folded into G r and G^T t
     int fuse_step_env;       // PLAMATRIX_AMD_FUSE_STEP: 0 off, 1 on, -1 unset
     bool single_reduction;   // CG / Jacobi-PCG as the two-kernel Chronopoulos-Gear iteration
@@ -1854,13 +1934,20 @@ struct Calls
                                     static_cast<const S*>(p_old), static_cast<S*>(p_new), static_cast<S*>(pb.q),
                                     pb.st, pb.partials, par, count_res));
         }
+        else if (pb.long_rows && pb.fuse_lanes)
+        {
+            out.push_back(make_call(k_dir_spmv_lanes<S, I>, dim3(pb.grid_rows), dim3(kDirBlock), pb.a->rows, ro(pb.a),
+                                    ci(pb.a), static_cast<const S*>(pb.a->values), zsrc,
+                                    static_cast<const S*>(p_old), static_cast<S*>(p_new), static_cast<S*>(pb.q),
+                                    pb.st, pb.partials, par, count_res));
+        }
         else
         {
             out.push_back(make_call(k_direction<S>, dim3(pb.grid_units), dim3(kBlock), pb.a->rows, zsrc,
                                     static_cast<const S*>(p_old), static_cast<S*>(p_new), pb.st, pb.partials, par,
                                     count_res));
         }
-        if (pb.dia.active && pb.fuse_direction)
+        if ((pb.dia.active && pb.fuse_direction) || (pb.long_rows && pb.fuse_lanes))
         {
             // q and p.q came with the direction
         }
@@ -2024,9 +2111,11 @@ int prepare(pm_workspace* ws, Problem& pb, hipStream_t stream)
     pb.dma = dma != nullptr && dma[0] == '1';
     // fusing the direction into the diagonal-layout SpMV saves a pass over z
     // and p_old but measured slower (41.7 vs 40.6 us per 128^3 diffusion iteration): off
-    // unless PLAMATRIX_AMD_FUSE_DIRECTION=1
+    // unless PLAMATRIX_AMD_FUSE_DIRECTION=1.  The few long rows' SpMV gains from it
+    // (k_dir_spmv_lanes): on unless it is 0
     const char* fuse = std::getenv("PLAMATRIX_AMD_FUSE_DIRECTION");
     pb.fuse_direction = fuse != nullptr && fuse[0] == '1';
+    pb.fuse_lanes = fuse == nullptr || fuse[0] != '0';
     const char* fuse_step = std::getenv("PLAMATRIX_AMD_FUSE_STEP");
     pb.fuse_step_env = fuse_step == nullptr ? -1 : (fuse_step[0] == '0' ? 0 : 1);
     pb.fuse_step = fuse_step_wanted(pb);
@@ -2073,7 +2162,7 @@ std::string plan_key(const Problem& pb, const char* kind, int64_t first, int64_t
                   static_cast<long long>(pb.bsize),
                   (pb.nt ? 1 : 0) | (pb.dma ? 2 : 0) | (pb.fuse_direction ? 4 : 0) | (pb.fuse_step ? 8 : 0) |
                       (pb.single_reduction ? 16 : 0) | (pb.cg_fused ? 32 : 0) | (pb.cg_factored ? 64 : 0) |
-                      (pb.long_rows ? 128 : 0),
+                      (pb.long_rows ? 128 : 0) | (pb.fuse_lanes ? 256 : 0),
                   pb.dia.active ? 1 : 0, pb.dia.args.ndiag, dia_sig, pb.dia.values, static_cast<const void*>(pb.dia.mask),
                   pb.grid_rows, pb.grid_units);
     std::string key(buf);
