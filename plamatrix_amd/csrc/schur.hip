@@ -387,13 +387,16 @@ __global__ __launch_bounds__(kBlock) void k_ne_primary(int64_t pc, int rs_runtim
 }
 
 // B_p and g_p with one wavefront per primary (lane = entry, ps*ps + ps of
-// them, RS x PS Jacobians): the wavefront stages the Jacobian rows, residuals
-// and weights of kNeStage residuals into LDS with coalesced loads, then each
-// lane accumulates its entry over them in the primary's residual order, the
-// arithmetic of k_ne_primary.  With one wavefront per primary the kernel is
-// latency-bound (2,000 wavefronts on the LM system), so each round stages 64
-// residuals: 124 us with 16 per round, 213 us with 128.
+// them, RS x PS Jacobians): each lane stages the Jacobian rows, residual and
+// weight of one residual into LDS, then accumulates its entry over the 64 of them
+// in the primary's residual order, the arithmetic of k_ne_primary.  With one
+// wavefront per primary the kernel is latency-bound (2,000 wavefronts on the LM
+// system): the next round's values and the ids after them are in flight while a
+// round is added up, whose LDS reads go eight residuals ahead of the ordered adds.
+// 101 us with a lane per value and one round at a time; now 67, the cache lines of
+// the gathers.  (Rounds of 16 residuals measured 124 us, of 128 213.)
 constexpr int kNeStage = 64;
+constexpr int kNeUnroll = 8;
 template <int RS, int PS>
 __global__ __launch_bounds__(kBlock) void k_ne_primary_staged(int64_t pc, const int64_t* __restrict__ offs,
                                                               const unsigned* __restrict__ perm,
@@ -406,7 +409,7 @@ __global__ __launch_bounds__(kBlock) void k_ne_primary_staged(int64_t pc, const 
     static_assert(PS * PS + PS <= kWave, "one lane per entry");
     constexpr int kPer = RS * PS + RS + 1;  // J rows, residual, weight
     constexpr int kVals = kNeStage * kPer;
-    constexpr int kPerLane = (kVals + kWave - 1) / kWave;
+    static_assert(kNeStage == kWave, "a lane per staged residual");
     __shared__ double stage_all[kBlock / kWave][kVals];
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
@@ -414,56 +417,48 @@ __global__ __launch_bounds__(kBlock) void k_ne_primary_staged(int64_t pc, const 
     const bool active = lane < PS * PS + PS;
     const bool is_b = lane < PS * PS;
     const int column = is_b ? lane / PS : lane - PS * PS;
-    const int other = is_b ? lane % PS : 0;
+    // the second factor: a Jacobian entry, or the residual
+    const int second = is_b ? lane % PS : RS * PS, step = is_b ? PS : 1;
     const int64_t waves = static_cast<int64_t>(gridDim.x) * (kBlock / kWave);
     for (int64_t p = static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + wave; p < pc; p += waves)
     {
         const int64_t k0 = offs[p], k1 = offs[p + 1];
         double acc = 0.0;
+        unsigned id = 0;
+        double val[kPer];
+        auto load_ids = [&](int64_t k) { id = k + lane < k1 ? perm[k + lane] : 0u; };
+        auto load_values = [&](int64_t k) {
+            if (k + lane >= k1) return;
+            const int64_t i = id;
+#pragma unroll
+            for (int m = 0; m < RS * PS; ++m) val[m] = jp[i * RS * PS + m];
+#pragma unroll
+            for (int m = 0; m < RS; ++m) val[RS * PS + m] = r[i * RS + m];
+            val[RS * PS + RS] = w[i];
+        };
+        load_ids(k0);
+        load_values(k0);
+        load_ids(k0 + kNeStage);
         for (int64_t k = k0; k < k1; k += kNeStage)
         {
             const int nr = static_cast<int>(k1 - k < kNeStage ? k1 - k : kNeStage);
-            const int total = nr * kPer;
-            unsigned id[kPerLane];
 #pragma unroll
-            for (int m = 0; m < kPerLane; ++m)
-            {
-                const int f = lane + m * kWave;
-                id[m] = f < total ? perm[k + f / kPer] : 0u;
-            }
-            double val[kPerLane];
-#pragma unroll
-            for (int m = 0; m < kPerLane; ++m)
-            {
-                const int f = lane + m * kWave;
-                const int within = f % kPer;
-                const int64_t i = id[m];
-                val[m] = 0.0;
-                if (f < total)
-                    val[m] = within < RS * PS ? jp[i * RS * PS + within]
-                                              : (within < RS * PS + RS ? r[i * RS + (within - RS * PS)] : w[i]);
-            }
-#pragma unroll
-            for (int m = 0; m < kPerLane; ++m)
-            {
-                const int f = lane + m * kWave;
-                if (f < total) st[f] = val[m];
-            }
+            for (int m = 0; m < kPer; ++m) st[lane * kPer + m] = val[m];
             wave_lds_sync();
+            load_values(k + kNeStage);
+            load_ids(k + 2 * kNeStage);
             if (active)
             {
-                for (int u = 0; u < nr; ++u)
-                {
-                    const double* J = st + u * kPer;
-                    const double* res = J + RS * PS;
+                auto add = [&](const double* J) {
                     const double wi = J[RS * PS + RS];
 #pragma unroll
-                    for (int row = 0; row < RS; ++row)
-                    {
-                        const double value = J[row * PS + column];
-                        acc += wi * value * (is_b ? J[row * PS + other] : res[row]);
-                    }
-                }
+                    for (int row = 0; row < RS; ++row) acc += wi * J[row * PS + column] * J[second + row * step];
+                };
+                int u = 0;
+                for (; u + kNeUnroll <= nr; u += kNeUnroll)
+#pragma unroll
+                    for (int q = 0; q < kNeUnroll; ++q) add(st + (u + q) * kPer);
+                for (; u < nr; ++u) add(st + u * kPer);
             }
             wave_lds_sync();
         }
@@ -513,6 +508,7 @@ __global__ __launch_bounds__(kBlock) void k_ne_eliminated(int64_t ec, int rs, in
 // k_ne_eliminated with the sizes at compile time and one thread per
 // eliminated block: its residuals are loaded once for all ES * ES + ES
 // entries (each summed in the same order as above, so the same bits).
+constexpr int kNeAhead = 4;
 template <int RS, int ES>
 __global__ __launch_bounds__(kBlock) void k_ne_eliminated_points(int64_t ec, const int64_t* __restrict__ offs,
                                                                  const unsigned* __restrict__ perm,
@@ -527,25 +523,40 @@ __global__ __launch_bounds__(kBlock) void k_ne_eliminated_points(int64_t ec, con
         double acc[ES * ES + ES];
 #pragma unroll
         for (int en = 0; en < ES * ES + ES; ++en) acc[en] = 0.0;
-        for (int64_t k = offs[e]; k < offs[e + 1]; ++k)
+        const int64_t k1 = offs[e + 1];
+        for (int64_t k = offs[e]; k < k1; k += kNeAhead)
         {
-            const int64_t i = perm[k];
-            const double wi = w[i];
-            double J[RS * ES], res[RS];
+            // the loads of kNeAhead residuals are in flight together
+            unsigned id[kNeAhead];
+            double wi[kNeAhead], J[kNeAhead][RS * ES], res[kNeAhead][RS];
 #pragma unroll
-            for (int j = 0; j < RS * ES; ++j) J[j] = je[i * RS * ES + j];
+            for (int q = 0; q < kNeAhead; ++q) id[q] = perm[k + q < k1 ? k + q : k];
 #pragma unroll
-            for (int j = 0; j < RS; ++j) res[j] = r[i * RS + j];
-#pragma unroll
-            for (int column = 0; column < ES; ++column)
+            for (int q = 0; q < kNeAhead; ++q)
             {
+                const int64_t i = id[q];
+                wi[q] = w[i];
 #pragma unroll
-                for (int other = 0; other < ES; ++other)
+                for (int j = 0; j < RS * ES; ++j) J[q][j] = je[i * RS * ES + j];
+#pragma unroll
+                for (int j = 0; j < RS; ++j) res[q][j] = r[i * RS + j];
+            }
+#pragma unroll
+            for (int q = 0; q < kNeAhead; ++q)
+            {
+                if (k + q >= k1) break;
+#pragma unroll
+                for (int column = 0; column < ES; ++column)
+                {
+#pragma unroll
+                    for (int other = 0; other < ES; ++other)
+#pragma unroll
+                        for (int row = 0; row < RS; ++row)
+                            acc[column * ES + other] += wi[q] * J[q][row * ES + column] * J[q][row * ES + other];
 #pragma unroll
                     for (int row = 0; row < RS; ++row)
-                        acc[column * ES + other] += wi * J[row * ES + column] * J[row * ES + other];
-#pragma unroll
-                for (int row = 0; row < RS; ++row) acc[ES * ES + column] += wi * J[row * ES + column] * res[row];
+                        acc[ES * ES + column] += wi[q] * J[q][row * ES + column] * res[q][row];
+                }
             }
         }
 #pragma unroll
@@ -1031,29 +1042,45 @@ __global__ __launch_bounds__(kBlock) void k_invert_order(int64_t n, const unsign
 // rhs_p = -g_p + sum over the primary's cross blocks in (primary, eliminated)
 // order of W C^-1 g_e (block_schur.cpp:158-181), the products precomputed by
 // k_cross_rhs; the ordered sum loads kRhsBatch products ahead of the adds.
-constexpr int kRhsBatch = 64;  // one thread per rhs entry (pc * ps of them): deep prefetch for the few chains
+// A workgroup per primary: all its products come into LDS with coalesced loads in
+// flight together, and ps lanes add them in order.  (A thread per rhs entry kept 188
+// wavefronts waiting for batches of 64 gathers: 12.7 us for 60 primaries, 37 for
+// 2,000; now 5.5 and 33.)
+constexpr int kRhsStage = 4096;  // doubles
 __global__ __launch_bounds__(kBlock) void k_reduced_rhs(int64_t pc, int ps, const double* __restrict__ gp,
                                                         const int64_t* __restrict__ prim_offs,
                                                         const double* __restrict__ crv, double* __restrict__ rhs)
 {
 #pragma clang fp contract(off)
-    for (int64_t t = gtid(); t < pc * ps; t += gstride())
+    __shared__ double st[kRhsStage];
+    const int tid = threadIdx.x;
+    const int64_t batch = kRhsStage / ps;
+    for (int64_t p = blockIdx.x; p < pc; p += gridDim.x)
     {
-        const int64_t p = t / ps;
-        const int row = static_cast<int>(t % ps);
-        double acc = -gp[t];
+        double acc = tid < ps ? -gp[p * ps + tid] : 0.0;
         const int64_t k1 = prim_offs[p + 1];
-        for (int64_t k = prim_offs[p]; k < k1; k += kRhsBatch)
+        for (int64_t k = prim_offs[p]; k < k1; k += batch)
         {
-            double v[kRhsBatch];
+            const int terms = static_cast<int>(k1 - k < batch ? k1 - k : batch), n = terms * ps;
+            __syncthreads();
+#pragma unroll 4
+            for (int f = tid; f < n; f += kBlock) st[f] = crv[k * ps + f];
+            __syncthreads();
+            if (tid < ps)
+            {
+                int u = 0;
+                for (; u + 8 <= terms; u += 8)
+                {
+                    double v[8];
 #pragma unroll
-            for (int u = 0; u < kRhsBatch; ++u)
-                v[u] = k + u < k1 ? crv[(k + u) * ps + row] : 0.0;
+                    for (int j = 0; j < 8; ++j) v[j] = st[(u + j) * ps + tid];
 #pragma unroll
-            for (int u = 0; u < kRhsBatch; ++u)
-                if (k + u < k1) acc += 1.0 * v[u];
+                    for (int j = 0; j < 8; ++j) acc += 1.0 * v[j];
+                }
+                for (; u < terms; ++u) acc += 1.0 * st[u * ps + tid];
+            }
         }
-        rhs[t] = acc;
+        if (tid < ps) rhs[p * ps + tid] = acc;
     }
 }
 
@@ -1213,10 +1240,8 @@ __global__ __launch_bounds__(kBlock) void k_assemble_slots(
 // ---- segmented assembly ------------------------------------------------------------
 //
 // Each slot's terms are cut into segments of at most kSegTerms (in the slot's
-// eliminated order).  k_assemble_segments gives every segment one wavefront:
-// the segment's W C^-1 and W blocks are staged into LDS with all loads in
-// flight, and each lane (one entry of the 6 x 6 block) sums -(W_l C^-1) W_r^T
-// over the segment's terms in order.  k_assemble_reduce then forms each value
+// eliminated order).  k_assemble_segments sums -(W_l C^-1) W_r^T over each
+// segment's terms on the matrix cores, all its loads in flight.  k_assemble_reduce then forms each value
 // as damped B, the primary cross markers and the segment sums in segment
 // order.  The summation order is fixed (deterministic run to run) but groups
 // the terms by segment, so values differ from the CPU accumulation
@@ -1233,12 +1258,7 @@ __global__ __launch_bounds__(kBlock) void k_assemble_slots(
 // symmetric only to rounding).  S is then symmetric bit for bit, and each
 // value still differs from the CPU accumulation by rounding only.
 constexpr int kSegTerms = 16;
-// Segments a wavefront of k_assemble_segments sums.  One per wavefront, over
-// a grid of every segment, measured fastest on the 2,000-primary LM system:
-// 0.88 ms for the assembly against 0.90 with two and 0.94 with four (their
-// loads in flight together cost occupancy: 134 VGPRs at four), and 1.01 ms
-// for two segments per wavefront in sequence under a 65,536-workgroup grid.
-constexpr int kSegsPerWave = 1;
+constexpr int kSegsPerWave = 2;  // two 6 x 6 segments share a 16 x 16 tile
 
 // Per slot: the number of terms (the run minus its trailing markers) and of
 // segments (none below the block diagonal); seg_count[slots] = 0 closes the
@@ -1328,86 +1348,55 @@ __global__ __launch_bounds__(kBlock) void k_segment_terms(int64_t nseg, const un
     }
 }
 
+// A wavefront per two segments.  A segment is a 6 x 6 contraction of at most
+// 16 x 3 products, so both go through v_mfma_f64_16x16x4f64: segment h has rows and
+// columns 8 h .. 8 h + 5 of the tile (the blocks off the tile's diagonal are not
+// read), lane (i, k) feeds entry i % 8 of term (4 step + k) / 3, straight from
+// global memory.  Staging the blocks in LDS and adding per entry read six LDS
+// doubles per term and lane and was bound by them: 4.2
+// million terms of the 2,000-primary LM system 290 us, now 226, bound by the gathers
+// from L2.
 template <int ES, int PS>
 __global__ __launch_bounds__(kBlock) void k_assemble_segments(int64_t nseg, const uint2* __restrict__ seg_terms,
                                                               const double* __restrict__ TW,
                                                               const double* __restrict__ W,
                                                               double* __restrict__ partial)
 {
-#pragma clang fp contract(off)
-    constexpr int BV = PS * ES;              // doubles of one cross block
-    constexpr int PER = 2 * BV;              // W C^-1 block, then W block
-    constexpr int STAGE = kSegTerms * PER;
-    constexpr int LOADS = (STAGE + kWave - 1) / kWave;
-    constexpr int kWaves = kBlock / kWave;
-    constexpr int SEGS = kSegsPerWave;
-    __shared__ double stage_all[kWaves][STAGE];
-    const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
-    double* st = stage_all[wave];
-    const bool active = lane < PS * PS;
-    const int lr = active ? lane / PS : 0, lc = active ? lane % PS : 0;
-    // each wavefront owns SEGS consecutive segments and each workgroup a
-    // contiguous, XCD-local range: neighbouring segments share slots and
-    // blocks, which then stay in one L2.  The term pairs of all SEGS
-    // segments are loaded before the first block load; a segment's valid
-    // pairs are a prefix of its kSegTerms.
-    const int64_t g0 = (xcd_logical_block(blockIdx.x, gridDim.x) * kWaves + wave) * SEGS;
-    unsigned idl[SEGS], idr[SEGS];
+    static_assert(PS <= 8, "a segment's rows fit half the tile");
+    constexpr int BV = PS * ES;  // doubles of one cross block
+    constexpr int STEPS = kSegTerms * ES / 4;
+    static_assert(kSegTerms * ES % 4 == 0 && kSegTerms <= kWave / 2, "whole steps; the pairs sit in half a wavefront");
+    typedef double d4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int half = (lane % 16) / 8, row = lane % 8, k0 = lane / 16;
+    // each workgroup has a contiguous, XCD-local range: neighbouring segments
+    // share slots and blocks, which then stay in one L2.  A segment's valid pairs
+    // are a prefix of its kSegTerms.
+    const int64_t g0 = (xcd_logical_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + wave) * kSegsPerWave;
+    uint2 pair = make_uint2(kNoTerm, kNoTerm);
+    if (lane % (kWave / 2) < kSegTerms && g0 + lane / (kWave / 2) < nseg)
+        pair = seg_terms[(g0 + lane / (kWave / 2)) * kSegTerms + lane % (kWave / 2)];
+    double a[STEPS], b[STEPS];
 #pragma unroll
-    for (int q = 0; q < SEGS; ++q)
+    for (int s = 0; s < STEPS; ++s)
     {
-        uint2 pair = make_uint2(kNoTerm, kNoTerm);
-        if (lane < kSegTerms && g0 + q < nseg) pair = seg_terms[(g0 + q) * kSegTerms + lane];
-        idl[q] = pair.x;
-        idr[q] = pair.y;
+        const int k = 4 * s + k0, term = k / ES, within = row * ES + k % ES;
+        const unsigned l = __shfl(pair.x, half * (kWave / 2) + term, kWave);
+        const unsigned r = __shfl(pair.y, half * (kWave / 2) + term, kWave);
+        const bool in = row < PS && l != kNoTerm;
+        a[s] = in ? TW[static_cast<int64_t>(l) * BV + within] : 0.0;
+        b[s] = in ? W[static_cast<int64_t>(r) * BV + within] : 0.0;
     }
-    int nt[SEGS];
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int q = 0; q < SEGS; ++q) nt[q] = static_cast<int>(__popcll(__ballot(idl[q] != kNoTerm)));
-    double val[SEGS][LOADS];
+    for (int s = 0; s < STEPS; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
+    // lane l, value i: row l / 16 + 4 i, column l % 16
 #pragma unroll
-    for (int q = 0; q < SEGS; ++q)
+    for (int i = 0; i < 4; ++i)
     {
-#pragma unroll
-        for (int m = 0; m < LOADS; ++m)
-        {
-            const int f = lane + m * kWave;
-            const int u = f / PER, within = f % PER;
-            const unsigned a = __shfl(idl[q], u < kWave ? u : 0, kWave);
-            const unsigned b = __shfl(idr[q], u < kWave ? u : 0, kWave);
-            val[q][m] = 0.0;
-            if (f < STAGE && u < nt[q])
-                val[q][m] = within < BV ? TW[static_cast<int64_t>(a) * BV + within]
-                                        : W[static_cast<int64_t>(b) * BV + (within - BV)];
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < SEGS; ++q)
-    {
-        if (nt[q] == 0) break;  // wave-uniform: later segments are past the end too
-#pragma unroll
-        for (int m = 0; m < LOADS; ++m)
-        {
-            const int f = lane + m * kWave;
-            if (f < STAGE) st[f] = val[q][m];
-        }
-        wave_lds_sync();
-        if (active)
-        {
-            double acc = 0.0;
-            for (int u = 0; u < nt[q]; ++u)
-            {
-                const double* t = st + u * PER + lr * ES;
-                const double* w = st + u * PER + BV + lc * ES;
-                double value = 0.0;
-#pragma unroll
-                for (int i = 0; i < ES; ++i) value += t[i] * w[i];
-                acc += -value;
-            }
-            partial[(g0 + q) * (PS * PS) + lane] = acc;
-        }
-        wave_lds_sync();
+        const int r = k0 + 4 * i;
+        if (r / 8 == half && r % 8 < PS && row < PS && g0 + half < nseg)
+            partial[(g0 + half) * (PS * PS) + r % 8 * PS + row] = -acc[i];
     }
 }
 
@@ -1567,7 +1556,26 @@ __global__ __launch_bounds__(kBlock) void k_back_substitute_point(int64_t ec, in
 #pragma unroll
         for (int i = 0; i < es; ++i) point[i] = -ge[e * es + i];
         const int64_t k1 = adj_offs[e + 1];
-        for (int64_t k = adj_offs[e]; k < k1; ++k)
+        int64_t k = adj_offs[e];
+        if constexpr (N > 0)
+        {
+            // four blocks' products in flight together
+            constexpr int U = 4;
+            for (; k + U <= k1; k += U)
+            {
+                double v[U][N];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int column = 0; column < N; ++column)
+                        v[u][column] = t[static_cast<int64_t>(adj[k + u]) * N + column];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int column = 0; column < N; ++column) point[column] -= v[u][column];
+            }
+        }
+        for (; k < k1; ++k)
         {
             const double* tc = t + static_cast<int64_t>(adj[k]) * es;
 #pragma unroll
@@ -2435,7 +2443,7 @@ int schur_assemble(pm_schur_workspace* w, const pm_normal_equations* eq, double 
         else if (nc > 0)
             hipLaunchKernelGGL((k_cross_rhs<>), dim3(grid_for(nc * ps)), dim3(kBlock), 0, stream, nc, ps, es,
                                w->prim_cross, eq->cross_eliminated, eq->cross_values, w->y, w->crv);
-        hipLaunchKernelGGL(k_reduced_rhs, dim3(static_cast<unsigned>(ceil_div(pd, kWave))), dim3(kWave), 0, stream, pc,
+        hipLaunchKernelGGL(k_reduced_rhs, dim3(static_cast<unsigned>(std::min<int64_t>(pc, 65536))), dim3(kBlock), 0, stream, pc,
                            ps, eq->primary_gradient, w->prim_offs, static_cast<const double*>(w->crv), w->rhs);
         if (es == 3 && ps == 6 && segmented_assembly_wanted())
         {
