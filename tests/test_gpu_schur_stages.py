@@ -33,9 +33,9 @@ def counted(counts, ec, seed):
 
 
 # stages of 64 residuals per primary (8 at a time), 682 products of a primary's rhs,
-# 4 residuals and 4 back-substituted blocks per secondary, segments of 16 terms in pairs
+# 256 residuals of 64 secondaries, 4 back-substituted blocks, segments of 16 terms in pairs
 @pytest.mark.parametrize("counts,ec", [([1], 1), ([15, 1, 17], 40), ([63, 64, 65, 7, 8, 129], 130),
-                                       ([681, 682, 683, 690], 700), ([1, 1500, 31, 1366], 1500)])
+                                       ([681, 682, 683, 690], 700), ([1, 1500, 31, 1366], 1500), ([130] * 9, 130)])
 def test_stage_edges(dev, oracle, counts, ec):
     inst = counted(counts, ec, len(counts))
     sw, ws = capi.SchurWorkspace(), capi.Workspace()
