@@ -1,4 +1,7 @@
-// Device COO -> CSR for gfx950.
+// Device COO -> CSR for gfx950.  The synchronous conversion goes by row buckets
+// (coo_bucket.hip) where coo_plan allows; this file holds the entry points and the
+// LSD path: the asynchronous and captured conversion, wide keys, very long rows and
+// rows too uneven for the buckets.
 //
 //   1. pack     key = (row << cb) | col  (cb = bits of cols-1), payload = the
 //               triplet's position; out-of-range coordinates and (optionally)
@@ -149,6 +152,9 @@ __global__ void k_coo_status_init(CooStatus* st, long long expected)
     st->invalid_value = ~0ull;
     st->nnz = 0;
     st->expected_nnz = expected;
+    st->unsorted = 0;
+    st->most = 0;
+    st->ticket = 0;
 }
 
 __global__ void k_coo_status_init_expected(CooStatus* st, long long expected) { st->expected_nnz = expected; }
@@ -271,13 +277,21 @@ __global__ __launch_bounds__(kBlock) void k_positions(int64_t count, unsigned* _
         perm[i] = static_cast<unsigned>(i);
 }
 
-__global__ void k_publish_coo(const CooStatus* st, CooStatus* host) { *host = *st; }
+// A copy of the record that answers to no conversion's ticket.
+__device__ __forceinline__ void publish_coo(const CooStatus* st, CooStatus* host)
+{
+    CooStatus s = *st;
+    s.ticket = 0;
+    *host = s;
+}
+
+__global__ void k_publish_coo(const CooStatus* st, CooStatus* host) { publish_coo(st, host); }
 
 // The record goes straight into pinned host memory (`host` may be null).
 __global__ void k_store_nnz(const unsigned* total, CooStatus* st, CooStatus* host)
 {
     st->nnz = static_cast<long long>(*total);
-    if (host) *host = *st;
+    if (host) publish_coo(st, host);
 }
 
 template <typename S>
