@@ -53,7 +53,10 @@ def pcg_iteration_bytes(n: int, nnz: int, value_bytes: int = 4, index_bytes: int
                                                                (13 vectors)
     With a unit diagonal (every Jacobi inverse exactly 1) u is r: no M^-1
     read and no u write or second read (11, 12, 10 vectors).  Gathers of
-    neighbouring rows are counted once, with the row's own read."""
+    neighbouring rows are counted once, with the row's own read.  These are the
+    bytes of the per-kernel forms: a solve that runs in one launch keeps the
+    matrix and vectors on the CUs and moves the exchanged words only, so its
+    figure can pass what memory delivers."""
     vectors = {3: (13, 11), 2: (16, 12), 1: (13, 10)}[form][1 if unit_diagonal else 0]
     if diagonals:
         return (value_streams or diagonals) * n * value_bytes + 2 * n + vectors * n * value_bytes
@@ -476,7 +479,8 @@ def run_poisson(args, torch, capi, generators):
                       "traffic": None, "kernel": {1: "PCG iteration (k_cg_fused_dia)", 2: "PCG iteration (k_cg_step + k_cg_spmv)",
                                  3: "PCG iteration (k_direction + k_spmv_den + k_update)"}[form],
                       "bytes_per_launch": it_bytes, "ms_per_launch": round(it_ms, 5),
-                      "note": f"latency-bound: {it_bytes / 1e6:.1f} MB per iteration"},
+                      "note": f"latency-bound: {it_bytes / 1e6:.1f} MB per iteration in the per-kernel form; "
+                              "one launch per solve keeps them on the CUs"},
                      cpu)
     line["solve"] = {"converged": rep.converged, "iterations": rep.iterations, "true_relres": relres}
     line["coo_to_csr"] = {"ms_steady": round(conv_ms, 4), "ms_synchronous": round(sync_ms, 4),
@@ -697,8 +701,8 @@ def run_batch(args, torch, capi, generators):
                               shape=(ln, ln))
         bb = b_host[b0:b0 + ln]
         worst = max(worst, float(np.linalg.norm(bb - A @ xh[b0:b0 + ln]) / np.linalg.norm(bb)))
-    # algorithmic bytes actually streamed: each system's iteration traffic times
-    # its iterations (a block-Jacobi row also reads its 6-value inverse row)
+    # algorithmic bytes of the per-kernel form (systems held on the CUs move fewer):
+    # each system's iteration traffic times its iterations (a block-Jacobi row also reads its 6-value inverse row)
     streamed = sum((pcg_iteration_bytes(ln, z) + (6 * 4 * ln if bs > 1 else 0)) * int(it)
                    for ln, z, it, bs in zip(lens, nnzs, its, blocks))
     gbs = streamed / (ms * 1e-3) / 1e9

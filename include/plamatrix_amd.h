@@ -99,7 +99,9 @@ int32_t pm_workspace_solver_value_streams(const pm_workspace* ws);
  * diagonal layout (PLAMATRIX_AMD_CG_FUSED=0 keeps 2).  4: the factored
  * single-reduction iteration with A, G and G^T on the diagonal layout (step
  * and G r, G^T t, SpMV).  5: the same with a four-diagonal lower G, G r and
- * G^T t in one kernel (PLAMATRIX_AMD_CG_FUSED=0 keeps 4).  A solve whose
+ * G^T t in one kernel (PLAMATRIX_AMD_CG_FUSED=0 keeps 4).  Forms 1, 2, 4 and
+ * 5 may run a whole solve in one launch with the same bits
+ * (PLAMATRIX_AMD_PERSISTENT=0 keeps the kernels).  A solve whose
  * single-reduction denominator loses positivity continues in the classic
  * form. */
 int32_t pm_workspace_solver_form(const pm_workspace* ws);

@@ -33,9 +33,9 @@
 // host runs the solve in the per-kernel form instead.
 //
 // Measured, solve time per-kernel / persistent: 65,536-row FP64 2-D Laplacian
-// (767 iterations, one row per lane) 7.67 / 4.48 ms, 5.7 us per iteration, two
+// (767 iterations, one row per lane) 7.50 / 3.90 ms, 5.0 us per iteration, two
 // exchange latencies; 2,097,152-row FP32 3-D diffusion (753 iterations, eight
-// rows per lane) 20.4 / 15.4 ms, 18.6 us per iteration.
+// rows per lane) 21.2 / 15.2 ms with refinement, 18.6 us per iteration.
 #include "persist.hpp"
 
 #include <algorithm>
