@@ -18,11 +18,11 @@
 //              bucket's heads in LDS
 //
 // Measured, both calls together, LSD sort / here: 10,903 FP32 triplets of a 2,025-row
-// stencil 143 / 71 us (18 launches and two copies / 7 launches); 5.76 M FP64
+// stencil 143 / 65 us (18 launches and two copies / 7 launches); 5.76 M FP64
 // triplets of a million rows 898 / 382 us, of them fold 125, sort 93, partition 75,
 // pack 32.
 //
-// Up to kBucketCap triplets with at most 32 key bits are one bucket: no partition.
+// Up to kBucketOne triplets with at most 32 key bits are one bucket: no partition.
 // Equal keys keep their input order at every step, so the result is the LSD path's.
 #include "coo_bucket.hpp"
 
@@ -575,25 +575,33 @@ int allow_lds(K kernel, size_t bytes)
 } // namespace
 
 // Buckets of 2^shift rows, the most that keep the mean at kBucketMean and a local
-// key in 32 bits (and kBucketRowBits): uneven rows may then be 2.7 times the mean before a bucket
-// outgrows its workgroup (the conversion then pays the partition's counts and goes
-// on in the LSD sort).  Longer rows, wider keys and more than kBucketsMost
+// key in 32 bits (and kBucketRowBits): uneven rows may then be 2.7 times the mean
+// before a bucket outgrows its workgroup (the conversion then pays the partition's
+// counts and goes on in the LSD sort).  Longer rows, wider keys and more than kBucketsMost
 // buckets stay on the LSD sort.
+//
+// Smaller conversions are cut finer, towards a bucket per CU but not below
+// kBucketMeanLeast: the passes of a bucket are serial (10,939 triplets as 22 buckets
+// 65 us, as 4 70; 89,549 68 against 74; no difference from 400,000 on).  One bucket
+// without a partition is level with several at 4,200 to 5,000 triplets (4,189: 61.5
+// against 62.4 us; 5,491: 65.1 against 63.0).
 CooPlan coo_plan(int64_t rows, int64_t cols, int64_t count)
 {
     CooPlan p{};
     const int rb = bits_for(rows), cb = bits_for(cols);
     if (count <= 0 || rows <= 0 || cols <= 0 || cb > 32 || rows >= (int64_t(1) << 40)) return p;
     p.cb = cb;
-    if (count <= kBucketCap && rb <= kBucketRowBits && rb + cb <= 32)
+    if (count <= kBucketOne && rb <= kBucketRowBits && rb + cb <= 32)
     {
         p.buckets = 1;
         p.shift = rb;
         return p;
     }
     int shift = std::min({rb, 32 - cb, kBucketRowBits});
+    const double mean = static_cast<double>(
+        std::min<int64_t>(kBucketMean, std::max<int64_t>(kBucketMeanLeast, count / kBucketsWanted)));
     while (shift > 0 && static_cast<double>(count) * static_cast<double>(int64_t(1) << shift) >
-                            static_cast<double>(kBucketMean) * static_cast<double>(rows))
+                            mean * static_cast<double>(rows))
         --shift;
     if (static_cast<double>(count) * static_cast<double>(int64_t(1) << shift) >
         static_cast<double>(kBucketMean) * static_cast<double>(rows))

@@ -13,6 +13,9 @@ namespace pm
 
 constexpr int kBucketCap = 8192;      // triplets a bucket may hold
 constexpr int kBucketMean = 3072;     // triplets of an average bucket, at most
+constexpr int kBucketMeanLeast = 512; // ... that a smaller conversion is cut down to
+constexpr int kBucketsWanted = 256;   // buckets below which the mean shrinks: one per CU
+constexpr int kBucketOne = 4608;      // triplets of a conversion that stays one bucket, at most
 constexpr int kBucketsMost = 4096;
 constexpr int kBucketRowBits = 13;    // a bucket's workgroup also writes its rows' offsets
 

@@ -2235,8 +2235,8 @@ Policy resolve_policy(const pm_solve_policy* p, int64_t rows)
 // Whether a running solve that goes on at its mean rate (a quarter more iterations
 // allowed) stops within the iterations already issued; the chunk after them would
 // then only delay what follows the solve (a reduced system of an LM step stops
-// after 5 to 8 iterations, and eight more empty ones took 27 us of a 2,000-primary step's 996).  A wrong guess
-// costs one wait of the host.  The single-reduction forms keep their schedule: a
+// after 5 to 8 iterations, and eight more empty ones took 27 us of a 2,000-primary
+// step's 996).  A wrong guess costs one wait of the host.  The single-reduction forms keep their schedule: a
 // restart hands over at an iteration that follows from it.
 bool stops_within(const SolverState& st, int64_t issued)
 {

@@ -37,7 +37,7 @@ def triplets(rows, cols, count, kind, dtype, seed):
 
 CASES = [
     (1, 1, 1, "uniform"), (1, 1, 5000, "uniform"), (3, 2, 64, "uniform"), (40, 7, 65, "one"),
-    (8192, 8192, 1025, "uniform"), (8193, 8192, 3000, "uniform"), (500, 500, 8192, "stencil"),
+    (8192, 8192, 1025, "uniform"), (8193, 8192, 3000, "uniform"), (500, 500, 8192, "stencil"), (600, 600, 4608, "stencil"), (600, 600, 4609, "uniform"),
     (5000, 5000, 8193, "stencil"), (2025, 2025, 10900, "stencil"), (5000, 900, 40000, "sorted"),
     (70000, 70000, 262145, "stencil"), (300, 300, 300000, "uniform"), (100000, 100000, 50000, "uniform"),
     (3, 1 << 29, 9000, "uniform"), (3, 1 << 33, 9000, "uniform"), (20000, 20000, 100000, "arrow"),
