@@ -476,6 +476,7 @@ bool coo_capturing(hipStream_t stream)
 int resolve_coo(pm_workspace* ws, const CooStatus& s, hipStream_t stream)
 {
     ws->coo_resolved = true;
+    ws->coo_most = static_cast<int64_t>(s.most);
     if (!s.unsorted) return PM_OK;
     ws->coo_buckets = false;
     size_t bytes = 0;
@@ -618,7 +619,7 @@ int finish_coo(int64_t* row_offsets, int64_t* col_out, void* val_out, int64_t ex
     {
         const CooBuckets cut = coo_buckets(ws, plan, b);
         const int check = ws->coo_flags & PM_COO_CHECK_FINITE;
-        const int64_t most = static_cast<int64_t>(ws->host_coo->most);
+        const int64_t most = ws->coo_most;
         if (ws->coo_dtype == PM_F32)
             PM_TRY(coo_bucket_finish<float>(cut, static_cast<const float*>(ws->coo_values), check, expected, row_offsets,
                                             col_out, static_cast<float*>(val_out), most, stream));

@@ -1375,7 +1375,7 @@ __global__ __launch_bounds__(kBlock) void k_segment_terms(int64_t nseg, const un
 // columns 8 h .. 8 h + 5 of the tile (the blocks off the tile's diagonal are not
 // read), lane (i, k) feeds entry i % 8 of term (4 step + k) / 3, straight from
 // global memory.  Staging the blocks in LDS and adding per entry read six LDS
-// doubles per term and lane and was bound by them: 4.2
+// doubles per term and lane and was bound by them: 4.4
 // million terms of the 2,000-primary LM system 290 us, now 226, bound by the gathers
 // from L2.
 template <int ES, int PS>
