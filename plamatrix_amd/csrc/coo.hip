@@ -270,13 +270,6 @@ __global__ __launch_bounds__(kBlock) void k_mark_heads(const unsigned long long*
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_positions(int64_t count, unsigned* __restrict__ perm)
-{
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += stride)
-        perm[i] = static_cast<unsigned>(i);
-}
-
 // A copy of the record that answers to no conversion's ticket.
 __device__ __forceinline__ void publish_coo(const CooStatus* st, CooStatus* host)
 {
@@ -471,35 +464,44 @@ bool coo_capturing(hipStream_t stream)
     return status != hipStreamCaptureStatusNone;
 }
 
-// A conversion by buckets that was given up continues on the LSD sort, from the
-// packed keys.  `s`: its status record.
-int resolve_coo(pm_workspace* ws, const CooStatus& s, hipStream_t stream)
+// A conversion prepared by buckets becomes what the LSD path prepares: keys in order
+// with their positions, run ids, the nnz.  From the packed keys where the buckets
+// were given up, else from the sorted words (in order already, which the stable sort
+// keeps).
+int leave_buckets(pm_workspace* ws, hipStream_t stream)
 {
-    ws->coo_resolved = true;
-    ws->coo_most = static_cast<int64_t>(s.most);
-    if (!s.unsorted) return PM_OK;
-    ws->coo_buckets = false;
+    const CooPlan plan = coo_plan(ws->coo_rows, ws->coo_cols, ws->coo_count);
     size_t bytes = 0;
-    const CooBuffers b = coo_layout(ws, ws->coo_count, 0, &bytes);
-    auto sort = [&](hipStream_t on) -> int {
-        const int grid = static_cast<int>(std::min<int64_t>(ceil_div(ws->coo_count, kBlock), 8192));
-        hipLaunchKernelGGL(k_positions, dim3(grid), dim3(kBlock), 0, on, ws->coo_count, b.vals_a);
-        PM_HIP(hipGetLastError());
-        return sort_coo(b, ws->coo_count, bits_for(ws->coo_rows), bits_for(ws->coo_cols), ws, on);
-    };
-    if (!coo_capturing(stream)) return sort(stream);
-    // prepared eagerly, finished in a capture: the sort stays out of the graph,
-    // which reads its result on every replay
+    const CooBuffers b = coo_layout(ws, ws->coo_count, coo_bucket_bytes(plan), &bytes);
+    ws->coo_buckets = false;
+    PM_TRY(coo_bucket_unpack(coo_buckets(ws, plan, b), b.vals_a, stream));
+    return sort_coo(b, ws->coo_count, bits_for(ws->coo_rows), bits_for(ws->coo_cols), ws, stream);
+}
+
+// The same while the caller's stream is being captured: it stays out of the graph,
+// which reads its result on every replay.  What was prepared has ended (await_coo).
+int leave_buckets_in_capture(pm_workspace* ws)
+{
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     PM_HIP(hipThreadExchangeStreamCaptureMode(&mode));
     const int status = [&]() -> int {
         PM_TRY(ws->ensure_aux());
-        PM_TRY(sort(ws->aux_stream));
+        PM_TRY(leave_buckets(ws, ws->aux_stream));
         PM_HIP(hipStreamSynchronize(ws->aux_stream));
         return PM_OK;
     }();
     PM_HIP(hipThreadExchangeStreamCaptureMode(&mode));
     return status;
+}
+
+// A conversion by buckets that was given up continues on the LSD sort.  `s`: its
+// status record.
+int resolve_coo(pm_workspace* ws, const CooStatus& s, hipStream_t stream)
+{
+    ws->coo_resolved = true;
+    ws->coo_most = static_cast<int64_t>(s.most);
+    if (!s.unsorted) return PM_OK;
+    return coo_capturing(stream) ? leave_buckets_in_capture(ws) : leave_buckets(ws, stream);
 }
 
 int prepare_coo(int64_t rows, int64_t cols, int64_t count, const int64_t* r, const int64_t* c, const void* v,
@@ -518,8 +520,10 @@ int prepare_coo(int64_t rows, int64_t cols, int64_t count, const int64_t* r, con
     if (ws->coo_pending_status)
         return fail(PM_LOGIC_ERROR, "workspace status must be checked before another COO conversion");
     // by buckets where the caller reads the nnz before it finishes: that read also
-    // tells whether a bucket outgrew its workgroup
-    const CooPlan plan = may_wait && !coo_capturing(stream) ? coo_plan(rows, cols, count) : CooPlan{};
+    // tells whether a bucket outgrew its workgroup.  A graph that holds a finish of
+    // this workspace reads what the LSD sort leaves, whatever is prepared for it
+    const bool buckets = may_wait && !ws->coo_in_graph && !coo_capturing(stream);
+    const CooPlan plan = buckets ? coo_plan(rows, cols, count) : CooPlan{};
     size_t bytes = 0;
     coo_layout(nullptr, count, coo_bucket_bytes(plan), &bytes);
     PM_TRY(ws->sort.reserve(bytes));
@@ -611,6 +615,13 @@ int finish_coo(int64_t* row_offsets, int64_t* col_out, void* val_out, int64_t ex
         CooStatus s{};
         PM_TRY(await_coo(ws, stream, &s));
         PM_TRY(resolve_coo(ws, s, stream));
+    }
+    if (coo_capturing(stream))
+    {
+        // the buckets' fold is launched for the sizes of this conversion's buckets; a
+        // replay may meet another one
+        ws->coo_in_graph = true;
+        if (ws->coo_buckets) PM_TRY(leave_buckets_in_capture(ws));
     }
     const CooPlan plan = ws->coo_buckets ? coo_plan(ws->coo_rows, ws->coo_cols, count) : CooPlan{};
     size_t bytes = 0;

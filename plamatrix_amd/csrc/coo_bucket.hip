@@ -564,6 +564,27 @@ __global__ __launch_bounds__(kThreads) void k_bucket_fold(CooBuckets b, Tables t
     if (blockIdx.x == 0) b.status->expected_nnz = capacity;
 }
 
+__global__ __launch_bounds__(kThreads) void k_bucket_unpack(CooBuckets b, Tables t, unsigned* __restrict__ positions)
+{
+    if (b.plan.tiles == 0 || b.status->unsorted)
+    {
+        for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < b.count;
+             i += static_cast<int64_t>(gridDim.x) * kThreads)
+            positions[i] = static_cast<unsigned>(i);
+        return;
+    }
+    for (int d = blockIdx.x; d < b.plan.buckets; d += gridDim.x)
+    {
+        const u64 high = static_cast<u64>(d) << (b.plan.cb + b.plan.shift);
+        for (int64_t i = t.base[d] + threadIdx.x; i < t.base[d + 1]; i += kThreads)
+        {
+            const u64 word = b.keys[i];
+            b.keys[i] = high | (word >> 32);
+            positions[i] = static_cast<unsigned>(word);
+        }
+    }
+}
+
 template <typename K>
 int allow_lds(K kernel, size_t bytes)
 {
@@ -659,6 +680,14 @@ int coo_bucket_finish(const CooBuckets& b, const S* v, int check_finite, int64_t
     PM_TRY(allow_lds(fold, lds));
     hipLaunchKernelGGL(fold, dim3(b.plan.buckets), dim3(kThreads), lds, stream, b, tables(b),
                        b.plan.tiles == 0 ? b.words : b.keys, v, check_finite, capacity, row_offsets, cols, vals, room);
+    PM_HIP(hipGetLastError());
+    return PM_OK;
+}
+
+int coo_bucket_unpack(const CooBuckets& b, unsigned* positions, hipStream_t stream)
+{
+    const int64_t grid = std::max<int64_t>(b.plan.buckets, std::min<int64_t>(ceil_div(b.count, kThreads), 2048));
+    hipLaunchKernelGGL(k_bucket_unpack, dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, stream, b, tables(b), positions);
     PM_HIP(hipGetLastError());
     return PM_OK;
 }

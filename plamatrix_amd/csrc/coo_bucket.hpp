@@ -30,7 +30,7 @@ struct CooPlan
 };
 CooPlan coo_plan(int64_t rows, int64_t cols, int64_t count);
 
-// Bytes behind CooBucketArgs::hist.
+// Bytes behind CooBuckets::tables.
 size_t coo_bucket_bytes(const CooPlan& plan);
 
 struct CooBuckets
@@ -54,5 +54,9 @@ int coo_bucket_prepare(const CooBuckets& b, const int64_t* r, const int64_t* c, 
 template <typename S>
 int coo_bucket_finish(const CooBuckets& b, const S* v, int check_finite, int64_t capacity, int64_t* row_offsets,
                       int64_t* cols, S* vals, int64_t most, hipStream_t stream);
+
+// What the LSD sort starts from, in `keys` and `positions`: the packed keys and their
+// positions in order where the record says unsorted, else the sorted ones.
+int coo_bucket_unpack(const CooBuckets& b, unsigned* positions, hipStream_t stream);
 
 } // namespace pm

@@ -122,3 +122,59 @@ def test_finish_without_reading_the_nnz(dev, kind, capture):
     else:
         assert torch.equal(got[0], want.row_offsets) and torch.equal(got[1], want.col_indices)
         assert torch.equal(got[2], want.values)
+
+
+def distinct(rows, count, kind, seed):
+    """Triplets of distinct places: as many of any kind have the same nnz.  "even":
+    buckets alike; "uneven": one of several times the mean; "over": one that outgrows
+    its workgroup."""
+    rng = np.random.default_rng(seed)
+    heavy = {"even": 0, "uneven": 3000, "over": 20000}[kind]
+    low = rng.permutation(128 * rows)[:heavy]
+    rest = 128 * rows + rng.permutation((rows - 128) * 64)[:count - heavy] * (rows // 64)
+    key = np.concatenate([low, rest])[rng.permutation(count)]
+    return key // rows, key % rows, rng.standard_normal(count)
+
+
+@pytest.mark.parametrize("read_nnz", [False, True])
+def test_replayed_finish_meets_new_triplets(dev, read_nnz):
+    """A captured finish folds whatever was prepared before its replay."""
+    rows, count = 20000, 60000
+    sets = {kind: [torch.from_numpy(t).to(dev) for t in distinct(rows, count, kind, seed)]
+            for seed, kind in enumerate(("even", "uneven", "over"))}
+    want = {kind: capi.coo_to_csr(rows, rows, *t, capi.Workspace()) for kind, t in sets.items()}
+    ws = capi.Workspace()
+    r, c, v = (t.clone() for t in sets["even"])
+    ro = torch.zeros(rows + 1, dtype=torch.int64, device=dev)
+    ci, vals = torch.zeros_like(c), torch.zeros_like(v)
+    i64, p = ctypes.c_int64, lambda t: ctypes.c_void_p(t.data_ptr())
+
+    def prepare(kind):
+        for to, t in zip((r, c, v), sets[kind]):
+            to.copy_(t)
+        capi.check(capi.lib().pm_coo_to_csr_prepare(i64(rows), i64(rows), i64(count), p(r), p(c), p(v),
+                                                    ctypes.c_int32(capi.dtype_code(v)), ctypes.c_int32(0), ws.handle,
+                                                    capi.current_stream()))
+        if read_nnz:
+            nnz = i64()
+            capi.check(capi.lib().pm_coo_to_csr_nnz(ws.handle, ctypes.byref(nnz)))
+            assert nnz.value == count
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        prepare("even")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        capi.check(capi.lib().pm_coo_to_csr_finish(p(ro), p(ci), p(vals), i64(count), ws.handle, capi.current_stream()))
+    with torch.cuda.stream(side):
+        for k, kind in enumerate(("even", "uneven", "over", "even")):
+            if k > 0:
+                prepare(kind)
+            for t in (ro, ci, vals):
+                t.zero_()
+            graph.replay()
+            side.synchronize()
+            ws.check_status()
+            assert torch.equal(ro, want[kind].row_offsets) and torch.equal(ci, want[kind].col_indices), kind
+            assert torch.equal(vals, want[kind].values), kind
