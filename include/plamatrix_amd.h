@@ -140,7 +140,10 @@ int pm_coo_to_csr_prepare(int64_t rows, int64_t cols, int64_t count, const int64
  * the deferred coordinate / value errors (lowest triplet position first). */
 int pm_coo_to_csr_nnz(pm_workspace* ws, int64_t* nnz);
 /* Fold duplicates and write CSR arrays of exactly expected_nnz entries
- * (asynchronous; a mismatch is reported by pm_workspace_check_status). */
+ * (asynchronous; a mismatch is reported by pm_workspace_check_status).  In a
+ * stream capture the call also waits for a conversion prepared before it.  A
+ * workspace whose finish was captured, or called before pm_coo_to_csr_nnz,
+ * prepares by the global sort from then on, which needs no read of the nnz. */
 int pm_coo_to_csr_finish(int64_t* row_offsets, int64_t* col_indices, void* values, int64_t expected_nnz,
                          pm_workspace* ws, hipStream_t stream);
 /* prepare + finish in one asynchronous call (cooToCsrAsync). */

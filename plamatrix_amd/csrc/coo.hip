@@ -522,7 +522,7 @@ int prepare_coo(int64_t rows, int64_t cols, int64_t count, const int64_t* r, con
     // by buckets where the caller reads the nnz before it finishes: that read also
     // tells whether a bucket outgrew its workgroup.  A graph that holds a finish of
     // this workspace reads what the LSD sort leaves, whatever is prepared for it
-    const bool buckets = may_wait && !ws->coo_in_graph && !coo_capturing(stream);
+    const bool buckets = may_wait && !ws->coo_lsd && !coo_capturing(stream);
     const CooPlan plan = buckets ? coo_plan(rows, cols, count) : CooPlan{};
     size_t bytes = 0;
     coo_layout(nullptr, count, coo_bucket_bytes(plan), &bytes);
@@ -610,19 +610,27 @@ int finish_coo(int64_t* row_offsets, int64_t* col_out, void* val_out, int64_t ex
     if (!row_offsets || (expected > 0 && (!col_out || !val_out)))
         return fail(PM_INVALID_ARGUMENT, "cooToCsr: null output arrays");
     const int64_t count = ws->coo_count;
-    if (!ws->coo_resolved)
-    {
-        CooStatus s{};
-        PM_TRY(await_coo(ws, stream, &s));
-        PM_TRY(resolve_coo(ws, s, stream));
-    }
     if (coo_capturing(stream))
     {
         // the buckets' fold is launched for the sizes of this conversion's buckets; a
         // replay may meet another one
-        ws->coo_in_graph = true;
-        if (ws->coo_buckets) PM_TRY(leave_buckets_in_capture(ws));
+        ws->coo_lsd = true;
+        if (ws->coo_buckets)
+        {
+            CooStatus s{};
+            if (!ws->coo_resolved) PM_TRY(await_coo(ws, stream, &s));
+            PM_TRY(leave_buckets_in_capture(ws));
+        }
     }
+    else if (!ws->coo_resolved)
+    {
+        // nobody knows whether the buckets held: the LSD sort needs no word from the
+        // device, so the call stays stream-ordered.  A caller that knows its nnz now
+        // will know the next one too
+        ws->coo_lsd = true;
+        PM_TRY(leave_buckets(ws, stream));
+    }
+    ws->coo_resolved = true;
     const CooPlan plan = ws->coo_buckets ? coo_plan(ws->coo_rows, ws->coo_cols, count) : CooPlan{};
     size_t bytes = 0;
     CooBuffers b = coo_layout(ws, count, coo_bucket_bytes(plan), &bytes);

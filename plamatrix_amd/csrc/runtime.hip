@@ -247,7 +247,7 @@ int pm_workspace_close(pm_workspace* ws)
     ws->bound = false;
     ws->stream = nullptr;
     ws->coo_prepared = false;
-    ws->coo_in_graph = false;
+    ws->coo_lsd = false;
     return PM_OK;
 }
 

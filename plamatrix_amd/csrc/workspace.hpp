@@ -157,7 +157,7 @@ struct pm_workspace
     bool coo_buckets = false;               // by buckets (coo_bucket.hpp)
     bool coo_resolved = false;              // ... and known to have been sorted
     int64_t coo_most = 0;                   // ... triplets of its largest bucket
-    bool coo_in_graph = false;              // a finish was captured: every conversion by the LSD sort
+    bool coo_lsd = false;                   // every conversion by the LSD sort: a finish was captured, or ran before its nnz was read
     bool coo_publish = false;               // kernels leave the status record in host_coo (prepare / nnz / finish)
     unsigned long long coo_ticket = 0;
     bool coo_pending_status = false;

@@ -178,3 +178,33 @@ def test_replayed_finish_meets_new_triplets(dev, read_nnz):
             ws.check_status()
             assert torch.equal(ro, want[kind].row_offsets) and torch.equal(ci, want[kind].col_indices), kind
             assert torch.equal(vals, want[kind].values), kind
+
+
+@pytest.mark.parametrize("kind", ["stencil", "arrow"])
+def test_finish_does_not_wait(dev, kind):
+    """Without a read of the nnz, prepare and finish are stream-ordered: both return
+    while the stream is still busy with what came before them."""
+    rows, count = 20000, 100000
+    r, c, v = (torch.from_numpy(t).to(dev) for t in triplets(rows, rows, count, kind, np.float64, 8))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    i64, p = ctypes.c_int64, lambda t: ctypes.c_void_p(t.data_ptr())
+    with torch.cuda.stream(side):
+        ws = capi.Workspace()
+        want = capi.coo_to_csr(rows, rows, r, c, v, ws)  # the storage is in place
+        got = [torch.zeros_like(t) for t in (want.row_offsets, want.col_indices, want.values)]
+        side.synchronize()
+        for _ in range(2):  # by buckets first, then by the sort
+            for t in got:
+                t.zero_()
+            torch.cuda._sleep(100_000_000)
+            capi.check(capi.lib().pm_coo_to_csr_prepare(i64(rows), i64(rows), i64(count), p(r), p(c), p(v),
+                                                        ctypes.c_int32(capi.dtype_code(v)), ctypes.c_int32(0), ws.handle,
+                                                        capi.current_stream()))
+            capi.check(capi.lib().pm_coo_to_csr_finish(p(got[0]), p(got[1]), p(got[2]), i64(want.nnz), ws.handle,
+                                                       capi.current_stream()))
+            assert not side.query()
+            side.synchronize()
+            ws.check_status()
+            assert torch.equal(got[0], want.row_offsets) and torch.equal(got[1], want.col_indices)
+            assert torch.equal(got[2], want.values)
