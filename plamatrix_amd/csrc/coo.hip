@@ -390,10 +390,9 @@ struct CooBuffers
     unsigned* scratch;
     unsigned* total;
     CooStatus* status;
-    char* tables;
 };
 
-CooBuffers coo_layout(pm_workspace* ws, int64_t count, size_t table_bytes, size_t* bytes_out)
+CooBuffers coo_layout(pm_workspace* ws, int64_t count, size_t* bytes_out)
 {
     auto align = [](size_t b) { return (b + 255) & ~size_t(255); };
     const int64_t tiles = ceil_div(count > 0 ? count : 1, kSortTile);
@@ -410,7 +409,6 @@ CooBuffers coo_layout(pm_workspace* ws, int64_t count, size_t table_bytes, size_
     size_t o_scr = off; off += align(sizeof(unsigned) * scan_scratch_words(big));
     size_t o_total = off; off += 256;
     size_t o_status = off; off += 256;
-    size_t o_tables = off; off += align(table_bytes);
     *bytes_out = off;
     CooBuffers b{};
     if (!ws) return b;
@@ -425,13 +423,13 @@ CooBuffers coo_layout(pm_workspace* ws, int64_t count, size_t table_bytes, size_
     b.scratch = reinterpret_cast<unsigned*>(base + o_scr);
     b.total = reinterpret_cast<unsigned*>(base + o_total);
     b.status = reinterpret_cast<CooStatus*>(base + o_status);
-    b.tables = base + o_tables;
     return b;
 }
 
 CooBuckets coo_buckets(const pm_workspace* ws, const CooPlan& plan, const CooBuffers& b)
 {
-    return CooBuckets{plan, ws->coo_rows, ws->coo_cols, ws->coo_count, b.keys_a, b.keys_b, b.tables, b.status};
+    return CooBuckets{plan, ws->coo_rows, ws->coo_cols, ws->coo_count, b.keys_a, b.keys_b,
+                      ws->coo_tables.as<char>(), b.status};
 }
 
 // The LSD sort of packed keys and what follows it.
@@ -472,7 +470,7 @@ int leave_buckets(pm_workspace* ws, hipStream_t stream)
 {
     const CooPlan plan = coo_plan(ws->coo_rows, ws->coo_cols, ws->coo_count);
     size_t bytes = 0;
-    const CooBuffers b = coo_layout(ws, ws->coo_count, coo_bucket_bytes(plan), &bytes);
+    const CooBuffers b = coo_layout(ws, ws->coo_count, &bytes);
     ws->coo_buckets = false;
     PM_TRY(coo_bucket_unpack(coo_buckets(ws, plan, b), b.vals_a, stream));
     return sort_coo(b, ws->coo_count, bits_for(ws->coo_rows), bits_for(ws->coo_cols), ws, stream);
@@ -525,9 +523,10 @@ int prepare_coo(int64_t rows, int64_t cols, int64_t count, const int64_t* r, con
     const bool buckets = may_wait && !ws->coo_lsd && !coo_capturing(stream);
     const CooPlan plan = buckets ? coo_plan(rows, cols, count) : CooPlan{};
     size_t bytes = 0;
-    coo_layout(nullptr, count, coo_bucket_bytes(plan), &bytes);
+    coo_layout(nullptr, count, &bytes);
     PM_TRY(ws->sort.reserve(bytes));
-    CooBuffers b = coo_layout(ws, count, coo_bucket_bytes(plan), &bytes);
+    PM_TRY(ws->coo_tables.reserve(coo_bucket_bytes(plan)));
+    CooBuffers b = coo_layout(ws, count, &bytes);
     ws->coo_rows = rows;
     ws->coo_cols = cols;
     ws->coo_count = count;
@@ -633,7 +632,7 @@ int finish_coo(int64_t* row_offsets, int64_t* col_out, void* val_out, int64_t ex
     ws->coo_resolved = true;
     const CooPlan plan = ws->coo_buckets ? coo_plan(ws->coo_rows, ws->coo_cols, count) : CooPlan{};
     size_t bytes = 0;
-    CooBuffers b = coo_layout(ws, count, coo_bucket_bytes(plan), &bytes);
+    CooBuffers b = coo_layout(ws, count, &bytes);
     if (ws->coo_buckets)
     {
         const CooBuckets cut = coo_buckets(ws, plan, b);
@@ -750,7 +749,7 @@ int pm_workspace_check_status(pm_workspace* ws)
     if (!ws->coo_publish)
     {
         size_t bytes = 0;
-        CooBuffers b = coo_layout(ws, ws->coo_count, 0, &bytes);
+        CooBuffers b = coo_layout(ws, ws->coo_count, &bytes);
         PM_HIP(hipMemcpy(ws->host_coo, b.status, sizeof(CooStatus), hipMemcpyDeviceToHost));
     }
     ws->coo_pending_status = false;

@@ -167,6 +167,7 @@ pm_workspace::~pm_workspace()
     state.release();
     scratch.release();
     sort.release();
+    coo_tables.release();
     refine.release();
     batch.release();
     dense.release();
@@ -234,6 +235,7 @@ int pm_workspace_close(pm_workspace* ws)
     ws->state.release();
     ws->scratch.release();
     ws->sort.release();
+    ws->coo_tables.release();
     ws->refine.release();
     ws->batch.release();
     ws->dense.release();
@@ -255,6 +257,7 @@ size_t pm_workspace_capacity_bytes(const pm_workspace* ws)
 {
     if (!ws) return 0;
     return ws->vectors.bytes + ws->partials.bytes + ws->state.bytes + ws->scratch.bytes + ws->sort.bytes +
+           ws->coo_tables.bytes +
            ws->refine.bytes + ws->batch.bytes + ws->dense.bytes +
            ws->dia.bytes + ws->dia_g.bytes + ws->dia_gt.bytes + ws->blocks.bytes + ws->persist.bytes + ws->teams.bytes;
 }

@@ -125,6 +125,7 @@ struct pm_workspace
     pm::DeviceBuffer batch;     // batched solver: layout, per-system state, per-chunk partials
     pm::DeviceBuffer blocks;    // batched solver: per-system block sizes and block-Jacobi inverse rows
     pm::DeviceBuffer dense;     // dense Cholesky: n x n lower triangle, diagonal-block inverses
+    pm::DeviceBuffer coo_tables; // COO conversion by buckets: beside `sort`, whose size graphs of the other path rely on
     pm::DeviceBuffer dia;       // diagonal layout of the solver's matrix
     pm::DeviceBuffer dia_g;     // ... of the factored preconditioner's G
     pm::DeviceBuffer dia_gt;    // ... and of G^T

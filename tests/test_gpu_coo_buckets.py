@@ -208,3 +208,35 @@ def test_finish_does_not_wait(dev, kind):
             ws.check_status()
             assert torch.equal(got[0], want.row_offsets) and torch.equal(got[1], want.col_indices)
             assert torch.equal(got[2], want.values)
+
+
+def test_buckets_leave_a_captured_conversion_alone(dev):
+    """A captured asynchronous conversion keeps its storage when the workspace then
+    converts by buckets, with more tables than the slack of that storage."""
+    rows, count = 5_000_000, 1000
+    r, c, v = (torch.from_numpy(t).to(dev) for t in triplets(rows, 50, count, "uniform", np.float64, 4))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = capi.coo_to_csr(rows, 50, r, c, v, capi.Workspace())
+        out = capi.DeviceCSR(rows, 50, torch.empty_like(want.row_offsets), torch.empty_like(want.col_indices),
+                             torch.empty_like(want.values))
+        ws = capi.Workspace()
+        capi.coo_to_csr_async(rows, 50, r, c, v, out, ws)
+        side.synchronize()
+        ws.check_status()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        capi.coo_to_csr_async(rows, 50, r, c, v, out, ws)
+    with torch.cuda.stream(side):
+        graph.replay()
+        side.synchronize()
+        ws.check_status()
+        for _ in range(3):
+            capi.coo_to_csr(rows, 50, r, c, v, ws)
+            for t in (out.row_offsets, out.col_indices, out.values):
+                t.zero_()
+            graph.replay()
+            side.synchronize()
+            assert torch.equal(out.row_offsets, want.row_offsets) and torch.equal(out.values, want.values)
+            assert torch.equal(out.col_indices, want.col_indices)
