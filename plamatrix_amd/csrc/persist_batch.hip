@@ -531,8 +531,8 @@ int batch_teams_look(pm_workspace* ws, const BatchTeams& b, std::vector<BatchLoo
 {
     look.assign(static_cast<size_t>(b.systems), BatchLook{0, 0});
     if (b.systems == 0 || b.chunks == 0 || !persist_enabled()) return PM_OK;
-    PM_TRY(ws->scratch.reserve(sizeof(BatchLook) * static_cast<size_t>(b.systems)));
-    auto* dev = ws->scratch.as<BatchLook>();
+    PM_TRY(ws->looks.reserve(sizeof(BatchLook) * static_cast<size_t>(b.systems)));
+    auto* dev = ws->looks.as<BatchLook>();
     hipLaunchKernelGGL(k_look_reset, dim3(1), dim3(kBlock), 0, stream, b.systems, dev);
     const dim3 grid(static_cast<unsigned>(ceil_div(b.chunks, kBlock / kWave)));
     if (use_compact(b.a))

@@ -177,6 +177,7 @@ pm_workspace::~pm_workspace()
     blocks.release();
     persist.release();
     teams.release();
+    looks.release();
     for (hipEvent_t& e : events)
         if (e) (void)hipEventDestroy(e);
     if (done_event) (void)hipEventDestroy(done_event);
@@ -245,6 +246,7 @@ int pm_workspace_close(pm_workspace* ws)
     ws->blocks.release();
     ws->persist.release();
     ws->teams.release();
+    ws->looks.release();
     ws->capacity_rows = 0;
     ws->bound = false;
     ws->stream = nullptr;
@@ -259,7 +261,8 @@ size_t pm_workspace_capacity_bytes(const pm_workspace* ws)
     return ws->vectors.bytes + ws->partials.bytes + ws->state.bytes + ws->scratch.bytes + ws->sort.bytes +
            ws->coo_tables.bytes +
            ws->refine.bytes + ws->batch.bytes + ws->dense.bytes +
-           ws->dia.bytes + ws->dia_g.bytes + ws->dia_gt.bytes + ws->blocks.bytes + ws->persist.bytes + ws->teams.bytes;
+           ws->dia.bytes + ws->dia_g.bytes + ws->dia_gt.bytes + ws->blocks.bytes + ws->persist.bytes + ws->teams.bytes +
+           ws->looks.bytes;
 }
 
 int64_t pm_workspace_capacity_rows(const pm_workspace* ws) { return ws ? ws->capacity_rows : 0; }

@@ -133,6 +133,7 @@ struct pm_workspace
     uint32_t persist_tag = 0;   // last exchange tag used in it
     bool cooperative_refused = false; // the runtime turned a cooperative launch down (another process has the queue)
     pm::DeviceBuffer teams;     // persistent batch: exchange words and control blocks
+    pm::DeviceBuffer looks;     // ... what it saw of each system's rows (scratch belongs to graphs that hold an SpMM)
     size_t teams_words = 0;     // words before its control blocks
     uint32_t teams_tag = 0;     // last exchange tag used in it
     int32_t last_diagonals = 0; // diagonals of the last solve's layout (0: CSR kernels)

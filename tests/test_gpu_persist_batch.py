@@ -117,3 +117,32 @@ def test_stops_before_the_launch(dev, monkeypatch):
             assert not bool(x[int(begin[1]):int(end[1])].any()) and not bool(x[int(begin[2]):int(end[2])].any())
         assert out["0"] == out["1"]
         assert out["1"][1][1] == 6 and out["1"][1][2] == row and out["1"][2][0]
+
+
+def test_a_captured_product_keeps_its_storage(dev):
+    # a graph holds an SpMM of this workspace, whose packed columns are smaller than
+    # what the batch notes of its 512 systems
+    small = capi.to_device_csr(diag_system(12), compact=True)
+    y, z = (torch.zeros((3, 12), dtype=torch.float64, device=dev) for _ in range(2))
+    v = torch.from_numpy(np.random.default_rng(1).standard_normal((3, 12))).to(dev)
+    hosts = [generators.laplacian2d_csr(8, 8)] * 512
+    h, begin, end = generators.block_diagonal(hosts, dtype=np.float64)
+    a = capi.to_device_csr(h, compact=True)
+    b = torch.ones(h.rows, dtype=torch.float64, device=dev)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ws = capi.Workspace()
+        capi.spmm(small, v, z, ws)
+        side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        capi.spmm(small, v, y, ws)
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            x = torch.zeros_like(b)
+            assert all(r.converged for r in capi.batch_pcg(a, begin, end, b, x, ws, relative_tolerance=1e-8))
+            y.zero_()
+            graph.replay()
+            side.synchronize()
+            assert torch.equal(y, z)
