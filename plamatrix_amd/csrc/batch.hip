@@ -1576,6 +1576,8 @@ int batch_solve(BatchProblem& b, const BatchPolicy& policy, pm_batch_report* rep
     PM_HIP(hipMemcpyAsync(hs, b.done_count, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
     PM_HIP(hipStreamSynchronize(stream));
     bool finished = static_cast<int64_t>(hs[0]) >= b.systems;
+    ws->last_one_launch = 0;
+    if (ws->persist_pause > 0) --ws->persist_pause;
     if (!finished && needed > 0 && b.single_reduction && !b.g && !b.split)
     {
         // systems of short, banded rows run to their end on their own CUs; the

@@ -2371,6 +2371,7 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     ws->last_value_streams = pb.dia.active ? pb.dia.streams : 0;
     ws->last_form = pb.cg_factored ? (pb.cg_fused ? 5 : 4) : pb.cg_fused ? 1 : pb.single_reduction ? 2 : 3;
     ws->last_preconditioner = pb.pre;
+    ws->last_one_launch = 0;
     if (a->rows == 0)
     {
         pm_solver_report rep{};
@@ -2388,6 +2389,7 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
     // diagonal layout over all CUs, a small CSR matrix in one workgroup, another
     // of short local rows with a row per lane (the device looks at its rows
     // ahead of the initialisation)
+    if (ws->persist_pause > 0) --ws->persist_pause;
     PersistProblem pp{};
     pp.rows = a->rows;
     pp.dtype = a->dtype;
@@ -2441,6 +2443,7 @@ int adaptive_solve(const pm_csr* a, const void* rhs, void* x, const void* inv_bl
         int outcome = 0;
         int64_t next = 0;
         PM_TRY(run(ws, pp, options->max_iterations, stream, &outcome, &next, &fin));
+        ws->last_one_launch = outcome != kPersistAbandoned ? 1 : run == persist_small_run ? 0 : -1;
         if (outcome == kPersistStopped)
         {
             PM_HIP(hipEventRecord(ws->done_event, stream));

@@ -169,9 +169,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
     if (tid == 0)
     {
         sh.hs.begin(a.st, a.t_end);
-        sh.fail = 0;
+        sh.fail = given_up(&a.ctl->abort);
     }
     __syncthreads();
+    if (sh.fail != 0) return;
 
     // the lane's rows of a vector into LDS and, where another workgroup reads
     // them, into the exchange

@@ -132,9 +132,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_batch_team(TeamArgs<S, I> a
         sh_alpha = static_cast<S>(state.alpha);
         sh_beta = static_cast<S>(state.beta);
         sh_code = state.done;
-        sh_fail = 0;
+        sh_fail = given_up(&a.ctl->abort);
     }
     __syncthreads();
+    if (sh_fail != 0) return;
     auto u_of = [&](int k) { return inv[k] * r[k]; };
 
     auto publish = [&](word* buf, unsigned tag, auto get) {
@@ -308,9 +309,12 @@ __global__ __launch_bounds__(kBlock) void k_team_commit(const TeamControl* ctl, 
     for (int l = threadIdx.x; l < size; l += kBlock) x[job.begin + first + l] = from[job.begin + first + l];
 }
 
-__global__ void k_team_states(const TeamControl* ctl, int slots, BatchState* st, unsigned long long* done_count)
+// *gave_up = 1 (host memory) when the launch was left unfinished.
+__global__ void k_team_states(const TeamControl* ctl, int slots, BatchState* st, unsigned long long* done_count,
+                              unsigned* gave_up)
 {
     const int slot = static_cast<int>(threadIdx.x);
+    if (slot == 0 && ctl->abort != 0u) *gave_up = 1u;
     if (slot >= slots) return;
     const TeamTask job = ctl->tasks[slot];
     if (job.piece != 0 || ctl->finished[slot] != static_cast<unsigned>(job.team)) return;
@@ -319,9 +323,11 @@ __global__ void k_team_states(const TeamControl* ctl, int slots, BatchState* st,
     atomicAdd(done_count, 1ull);
 }
 
-__global__ void k_team_reset(TeamControl* ctl)
+// `before`: the call's launch before this one (or null); after one that gave up the
+// next ones do too, so that a call waits for one of them at most.
+__global__ void k_team_reset(TeamControl* ctl, const TeamControl* before, unsigned abort)
 {
-    if (threadIdx.x == 0) ctl->abort = 0u;
+    if (threadIdx.x == 0) ctl->abort = before != nullptr && before->abort != 0u ? 1u : abort;
     if (threadIdx.x < kTeamSlots) ctl->finished[threadIdx.x] = 0u;
 }
 
@@ -496,6 +502,10 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         PM_HIP(hipMemcpyAsync(ctl->tasks, launches[k].data(), sizeof(TeamTask) * launches[k].size(),
                               hipMemcpyHostToDevice, stream));
     }
+    unsigned* gave_up = &ws->host_state[0].counters[0];
+    *gave_up = 0u;
+    ws->last_one_launch = 1;
+    const TeamControl* before = nullptr;
     for (size_t k = 0; k < launches.size(); ++k)
     {
         auto* ctl = reinterpret_cast<TeamControl*>(blocks0 + k * control);
@@ -508,20 +518,31 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         a.give_up = reinterpret_cast<PersistControl*>(ctl);
         a.tag = ws->teams_tag;
         ws->teams_tag += static_cast<uint32_t>(b.max_iterations) + 2u;
-        hipLaunchKernelGGL(k_team_reset, dim3(1), dim3(kTeamSlots), 0, stream, ctl);
+        hipLaunchKernelGGL(k_team_reset, dim3(1), dim3(kTeamSlots), 0, stream, ctl, before,
+                           persist_test("give_up=", -1) == static_cast<int64_t>(k) ? 1u : 0u);
+        before = ctl;
         PM_HIP(hipGetLastError());
         void* args[] = {&a};
-        const hipError_t err = hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(kPersistThreads), args,
-                                                          static_cast<unsigned>(lds), stream);
-        if (persist_refused(err, ws)) break;
+        const hipError_t err = persist_launch(kernel, grid, args, lds, stream, static_cast<int64_t>(k));
+        if (persist_refused(err, ws))
+        {
+            ws->last_one_launch = -1;
+            break;
+        }
         PM_HIP(err);
         hipLaunchKernelGGL(k_team_commit<S>, dim3(grid), dim3(kBlock), 0, stream, ctl, static_cast<int>(piece),
                            static_cast<const S*>(b.x_out), static_cast<S*>(b.x));
-        hipLaunchKernelGGL(k_team_states, dim3(1), dim3(kTeamSlots), 0, stream, ctl, grid, b.st, b.done_count);
+        hipLaunchKernelGGL(k_team_states, dim3(1), dim3(kTeamSlots), 0, stream, ctl, grid, b.st, b.done_count,
+                           gave_up);
         PM_HIP(hipGetLastError());
     }
     // the launches vector is the source of the copies above
     PM_HIP(hipStreamSynchronize(stream));
+    if (*gave_up != 0u)
+    {
+        ws->persist_pause = kPersistPause;
+        ws->last_one_launch = -1;
+    }
     return PM_OK;
 }
 

@@ -128,6 +128,12 @@ __device__ __forceinline__ bool wait_for(PersistControl* ctl, Poll poll)
     return true;
 }
 
+// Whether another workgroup already gave up: a workgroup that starts late leaves at once.
+__device__ __forceinline__ int given_up(const unsigned* abort)
+{
+    return __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ? 1 : 0;
+}
+
 // The workgroup-shared part of a persistent solve.
 template <typename S>
 struct PersistShared

@@ -4,15 +4,16 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 
 #include "persist_device.hpp"
 
 namespace pm
 {
 
-static __global__ void k_persist_reset(PersistControl* ctl, SolverState* st)
+static __global__ void k_persist_reset(PersistControl* ctl, SolverState* st, unsigned abort)
 {
-    ctl->abort = 0u;
+    ctl->abort = abort;
     ctl->finished = 0u;
     st->counters[kCounterOutcome] = 0u;
 }
@@ -45,10 +46,25 @@ inline bool persist_enabled()
     return env == nullptr || env[0] != '0';
 }
 
+// What a test asks of the launches in PLAMATRIX_AMD_PERSIST_TEST, a list of
+// name=number: the number, or `none`.  refuse=k: launch k of a call is turned down;
+// give_up=k: its workgroups find a notice to give up.
+inline int64_t persist_test(const char* name, int64_t none)
+{
+    const char* env = std::getenv("PLAMATRIX_AMD_PERSIST_TEST");
+    const char* at = env != nullptr ? std::strstr(env, name) : nullptr;
+    return at != nullptr ? std::atoll(at + std::strlen(name)) : none;
+}
+
+// Solves (passes of a refinement, batches) for which a workspace stays on the
+// per-kernel forms after a launch was refused or gave up: whatever kept its
+// workgroups from running together would cost each of them up to kWaitSeconds.
+constexpr int kPersistPause = 64;
+
 // Whether `blocks` workgroups of a CU each can run together.
 inline bool persist_resident(const pm_workspace* ws, int blocks)
 {
-    if (ws->cooperative_refused) return false;
+    if (ws->persist_pause > 0) return false;
     const int device = ws->device;
     int coop = 0, cus = 0;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess ||
@@ -62,15 +78,22 @@ inline bool persist_resident(const pm_workspace* ws, int blocks)
 
 // A cooperative launch that the runtime turned down, as it does for every
 // process but the first that holds a cooperative queue on the device
-// (hipErrorIllegalState): the workspace stays on the per-kernel forms from then
-// on, without an error.
+// (hipErrorIllegalState): the workspace turns to the per-kernel forms, without an
+// error.
 inline bool persist_refused(hipError_t err, pm_workspace* ws)
 {
     if (err != hipErrorCooperativeLaunchTooLarge && err != hipErrorNotSupported && err != hipErrorIllegalState)
         return false;
     (void)hipGetLastError();
-    ws->cooperative_refused = true;
+    ws->persist_pause = kPersistPause;
     return true;
+}
+
+// Launch `number` of a call.
+inline hipError_t persist_launch(const void* kernel, int blocks, void** args, size_t lds, hipStream_t stream, int64_t number)
+{
+    if (persist_test("refuse=", -1) == number) return hipErrorIllegalState;
+    return hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads), args, static_cast<unsigned>(lds), stream);
 }
 
 // Every workgroup decides for itself, or eight decide and answer the rest.
@@ -102,7 +125,8 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
     a.xu = reinterpret_cast<word*>(ws->persist.as<char>() + control);
     a.xx = a.xu + words;
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>(ceil_div(p.rows, kBlock), 2048));
-    for (int64_t t = 0;; )
+    int64_t number = 0;
+    for (int64_t t = 0;; ++number)
     {
         // an even number of iterations, the last one's decision included
         const int64_t left = max_iterations + 2 - t;
@@ -112,11 +136,11 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
         if (t > 0) a.x_in = a.x_out;
         a.tag = ws->persist_tag;
         ws->persist_tag += static_cast<uint32_t>(count) + 2u;
-        hipLaunchKernelGGL(k_persist_reset, dim3(1), dim3(1), 0, stream, a.ctl, p.st);
+        hipLaunchKernelGGL(k_persist_reset, dim3(1), dim3(1), 0, stream, a.ctl, p.st,
+                           persist_test("give_up=", -1) == number ? 1u : 0u);
         PM_HIP(hipGetLastError());
         void* args[] = {&a};
-        const hipError_t err = hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads), args,
-                                                          static_cast<unsigned>(lds), stream);
+        const hipError_t err = persist_launch(kernel, blocks, args, lds, stream, number);
         if (persist_refused(err, ws)) return PM_OK;
         PM_HIP(err);
         hipLaunchKernelGGL(k_persist_commit<S>, dim3(grid), dim3(kBlock), 0, stream, p.rows,
@@ -126,7 +150,11 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
         PM_HIP(hipMemcpyAsync(ws->host_state, p.st, sizeof(SolverState), hipMemcpyDeviceToHost, stream));
         PM_HIP(hipStreamSynchronize(stream));
         *state = ws->host_state[0];
-        if (state->counters[kCounterOutcome] != 1u) return PM_OK;
+        if (state->counters[kCounterOutcome] != 1u)
+        {
+            ws->persist_pause = kPersistPause;
+            return PM_OK;
+        }
         if (state->done != kRunning)
         {
             *outcome = kPersistStopped;

@@ -131,7 +131,8 @@ struct pm_workspace
     pm::DeviceBuffer dia_gt;    // ... and of G^T
     pm::DeviceBuffer persist;   // persistent solver: control block and exchange words
     uint32_t persist_tag = 0;   // last exchange tag used in it
-    bool cooperative_refused = false; // the runtime turned a cooperative launch down (another process has the queue)
+    int persist_pause = 0;      // solves left on the per-kernel forms after a one-launch form was refused or gave up
+    int32_t last_one_launch = 0; // the last solve in one launch: 1, fell back from it: -1, neither: 0
     pm::DeviceBuffer teams;     // persistent batch: exchange words and control blocks
     pm::DeviceBuffer looks;     // ... what it saw of each system's rows (scratch belongs to graphs that hold an SpMM)
     size_t teams_words = 0;     // words before its control blocks

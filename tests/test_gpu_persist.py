@@ -284,3 +284,50 @@ def test_factored_solve_is_bitwise(dev, monkeypatch, kind, dims, dtype, refresh)
             storage[flag] = ws.capacity_bytes
         assert storage["1"] > storage["0"]  # the exchange words: the persistent kernel ran
         assert out["0"] == out["1"], most
+
+
+def form_solve(form, dev):
+    """A solver of a fixed system of that one-launch form: f(ws, most) -> report and x."""
+    if form == "csr":
+        h = generators.laplacian2d_csr(90, 80)
+    elif form == "small":
+        h = generators.laplacian2d_csr(45, 37)
+    else:
+        h = matrix(*{"dia": ("laplace", (300, 290), np.float64), "factored": ("diffusion", (41, 43, 40), np.float32)}[form])
+    a = capi.to_device_csr(h, compact=True)
+    b = torch.from_numpy(generators.rhs_normal(a.rows, seed=41).astype(h.values.dtype)).to(dev)
+    graph = None
+    if form == "factored":
+        net = capi.FsaiNet(seed=0)
+        net.parameters = capi.fsai_initial_parameters(2)
+        graph = capi.FsaiGraph(a)
+        capi.fsai_forward(net, graph)
+
+    def run(ws, most=300):
+        x = torch.full_like(b, 0.5)
+        kw = dict(relative_tolerance=1e-5, max_iterations=most)
+        pol = capi.policy(refresh_interval=20)
+        rep = capi.pcg(a, b, x, ws, pol, **kw) if graph is None else capi.pcg_factored(a, b, x, graph, ws, pol=pol, **kw)
+        torch.cuda.synchronize()
+        return rep.converged, rep.iterations, rep.initial_residual, rep.final_residual, x.cpu().numpy().tobytes()
+
+    return run
+
+
+@pytest.mark.parametrize("form", ["dia", "csr", "factored"])
+@pytest.mark.parametrize("fault", ["refuse=0", "give_up=0"])
+def test_falls_back_to_the_kernels(dev, monkeypatch, form, fault):
+    # a launch that is turned down or gives up leaves x alone and the kernels run the
+    # solve; the workspace stays with them for 64 solves, then tries again
+    run = form_solve(form, dev)
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "0")
+    ref = run(capi.Workspace())
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "1")
+    ws = capi.Workspace()
+    assert run(ws) == ref and ws.solver_one_launch == 1
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", fault)
+    assert run(ws) == ref and ws.solver_one_launch == -1
+    monkeypatch.delenv("PLAMATRIX_AMD_PERSIST_TEST")
+    for k in range(63):
+        assert run(ws, 300 if k == 0 else 1)[1] >= 1 and ws.solver_one_launch == 0
+    assert run(ws) == ref and ws.solver_one_launch == 1

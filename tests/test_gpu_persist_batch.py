@@ -146,3 +146,35 @@ def test_a_captured_product_keeps_its_storage(dev):
             graph.replay()
             side.synchronize()
             assert torch.equal(y, z)
+
+
+@pytest.mark.parametrize("fault", ["refuse=0", "give_up=0", "refuse=1", "give_up=1"])
+def test_falls_back_to_the_kernels(dev, monkeypatch, fault):
+    # "launches": the teams of launches before the one that is turned down or gives up
+    # keep their solutions, the kernels solve the other systems
+    h, begin, end = batch("launches", np.float64)
+    a = capi.to_device_csr(h, compact=True)
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=3).astype(np.float64)).to(dev)
+
+    def run(ws):
+        x = torch.zeros_like(b)
+        reps = capi.batch_pcg(a, begin, end, b, x, ws, relative_tolerance=1e-10, max_iterations=3000)
+        torch.cuda.synchronize()
+        assert all(r.converged for r in reps)
+        return [r.iterations for r in reps], x
+
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "0")
+    kernels = run(capi.Workspace())
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "1")
+    teams = run(capi.Workspace())
+    ws = capi.Workspace()
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", fault)
+    got = run(ws)
+    assert ws.solver_one_launch == -1
+    one = [got[0][i] == kernels[0][i] and torch.equal(got[1][s:e], kernels[1][s:e]) for i, (s, e) in enumerate(zip(begin, end))]
+    two = [got[0][i] == teams[0][i] and torch.equal(got[1][s:e], teams[1][s:e]) for i, (s, e) in enumerate(zip(begin, end))]
+    assert all(p or q for p, q in zip(one, two))
+    assert all(one) if fault.endswith("0") else any(p and not q for p, q in zip(one, two)) and any(q and not p for p, q in zip(one, two))
+    monkeypatch.delenv("PLAMATRIX_AMD_PERSIST_TEST")
+    again = run(ws)  # the pause: the kernels
+    assert ws.solver_one_launch == 0 and again[0] == kernels[0] and torch.equal(again[1], kernels[1])
