@@ -172,7 +172,6 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
         sh.fail = given_up(&a.ctl->abort);
     }
     __syncthreads();
-    if (sh.fail != 0) return;
 
     // the lane's rows of a vector into LDS and, where another workgroup reads
     // them, into the exchange

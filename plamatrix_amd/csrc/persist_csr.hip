@@ -143,7 +143,6 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_csr(CsrArgs<S, I> a)
         sh.fail = given_up(&a.ctl->abort);
     }
     __syncthreads();
-    if (sh.fail != 0) return;
     auto u_of = [&]() { return JACOBI ? inv * r : r; };
 
     auto publish = [&](word* buf, unsigned tag, S v) {

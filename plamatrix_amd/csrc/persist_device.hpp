@@ -128,7 +128,8 @@ __device__ __forceinline__ bool wait_for(PersistControl* ctl, Poll poll)
     return true;
 }
 
-// Whether another workgroup already gave up: a workgroup that starts late leaves at once.
+// Whether another workgroup already gave up: a workgroup that starts late leaves at its
+// first decision (no exit of its own before: it costs the solve kernels registers).
 __device__ __forceinline__ int given_up(const unsigned* abort)
 {
     return __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ? 1 : 0;

@@ -107,7 +107,6 @@ __global__ __launch_bounds__(kPersistThreads) void k_cgf_persist(FactoredArgs<S>
         sh.fail = given_up(&a.ctl->abort);
     }
     __syncthreads();
-    if (sh.fail != 0) return;
 
     auto publish = [&](word* buf, S* win, unsigned tag, const S (&v)[R]) {
         int l = l0;
