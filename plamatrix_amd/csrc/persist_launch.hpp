@@ -47,8 +47,8 @@ inline bool persist_enabled()
 }
 
 // What a test asks of the launches in PLAMATRIX_AMD_PERSIST_TEST, a list of
-// name=number: the number, or `none`.  refuse=k: launch k of a call is turned down;
-// give_up=k: its workgroups find a notice to give up.
+// name=number: the number, or `none`.  refuse=k, too_large=k: launch k of a call is
+// turned down with that error; give_up=k: its workgroups find a notice to give up.
 inline int64_t persist_test(const char* name, int64_t none)
 {
     const char* env = std::getenv("PLAMATRIX_AMD_PERSIST_TEST");
@@ -76,16 +76,16 @@ inline bool persist_resident(const pm_workspace* ws, int blocks)
     return coop != 0 && blocks <= cus;
 }
 
-// A cooperative launch that the runtime turned down, as it does for every
-// process but the first that holds a cooperative queue on the device
-// (hipErrorIllegalState): the workspace turns to the per-kernel forms, without an
-// error.
+// A cooperative launch that the runtime turned down, without an error.  As it does
+// for every process but the first that holds a cooperative queue on the device
+// (hipErrorIllegalState): the workspace turns to the per-kernel forms.  A launch too
+// large for the device says nothing about the next one's shape.
 inline bool persist_refused(hipError_t err, pm_workspace* ws)
 {
     if (err != hipErrorCooperativeLaunchTooLarge && err != hipErrorNotSupported && err != hipErrorIllegalState)
         return false;
     (void)hipGetLastError();
-    ws->persist_pause = kPersistPause;
+    if (err != hipErrorCooperativeLaunchTooLarge) ws->persist_pause = kPersistPause;
     return true;
 }
 
@@ -93,6 +93,7 @@ inline bool persist_refused(hipError_t err, pm_workspace* ws)
 inline hipError_t persist_launch(const void* kernel, int blocks, void** args, size_t lds, hipStream_t stream, int64_t number)
 {
     if (persist_test("refuse=", -1) == number) return hipErrorIllegalState;
+    if (persist_test("too_large=", -1) == number) return hipErrorCooperativeLaunchTooLarge;
     return hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads), args, static_cast<unsigned>(lds), stream);
 }
 

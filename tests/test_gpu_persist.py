@@ -331,3 +331,15 @@ def test_falls_back_to_the_kernels(dev, monkeypatch, form, fault):
     for k in range(63):
         assert run(ws, 300 if k == 0 else 1)[1] >= 1 and ws.solver_one_launch == 0
     assert run(ws) == ref and ws.solver_one_launch == 1
+
+
+@pytest.mark.parametrize("form", ["dia", "csr", "factored"])
+def test_a_launch_too_large_keeps_other_shapes(dev, monkeypatch, form):
+    run, other = form_solve(form, dev), form_solve("dia" if form == "csr" else "csr", dev)
+    ws, fresh = capi.Workspace(), capi.Workspace()
+    ref = run(fresh), other(fresh)
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", "too_large=0")
+    assert run(ws) == ref[0] and ws.solver_one_launch == -1
+    monkeypatch.delenv("PLAMATRIX_AMD_PERSIST_TEST")
+    assert other(ws) == ref[1] and ws.solver_one_launch == 1
+    assert run(ws) == ref[0] and ws.solver_one_launch == 1
