@@ -110,8 +110,9 @@ int32_t pm_workspace_solver_form(const pm_workspace* ws);
  * held some of a batch's systems on the CUs; -1 if it fell back to the kernels
  * because such a launch was refused (another process has the device's
  * cooperative queue) or gave up waiting for workgroups that did not run
- * together with it (after up to 4 seconds), which keeps the workspace on the
- * kernels for its next 64 solves; else 0. */
+ * together with it (after up to 4 seconds), either of which keeps the workspace
+ * on the kernels for its next 64 solves, or because there was no memory for its
+ * exchange; else 0. */
 int32_t pm_workspace_solver_one_launch(const pm_workspace* ws);
 /* No reference counterpart: the preconditioner the last adaptive solve ran
  * (0: none, 1: Jacobi, 2: block-Jacobi, 3: factored G^T G).  A Jacobi solve of

@@ -468,7 +468,11 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
     // cleared with the whole buffer when the layout changes)
     if (need > ws->teams.bytes || ws->teams_words != plane_words || ws->teams_tag > 0xf0000000u)
     {
-        PM_TRY(ws->teams.reserve(need));
+        if (!persist_storage(ws->teams, need))
+        {
+            ws->last_one_launch = -1;
+            return PM_OK;
+        }
         hipLaunchKernelGGL(k_persist_clear, dim3(1024), dim3(kBlock), 0, stream, ws->teams.as<word>(),
                            static_cast<int64_t>(ws->teams.bytes / sizeof(word)));
         PM_HIP(hipGetLastError());
@@ -552,7 +556,12 @@ int batch_teams_look(pm_workspace* ws, const BatchTeams& b, std::vector<BatchLoo
 {
     look.assign(static_cast<size_t>(b.systems), BatchLook{0, 0});
     if (b.systems == 0 || b.chunks == 0 || !persist_enabled()) return PM_OK;
-    PM_TRY(ws->looks.reserve(sizeof(BatchLook) * static_cast<size_t>(b.systems)));
+    if (!persist_storage(ws->looks, sizeof(BatchLook) * static_cast<size_t>(b.systems)))
+    {
+        look.assign(look.size(), BatchLook{kTeamEntries + 1, 0});  // none fits
+        ws->last_one_launch = -1;
+        return PM_OK;
+    }
     auto* dev = ws->looks.as<BatchLook>();
     hipLaunchKernelGGL(k_look_reset, dim3(1), dim3(kBlock), 0, stream, b.systems, dev);
     const dim3 grid(static_cast<unsigned>(ceil_div(b.chunks, kBlock / kWave)));

@@ -48,12 +48,19 @@ inline bool persist_enabled()
 
 // What a test asks of the launches in PLAMATRIX_AMD_PERSIST_TEST, a list of
 // name=number: the number, or `none`.  refuse=k, too_large=k: launch k of a call is
-// turned down with that error; give_up=k: its workgroups find a notice to give up.
+// turned down with that error; give_up=k: its workgroups find a notice to give up;
+// storage=0: there is no memory for the exchange.
 inline int64_t persist_test(const char* name, int64_t none)
 {
     const char* env = std::getenv("PLAMATRIX_AMD_PERSIST_TEST");
     const char* at = env != nullptr ? std::strstr(env, name) : nullptr;
     return at != nullptr ? std::atoll(at + std::strlen(name)) : none;
+}
+
+// Storage that only the one-launch forms need: without it a solve takes the kernels.
+inline bool persist_storage(DeviceBuffer& buffer, size_t need)
+{
+    return persist_test("storage=", 1) != 0 && buffer.reserve(need) == PM_OK;
 }
 
 // Solves (passes of a refinement, batches) for which a workspace stays on the
@@ -113,7 +120,7 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
     const size_t control = (sizeof(PersistControl) + 255) & ~size_t(255);
     const size_t need = control + static_cast<size_t>(vectors) * words * sizeof(word);
     const bool grown = need > ws->persist.bytes;
-    PM_TRY(ws->persist.reserve(need));
+    if (!persist_storage(ws->persist, need)) return PM_OK;
     if (grown || ws->persist_tag > 0xf0000000u)
     {
         // no word may carry a tag that is still to come

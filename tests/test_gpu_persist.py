@@ -343,3 +343,14 @@ def test_a_launch_too_large_keeps_other_shapes(dev, monkeypatch, form):
     monkeypatch.delenv("PLAMATRIX_AMD_PERSIST_TEST")
     assert other(ws) == ref[1] and ws.solver_one_launch == 1
     assert run(ws) == ref[0] and ws.solver_one_launch == 1
+
+
+@pytest.mark.parametrize("form", ["dia", "csr", "factored"])
+def test_solves_without_the_exchange_storage(dev, monkeypatch, form):
+    run = form_solve(form, dev)
+    ref = run(capi.Workspace())
+    ws = capi.Workspace()
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", "storage=0")
+    assert run(ws) == ref and ws.solver_one_launch == -1
+    monkeypatch.delenv("PLAMATRIX_AMD_PERSIST_TEST")
+    assert run(ws) == ref and ws.solver_one_launch == 1

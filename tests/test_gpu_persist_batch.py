@@ -178,3 +178,18 @@ def test_falls_back_to_the_kernels(dev, monkeypatch, fault):
     monkeypatch.delenv("PLAMATRIX_AMD_PERSIST_TEST")
     again = run(ws)  # the pause: the kernels
     assert ws.solver_one_launch == 0 and again[0] == kernels[0] and torch.equal(again[1], kernels[1])
+
+
+def test_solves_without_the_teams_storage(dev, monkeypatch):
+    h, begin, end = batch("teams", np.float64)
+    a = capi.to_device_csr(h, compact=True)
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=3).astype(np.float64)).to(dev)
+    out = []
+    for name, value in (("PLAMATRIX_AMD_PERSISTENT", "0"), ("PLAMATRIX_AMD_PERSIST_TEST", "storage=0")):
+        with monkeypatch.context() as m:
+            m.setenv(name, value)
+            ws, x = capi.Workspace(), torch.zeros_like(b)
+            reps = capi.batch_pcg(a, begin, end, b, x, ws, relative_tolerance=1e-10, max_iterations=3000)
+            torch.cuda.synchronize()
+            out.append(([(r.converged, r.iterations) for r in reps], x.cpu().numpy().tobytes()))
+    assert out[0] == out[1] and ws.solver_one_launch == -1
