@@ -2073,9 +2073,11 @@ int prepare(pm_workspace* ws, Problem& pb, hipStream_t stream)
     const int64_t n = pb.a->rows;
     const size_t vec = ((elem_size(pb.a->dtype) * static_cast<size_t>(n > 0 ? n : 1)) + 255) & ~size_t(255);
     // a matrix the diagonal layout may take also gets the second buffers of
-    // the one-kernel single-reduction iteration
+    // the one-kernel single-reduction iteration; without them a size that the
+    // persistent CSR solve may take gets the vector it leaves x in
     const bool second = dia_wanted(pb.a);
-    PM_TRY(ws->vectors.reserve(vec * (second ? 10 : 7)));
+    const bool spare = second || n <= kPersistCsrRows;
+    PM_TRY(ws->vectors.reserve(vec * (second ? 10 : spare ? 7 : 6)));
     if (n > ws->capacity_rows) ws->capacity_rows = n;
     PM_TRY(ws->partials.reserve(sizeof(double) * kPartialsDoubles));
     PM_TRY(ws->state.reserve(4096));
@@ -2086,7 +2088,7 @@ int prepare(pm_workspace* ws, Problem& pb, hipStream_t stream)
     pb.p0 = base + 3 * vec;
     pb.p1 = base + 4 * vec;
     pb.inv = base + 5 * vec;
-    pb.spare = base + 6 * vec;
+    pb.spare = spare ? base + 6 * vec : nullptr;
     pb.r2 = second ? base + 6 * vec : nullptr;
     pb.z2 = second ? base + 7 * vec : nullptr;
     pb.q2 = second ? base + 8 * vec : nullptr;

@@ -14,6 +14,9 @@
 namespace pm
 {
 
+// Rows that the persistent solve of a CSR matrix takes, at most: a row per lane.
+constexpr int64_t kPersistCsrRows = 262144;
+
 // Largest chunk of iterations a solve's schedule grows to (adaptive_solve).
 constexpr int kMaxGrownChunk = 64;
 
@@ -31,7 +34,7 @@ struct PersistProblem
     void* x;
     void *r, *u, *w, *p, *s;
     const void* inv;
-    void* x_out;       // scratch vector the new x is written to before it is committed to x
+    void* x_out;       // scratch vector the new x is written to before it is committed to x (null where no form needs it)
     SolverState* st;
     double* region;    // partials of iteration t0 - 1 (t0 even)
     int count;         // workgroups of the per-kernel iteration (its partial sums)

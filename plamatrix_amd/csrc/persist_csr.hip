@@ -255,7 +255,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_csr(CsrArgs<S, I> a)
 
 // The split: a row per lane (the per-kernel workgroups hold at most four chunks
 // of 64 rows), so up to 262,144 rows on 256 CUs.
-constexpr int64_t kCsrRows = static_cast<int64_t>(kSolverGrid) * kBlock;
+static_assert(kPersistCsrRows == static_cast<int64_t>(kSolverGrid) * kBlock, "a row per lane of the solver grid");
 
 int csr_per(const PersistProblem& p)
 {
@@ -302,7 +302,7 @@ int csr_run(pm_workspace* ws, const PersistProblem& p, const I* ro, const I* ci,
 
 bool persist_csr_candidate(const PersistProblem& p, const pm_workspace* ws)
 {
-    return persist_enabled() && p.rows > 0 && p.rows <= kCsrRows && p.a->nnz <= p.rows * kCsrEntries &&
+    return persist_enabled() && p.rows > 0 && p.rows <= kPersistCsrRows && p.a->nnz <= p.rows * kCsrEntries &&
            csr_per(p) <= kWavesPerBlock && persist_resident(ws, csr_blocks(p));
 }
 

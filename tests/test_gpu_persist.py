@@ -354,3 +354,19 @@ def test_solves_without_the_exchange_storage(dev, monkeypatch, form):
     assert run(ws) == ref and ws.solver_one_launch == -1
     monkeypatch.delenv("PLAMATRIX_AMD_PERSIST_TEST")
     assert run(ws) == ref and ws.solver_one_launch == 1
+
+
+def test_large_solves_reserve_six_vectors(dev):
+    # past the sizes of the one-launch CSR solve, more diagonals than the layout takes
+    n, offsets = 262144 + 64, range(-8, 9)
+    i = np.arange(n)
+    valid = np.stack([(i + o >= 0) & (i + o < n) for o in offsets], axis=1)
+    cols = (i[:, None] + np.array(offsets))[valid]
+    values = np.where(cols == np.repeat(i, valid.sum(axis=1)), 17.0, -1.0)
+    ro = np.concatenate([[0], np.cumsum(valid.sum(axis=1))])
+    a = capi.to_device_csr(generators.CSRHost(n, n, ro, cols, values), compact=True)
+    b = torch.ones(n, dtype=torch.float64, device=dev)
+    ws = capi.Workspace()
+    rep = capi.pcg(a, b, torch.zeros_like(b), ws, relative_tolerance=1e-8, max_iterations=100)
+    assert rep.converged and ws.solver_form == 2 and ws.solver_one_launch == 0
+    assert ws.capacity_bytes < 6 * 8 * n * 9 / 8 + (2 << 20)  # storage grows by an eighth; partials and state
