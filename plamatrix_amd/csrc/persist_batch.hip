@@ -466,7 +466,10 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
     const size_t need = 2 * plane_words * sizeof(word) + control_all;
     // (blocks in a place that earlier held words, or the other way round, are
     // cleared with the whole buffer when the layout changes)
-    if (need > ws->teams.bytes || ws->teams_words != plane_words || ws->teams_tag > 0xf0000000u)
+    ws->teams_tag = static_cast<uint32_t>(persist_test("tag=", ws->teams_tag));
+    const uint64_t tags = launches.size() * (static_cast<uint64_t>(b.max_iterations) + 2u);
+    if (tags > kLastTag) return PM_OK;
+    if (need > ws->teams.bytes || ws->teams_words != plane_words || ws->teams_tag + tags > kLastTag)
     {
         if (!persist_storage(ws->teams, need))
         {

@@ -49,7 +49,8 @@ inline bool persist_enabled()
 // What a test asks of the launches in PLAMATRIX_AMD_PERSIST_TEST, a list of
 // name=number: the number, or `none`.  refuse=k, too_large=k: launch k of a call is
 // turned down with that error; give_up=k: its workgroups find a notice to give up;
-// storage=0: there is no memory for the exchange.
+// storage=0: there is no memory for the exchange; segment=n: launches of n (even)
+// iterations; tag=n: the last exchange tag used.
 inline int64_t persist_test(const char* name, int64_t none)
 {
     const char* env = std::getenv("PLAMATRIX_AMD_PERSIST_TEST");
@@ -104,6 +105,9 @@ inline hipError_t persist_launch(const void* kernel, int blocks, void** args, si
     return hipLaunchCooperativeKernel(kernel, dim3(blocks), dim3(kPersistThreads), args, static_cast<unsigned>(lds), stream);
 }
 
+// Exchange tags run up to here before the words are cleared and they start again.
+constexpr uint32_t kLastTag = 0xf0000000u;
+
 // Every workgroup decides for itself, or eight decide and answer the rest.
 inline int persist_leaders(int blocks) { return blocks <= 64 ? blocks : kXcds; }
 
@@ -121,14 +125,9 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
     const size_t need = control + static_cast<size_t>(vectors) * words * sizeof(word);
     const bool grown = need > ws->persist.bytes;
     if (!persist_storage(ws->persist, need)) return PM_OK;
-    if (grown || ws->persist_tag > 0xf0000000u)
-    {
-        // no word may carry a tag that is still to come
-        hipLaunchKernelGGL(k_persist_clear, dim3(1024), dim3(kBlock), 0, stream, ws->persist.as<word>(),
-                           static_cast<int64_t>(ws->persist.bytes / sizeof(word)));
-        PM_HIP(hipGetLastError());
-        ws->persist_tag = 0;
-    }
+    if (grown) ws->persist_tag = kLastTag;
+    else ws->persist_tag = static_cast<uint32_t>(persist_test("tag=", ws->persist_tag));
+    const int64_t segment = persist_test("segment=", kSegment);
     a.ctl = ws->persist.as<PersistControl>();
     a.xu = reinterpret_cast<word*>(ws->persist.as<char>() + control);
     a.xx = a.xu + words;
@@ -138,10 +137,18 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
     {
         // an even number of iterations, the last one's decision included
         const int64_t left = max_iterations + 2 - t;
-        const int64_t count = std::min<int64_t>(kSegment, left + (left & 1));
+        const int64_t count = std::min<int64_t>(segment, left + (left & 1));
         a.t0 = static_cast<int>(t);
         a.t_end = static_cast<int>(t + count);
         if (t > 0) a.x_in = a.x_out;
+        if (ws->persist_tag >= kLastTag)
+        {
+            // no word may carry a tag that is still to come
+            hipLaunchKernelGGL(k_persist_clear, dim3(1024), dim3(kBlock), 0, stream, ws->persist.as<word>(),
+                               static_cast<int64_t>(ws->persist.bytes / sizeof(word)));
+            PM_HIP(hipGetLastError());
+            ws->persist_tag = 0;
+        }
         a.tag = ws->persist_tag;
         ws->persist_tag += static_cast<uint32_t>(count) + 2u;
         hipLaunchKernelGGL(k_persist_reset, dim3(1), dim3(1), 0, stream, a.ctl, p.st,

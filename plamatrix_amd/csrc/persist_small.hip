@@ -281,12 +281,13 @@ int small_run(pm_workspace* ws, const PersistProblem& p, const I* ro, const I* c
     a.grow = p.grow ? 1 : 0;
     const void* kernel = small_kernel<S, I>(static_cast<int>(ceil_div(p.count, kSmallGroups)), p.jacobi);
     *outcome = kPersistAbandoned;
+    const int64_t segment = persist_test("segment=", kSmallSegment);
     for (int64_t t = 0;;)
     {
         // an even number of iterations, the last one's decision included
         const int64_t left = max_iterations + 2 - t;
         a.t0 = static_cast<int>(t);
-        a.t_end = static_cast<int>(t + std::min<int64_t>(kSmallSegment, left + (left & 1)));
+        a.t_end = static_cast<int>(t + std::min<int64_t>(segment, left + (left & 1)));
         void* args[] = {&a};
         PM_HIP(hipLaunchKernel(kernel, dim3(1), dim3(kSmallThreads), args, 0, stream));
         PM_HIP(hipMemcpyAsync(ws->host_state, p.st, sizeof(SolverState), hipMemcpyDeviceToHost, stream));

@@ -370,3 +370,32 @@ def test_large_solves_reserve_six_vectors(dev):
     rep = capi.pcg(a, b, torch.zeros_like(b), ws, relative_tolerance=1e-8, max_iterations=100)
     assert rep.converged and ws.solver_form == 2 and ws.solver_one_launch == 0
     assert ws.capacity_bytes < 6 * 8 * n * 9 / 8 + (2 << 20)  # storage grows by an eighth; partials and state
+
+
+@pytest.mark.parametrize("form", ["dia", "csr", "small", "factored"])
+@pytest.mark.parametrize("test", ["segment=2", "segment=6", "segment=6,tag=4026531830"])
+def test_a_solve_of_several_launches(dev, monkeypatch, form, test):
+    # a launch continues the one before it: x, vectors, partials, history and tags; the
+    # last exchange tags used are just below 0xf0000000, where the words are cleared
+    run = form_solve(form, dev)
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "0")
+    ref = [run(capi.Workspace(), most) for most in (300, 5, 12)]
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "1")
+    ws = capi.Workspace()
+    assert run(ws) == ref[0] and ref[0][1] > 12  # the storage is in place
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", test)
+    for most, want in zip((300, 5, 12), ref):
+        assert run(ws, most) == want and ws.solver_one_launch == 1
+
+
+@pytest.mark.parametrize("form", ["dia", "csr", "factored"])
+@pytest.mark.parametrize("fault", ["refuse=2", "give_up=2"])
+def test_falls_back_after_a_launch(dev, monkeypatch, form, fault):
+    # two launches of the solve have ended: x is still the caller's
+    run = form_solve(form, dev)
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "0")
+    ref = run(capi.Workspace())
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", "1")
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", "segment=4," + fault)
+    ws = capi.Workspace()
+    assert run(ws) == ref and ws.solver_one_launch == -1

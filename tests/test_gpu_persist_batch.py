@@ -193,3 +193,18 @@ def test_solves_without_the_teams_storage(dev, monkeypatch):
             torch.cuda.synchronize()
             out.append(([(r.converged, r.iterations) for r in reps], x.cpu().numpy().tobytes()))
     assert out[0] == out[1] and ws.solver_one_launch == -1
+
+
+def test_exchange_tags_start_again(dev, monkeypatch):
+    h, begin, end = batch("launches", np.float32)
+    a = capi.to_device_csr(h, compact=True)
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=3)).to(dev)
+    ws, out = capi.Workspace(), []
+    for test in ("", "tag=4026531830", ""):
+        monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", test)
+        x = torch.zeros_like(b)
+        reps = capi.batch_pcg(a, begin, end, b, x, ws, relative_tolerance=1e-5, max_iterations=3000)
+        torch.cuda.synchronize()
+        assert ws.solver_one_launch == 1
+        out.append(([(r.converged, r.iterations) for r in reps], x.cpu().numpy().tobytes()))
+    assert out[0] == out[1] == out[2]
