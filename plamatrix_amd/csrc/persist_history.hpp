@@ -11,6 +11,7 @@ namespace pm
 constexpr int kHandOver = 100;      // decision code: leave without deciding
 constexpr int kCounterOutcome = 1;  // SolverState::counters slot: what became of a launch
 constexpr int kCounterNext = 2;     // ... iteration the launch handed over at
+constexpr int kCounterOver = 3;     // ... iteration a restart hands over at (0: none yet)
 
 // Kept in LDS by the one thread that decides: as registers it would take some
 // from every lane.
@@ -18,7 +19,8 @@ struct PersistHistory
 {
     CgHistory h;
     double rr, rr0, alpha;
-    int completed, t_stop, restarted;
+    int completed, t_stop;
+    int over;  // iteration a restart hands over at, in this launch or a later one; 0: none
 
     // before iteration t0 (even) of a solve, launched up to iteration t_end
     __device__ __forceinline__ void begin(const SolverState* st, int t_end)
@@ -28,8 +30,8 @@ struct PersistHistory
         completed = st->iter[1] + 1;
         rr0 = st->rr0;
         rr = alpha = 0.0;
-        t_stop = t_end;
-        restarted = 0;
+        over = static_cast<int>(st->counters[kCounterOver]);
+        t_stop = over != 0 && over < t_end ? over : t_end;
     }
 
     // The decision at the head of iteration t; kHandOver at the iteration the
@@ -48,11 +50,11 @@ struct PersistHistory
         h.tol = d.tol;
         h.gamma_prev = gamma;
         h.den_prev = d.den;
-        if (d.restart && restarted == 0)
+        if (d.restart && over == 0)
         {
-            restarted = 1;
-            const int64_t over = hand_over_iteration(t, chunk, grow, kMaxGrownChunk);
-            if (over < t_stop) t_stop = static_cast<int>(over);
+            const int64_t at = hand_over_iteration(t, chunk, grow, kMaxGrownChunk);
+            over = at < INT32_MAX ? static_cast<int>(at) : INT32_MAX;
+            if (over < t_stop) t_stop = over;
         }
         ++completed;
         return d.code;
@@ -71,7 +73,8 @@ struct PersistHistory
         st->rho[par] = h.gamma_prev;
         st->den[par] = h.den_prev;
         st->alpha = alpha;
-        if (restarted) st->counters[kCounterRestart] = 1u;
+        st->counters[kCounterOver] = static_cast<unsigned>(over);
+        if (over != 0 && (code != kHandOver || completed >= over)) st->counters[kCounterRestart] = 1u;
         st->counters[kCounterNext] = static_cast<unsigned>(completed);
         if (code != kHandOver) st->done = code;
     }

@@ -399,3 +399,27 @@ def test_falls_back_after_a_launch(dev, monkeypatch, form, fault):
     monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", "segment=4," + fault)
     ws = capi.Workspace()
     assert run(ws) == ref and ws.solver_one_launch == -1
+
+
+@pytest.mark.parametrize("dims", [(45, 37), (90, 80), (300, 290)])
+def test_hand_over_after_several_launches(dev, monkeypatch, dims):
+    # an indefinite matrix in the one-workgroup, CSR and diagonal-layout forms
+    h = generators.laplacian2d_csr(*dims)
+    rows = np.repeat(np.arange(h.rows), np.diff(h.row_offsets))
+    for shift in (3.9, 0.05, 0.01):
+        v = h.values - shift * (rows == h.col_indices)
+        a = capi.to_device_csr(generators.CSRHost(h.rows, h.cols, h.row_offsets, h.col_indices, v), compact=True)
+        b = torch.from_numpy(generators.rhs_normal(h.rows, seed=31).astype(np.float64)).to(dev)
+        out = []
+        for persistent, test in (("0", ""), ("1", "segment=6")):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", persistent)
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSIST_TEST", test)
+            x = torch.zeros_like(b)
+            try:
+                rep = capi.cg(a, b, x, capi.Workspace(), relative_tolerance=1e-9, max_iterations=400)
+                got = ("ok", rep.iterations, rep.final_residual)
+            except capi.PlamatrixError as e:
+                got = (e.kind, str(e))
+            torch.cuda.synchronize()
+            out.append(got + (x.cpu().numpy().tobytes(),))
+        assert out[0] == out[1], shift
