@@ -1595,7 +1595,6 @@ int batch_solve(BatchProblem& b, const BatchPolicy& policy, pm_batch_report* rep
         teams.rhs = b.rhs;
         teams.x = b.x;
         teams.r = b.r;
-        teams.u = b.z;
         teams.w = b.q;
         teams.p = b.p0;
         teams.s = b.p1;
@@ -1606,11 +1605,15 @@ int batch_solve(BatchProblem& b, const BatchPolicy& policy, pm_batch_report* rep
         teams.max_iterations = b.max_iterations;
         teams.refresh = policy.refresh;
         if (b.look.empty()) PM_TRY(batch_teams_look(ws, teams, b.look, stream));
-        PM_TRY(batch_teams_run(ws, teams, b.look, stream));
-        PM_HIP(hipMemcpyAsync(hs, b.done_count, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
-        PM_HIP(hipStreamSynchronize(stream));
-        finished = static_cast<int64_t>(hs[0]) >= b.systems;
-        if (!finished) PM_TRY(batch_plan<S>(ws, b, 2, 0, 0, 0)->run(stream, false));
+        bool ran = false;
+        PM_TRY(batch_teams_run(ws, teams, b.look, stream, &ran));
+        if (ran)
+        {
+            PM_HIP(hipMemcpyAsync(hs, b.done_count, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
+            PM_HIP(hipStreamSynchronize(stream));
+            finished = static_cast<int64_t>(hs[0]) >= b.systems;
+            if (!finished) PM_TRY(batch_plan<S>(ws, b, 2, 0, 0, 0)->run(stream, false));
+        }
     }
     unsigned long long listed_at = hs[0];  // stopped systems when the list was last built
     if (!finished && needed > 0)

@@ -331,50 +331,63 @@ __global__ void k_team_reset(TeamControl* ctl, const TeamControl* before, unsign
     if (threadIdx.x < kTeamSlots) ctl->finished[threadIdx.x] = 0u;
 }
 
-// Longest row and band per system, a wavefront per 64-row chunk.
+// The band of every system of short rows, kNoBand for the others: rows too long, a
+// column outside the system, or more than `largest` rows.  A wavefront takes
+// consecutive 64-row chunks and tells a system's value once per run of its chunks
+// (once per chunk, 24,752 chunks of 8 systems waited 0.55 ms for the one cache line;
+// now DDD us).
+constexpr int kNoBand = 0x7fffffff;
+constexpr int kLookWaves = 2048;
 template <typename I>
 __global__ __launch_bounds__(kBlock) void k_team_look(int64_t chunks, const int32_t* __restrict__ chunk_sys,
                                                       const int64_t* __restrict__ sys_end,
                                                       const int64_t* __restrict__ sys_chunk0,
                                                       const I* __restrict__ ro, const I* __restrict__ ci,
-                                                      BatchLook* look)
+                                                      int64_t largest, BatchLook* look)
 {
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave;
-    if (c >= chunks) return;
-    const int32_t s = chunk_sys[c];
-    if (s < 0) return;
-    const int64_t row = c * kChunkRows + threadIdx.x % kWave;
-    int longest = 0, band = 0;
-    if (row < sys_end[s])
+    const int64_t waves = static_cast<int64_t>(gridDim.x) * (kBlock / kWave);
+    const int64_t per = (chunks + waves - 1) / waves;
+    const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + threadIdx.x / kWave;
+    const int64_t c1 = (wave + 1) * per < chunks ? (wave + 1) * per : chunks;
+    int32_t now = -1;
+    int band = 0;
+    auto tell = [&]() {
+        if (now < 0) return;
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off /= 2) band = max(band, __shfl_xor(band, off, kWave));
+        if (threadIdx.x % kWave == 0) atomicMax(&look[now].band, band);
+    };
+    for (int64_t c = wave * per; c < c1; ++c)
     {
+        const int32_t s = chunk_sys[c];
+        if (s != now)
+        {
+            tell();
+            now = s;
+            band = 0;
+        }
+        if (s < 0) continue;
+        const int64_t row = c * kChunkRows + threadIdx.x % kWave;
+        const int64_t begin = sys_chunk0[s] * kChunkRows, end = sys_end[s];
+        if (end - begin > largest) band = kNoBand;
+        if (row >= end || band == kNoBand) continue;
         const int64_t b = static_cast<int64_t>(ro[row]), e = static_cast<int64_t>(ro[row + 1]);
-        longest = static_cast<int>(e - b);
-        if (longest <= kTeamEntries)
+        if (e - b > kTeamEntries) band = kNoBand;
+        else
             for (int64_t k = b; k < e; ++k)
             {
                 const int64_t col = static_cast<int64_t>(ci[k]);
-                const int64_t far = col < row ? row - col : col - row;
-                band = far > band ? static_cast<int>(far > 0x3fffffff ? 0x3fffffff : far) : band;
-                // a column outside the system leaves it to the per-kernel form
-                if (col < sys_chunk0[s] * kChunkRows || col >= sys_end[s]) longest = kTeamEntries + 1;
+                // a system has at most 2^18 rows here
+                if (col < begin || col >= end) band = kNoBand;
+                else band = max(band, static_cast<int>(col < row ? row - col : col - row));
             }
     }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off /= 2)
-    {
-        longest = max(longest, __shfl_xor(longest, off, kWave));
-        band = max(band, __shfl_xor(band, off, kWave));
-    }
-    if (threadIdx.x % kWave == 0)
-    {
-        atomicMax(&look[s].longest, longest);
-        atomicMax(&look[s].band, band);
-    }
+    tell();
 }
 
 __global__ void k_look_reset(int64_t systems, BatchLook* look)
 {
-    for (int64_t s = threadIdx.x; s < systems; s += blockDim.x) look[s] = BatchLook{0, 0};
+    for (int64_t s = threadIdx.x; s < systems; s += blockDim.x) look[s] = BatchLook{0};
 }
 
 size_t team_lds(int es, int rows_per_lane, int halo)
@@ -393,16 +406,33 @@ const void* team_kernel(int rows_per_lane)
     return nullptr;
 }
 
+// Rows per lane that the registers hold.
+template <typename S>
+constexpr int team_rows()
+{
+    return sizeof(S) == 4 ? 4 : 2;
+}
+
+// Workgroups of a launch at most; 0: no teams.
+int team_slots(const pm_workspace* ws, const BatchTeams& b, int* slots)
+{
+    *slots = 0;
+    if (!persist_enabled() || !persist_resident(ws, 1) || b.max_iterations > kTeamIterations) return PM_OK;
+    int cus = 0;
+    PM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ws->device));
+    *slots = std::min(cus, kTeamSlots);
+    return PM_OK;
+}
+
 template <typename S, typename I>
 int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook>& look, const I* ro, const I* ci,
-              hipStream_t stream)
+              hipStream_t stream, bool* ran)
 {
-    const int most = sizeof(S) == 4 ? 4 : 2;  // rows per lane that the registers hold
+    *ran = false;
+    const int most = team_rows<S>();
     const int es = static_cast<int>(sizeof(S));
-    int cus = 0;
-    if (!persist_enabled() || !persist_resident(ws, 1) || b.max_iterations > kTeamIterations) return PM_OK;
-    PM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ws->device));
-    const int slots = std::min(cus, kTeamSlots);
+    int slots = 0;
+    PM_TRY(team_slots(ws, b, &slots));
     std::vector<int> order;
     int64_t total[3] = {0, 0, 0};  // workgroups with 1, 2, 4 rows per lane
     for (int64_t s = 0; s < b.systems; ++s)
@@ -411,12 +441,13 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         const BatchLook& l = look[static_cast<size_t>(s)];
         const int64_t piece = static_cast<int64_t>(most) * kPersistThreads;
         const int64_t team = ceil_div(n, piece);
-        if (n <= 0 || b.skip[s] || l.longest > kTeamEntries || team > std::min(kTeamLargest, slots)) continue;
+        if (n <= 0 || b.skip[s] || l.band == kNoBand || team > std::min(kTeamLargest, slots)) continue;
         if (team > 1 && (team_lds(es, most, l.band) > kTeamLds || piece + 2 * static_cast<int64_t>(l.band) > 65535)) continue;
         order.push_back(static_cast<int>(s));
         for (int k = 0; k < 3; ++k) total[k] += ceil_div(n, static_cast<int64_t>(kPersistThreads) << k);
     }
     if (order.empty()) return PM_OK;
+    *ran = true;
     // as few rows per lane as let all teams run together (and no team grow past
     // its decision's lanes)
     int rows_per_lane = most;
@@ -557,38 +588,44 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
 
 int batch_teams_look(pm_workspace* ws, const BatchTeams& b, std::vector<BatchLook>& look, hipStream_t stream)
 {
-    look.assign(static_cast<size_t>(b.systems), BatchLook{0, 0});
-    if (b.systems == 0 || b.chunks == 0 || !persist_enabled()) return PM_OK;
+    look.assign(static_cast<size_t>(b.systems), BatchLook{kNoBand});  // none fits
+    int slots = 0;
+    PM_TRY(team_slots(ws, b, &slots));
+    const int64_t piece = static_cast<int64_t>(b.a->dtype == PM_F64 ? team_rows<double>() : team_rows<float>()) * kPersistThreads;
+    const int64_t largest = piece * std::min(kTeamLargest, slots);
+    bool any = false;
+    for (int64_t s = 0; s < b.systems && !any; ++s) any = !b.skip[s] && b.end[s] > b.begin[s] && b.end[s] - b.begin[s] <= largest;
+    if (!any || b.chunks == 0) return PM_OK;
     if (!persist_storage(ws->looks, sizeof(BatchLook) * static_cast<size_t>(b.systems)))
     {
-        look.assign(look.size(), BatchLook{kTeamEntries + 1, 0});  // none fits
         ws->last_one_launch = -1;
         return PM_OK;
     }
     auto* dev = ws->looks.as<BatchLook>();
     hipLaunchKernelGGL(k_look_reset, dim3(1), dim3(kBlock), 0, stream, b.systems, dev);
-    const dim3 grid(static_cast<unsigned>(ceil_div(b.chunks, kBlock / kWave)));
+    const dim3 grid(static_cast<unsigned>(ceil_div(std::min<int64_t>(b.chunks, kLookWaves), kBlock / kWave)));
     if (use_compact(b.a))
         hipLaunchKernelGGL(k_team_look<int32_t>, grid, dim3(kBlock), 0, stream, b.chunks, b.chunk_sys, b.sys_end,
-                           b.sys_chunk0, b.a->row_offsets32, b.a->col_indices32, dev);
+                           b.sys_chunk0, b.a->row_offsets32, b.a->col_indices32, largest, dev);
     else
         hipLaunchKernelGGL(k_team_look<int64_t>, grid, dim3(kBlock), 0, stream, b.chunks, b.chunk_sys, b.sys_end,
-                           b.sys_chunk0, b.a->row_offsets, b.a->col_indices, dev);
+                           b.sys_chunk0, b.a->row_offsets, b.a->col_indices, largest, dev);
     PM_HIP(hipGetLastError());
     PM_HIP(hipMemcpyAsync(look.data(), dev, sizeof(BatchLook) * look.size(), hipMemcpyDeviceToHost, stream));
     PM_HIP(hipStreamSynchronize(stream));
     return PM_OK;
 }
 
-int batch_teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook>& look, hipStream_t stream)
+int batch_teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook>& look, hipStream_t stream,
+                    bool* ran)
 {
     const pm_csr* m = b.a;
     const bool compact = use_compact(m);
     if (m->dtype == PM_F64)
-        return compact ? teams_run<double>(ws, b, look, m->row_offsets32, m->col_indices32, stream)
-                       : teams_run<double>(ws, b, look, m->row_offsets, m->col_indices, stream);
-    return compact ? teams_run<float>(ws, b, look, m->row_offsets32, m->col_indices32, stream)
-                   : teams_run<float>(ws, b, look, m->row_offsets, m->col_indices, stream);
+        return compact ? teams_run<double>(ws, b, look, m->row_offsets32, m->col_indices32, stream, ran)
+                       : teams_run<double>(ws, b, look, m->row_offsets, m->col_indices, stream, ran);
+    return compact ? teams_run<float>(ws, b, look, m->row_offsets32, m->col_indices32, stream, ran)
+                   : teams_run<float>(ws, b, look, m->row_offsets, m->col_indices, stream, ran);
 }
 
 } // namespace pm

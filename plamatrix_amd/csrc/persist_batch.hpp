@@ -11,11 +11,10 @@ namespace pm
 // What the device saw of one system's rows.
 struct BatchLook
 {
-    int longest;  // entries of its longest row
-    int band;     // largest |column - row| (rows no longer than the kernel takes)
+    int band;  // largest |column - row|, or the largest int: not for a team
 };
 
-// A batched CG / Jacobi solve after its initialisation: r, u (z), w (q), p (p0),
+// A batched CG / Jacobi solve after its initialisation: r, w (q), p (p0),
 // s (p1) and the states of iteration 0 are in place.
 struct BatchTeams
 {
@@ -30,7 +29,7 @@ struct BatchTeams
     const int64_t* sys_chunk0; // device: first 64-row chunk
     const void* rhs;
     void* x;
-    const void *r, *u, *w, *p, *s;
+    const void *r, *w, *p, *s;
     const void* inv;           // null: no preconditioner
     void* x_out;               // scratch vector
     BatchState* st;
@@ -39,11 +38,12 @@ struct BatchTeams
     int refresh;
 };
 
-// Looks at the rows of every system (once per matrix and call) into `look`;
-// waits for the stream.
+// Looks at the rows of every system of a fitting size (once per matrix and call) into
+// `look`; waits for the stream if there is one.
 int batch_teams_look(pm_workspace* ws, const BatchTeams& b, std::vector<BatchLook>& look, hipStream_t stream);
 // Solves every system that fits, committing x, its state and the stopped
-// count; the others are left as they are.  Stream-ordered.
-int batch_teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook>& look, hipStream_t stream);
+// count; the others are left as they are.  *ran: there was one.  Waits for the stream.
+int batch_teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook>& look, hipStream_t stream,
+                    bool* ran);
 
 } // namespace pm

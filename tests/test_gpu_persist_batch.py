@@ -208,3 +208,32 @@ def test_exchange_tags_start_again(dev, monkeypatch):
         assert ws.solver_one_launch == 1
         out.append(([(r.converged, r.iterations) for r in reps], x.cpu().numpy().tobytes()))
     assert out[0] == out[1] == out[2]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_systems_past_a_team(dev, monkeypatch, dtype):
+    # more rows than 64 workgroups hold (FP32 262,144, FP64 131,072), rows too long or a
+    # column of another system in the last chunk of many: the kernels, bit for bit; the
+    # systems beside them in teams
+    lap = generators.laplacian2d_csr
+    hosts = [lap(520, 510), lap(60, 60), lap(410, 330), long_rows(60, 1), lap(257, 256), lap(50, 50)]
+    hosts = [generators.CSRHost(h.rows, h.cols, h.row_offsets, h.col_indices, h.values.astype(dtype)) for h in hosts]
+    h, begin, end = generators.block_diagonal(hosts, dtype=dtype)
+    far = h.row_offsets[int(end[4])] - 1  # the last entry of the fifth system
+    h.col_indices[far] = int(begin[5]) + 3
+    h.values[far] = 0.0
+    a = capi.to_device_csr(h, compact=True)
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=5).astype(dtype)).to(dev)
+    out = {}
+    for flag in ("0", "1"):
+        monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+        ws, x = capi.Workspace(), torch.zeros_like(b)
+        reps = capi.batch_pcg(a, begin, end, b, x, ws, relative_tolerance=1e-30, max_iterations=30)
+        torch.cuda.synchronize()
+        out[flag] = [(r.iterations, r.final_residual, x[s:e].cpu().numpy()) for r, s, e in zip(reps, begin, end)]
+        assert ws.solver_one_launch == int(flag)
+    for i, (p, q) in enumerate(zip(out["0"], out["1"])):
+        same = p[0] == q[0] and p[1] == q[1] and np.array_equal(p[2], q[2])
+        kernels = i in (0, 3, 4) or (i == 2 and dtype == np.float64)
+        assert same or not kernels, i
+        assert np.linalg.norm(p[2] - q[2]) <= (1e-3 if dtype == np.float32 else 1e-10) * np.linalg.norm(p[2]), i
