@@ -11,8 +11,11 @@
 // sums per iteration as tagged 64-bit words (persist.hip), every workgroup of it
 // decides alike, and teams never wait for each other, so a stopped system frees
 // its CUs' bandwidth at once.  Teams that do not fit the chip together run in
-// successive launches, largest systems first, so that a launch's systems are of
-// like length.
+// successive cooperative launches, largest systems first, so that a launch's systems
+// are of like length; the one-workgroup systems past the last of them wait for nobody
+// and run in one ordinary launch (in cooperative ones of 256, each 130 us before its
+// first iteration, 2,048 systems of 1,000 FP32 rows took 2.93 ms for 100 iterations;
+// now 2.11, in the kernels 7.5).
 //
 // The iteration is that of the per-kernel batch (BatchState::advance); its dot
 // products are summed per workgroup and then per team instead of per 64-row
@@ -66,6 +69,7 @@ struct TeamArgs
     const S *p, *r, *s, *w;
     const S* inv;
     const BatchState* st;
+    const TeamTask* tasks;
     TeamControl* ctl;
     PersistControl* give_up;  // its abort notice alone is used: TeamControl starts with it
     word* xu;                 // [slot][row of the piece]
@@ -74,6 +78,8 @@ struct TeamArgs
     unsigned tag;
     int32_t max_iterations;
     int refresh;
+    BatchState* end;                 // teams of one workgroup: the states and the count of stopped
+    unsigned long long* done_count;  // systems, which they write themselves (null: k_team_states)
 };
 
 template <typename S, typename I, int R>
@@ -89,7 +95,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_batch_team(TeamArgs<S, I> a
     __shared__ int sh_code, sh_fail;
 
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    const TeamTask job = a.ctl->tasks[blockIdx.x];
+    const TeamTask job = a.tasks[blockIdx.x];
     const int H = job.team > 1 ? job.halo : 0;
     const int first = job.piece * kPiece;  // the piece's first row of the system
     const int size = job.rows - first < kPiece ? job.rows - first : kPiece;
@@ -285,12 +291,17 @@ __global__ __launch_bounds__(kPersistThreads) void k_batch_team(TeamArgs<S, I> a
         const int l = k * kPersistThreads + tid;
         if (l < size) a.x_out[job.begin + first + l] = x[k];
     }
-    if (tid == 0 && job.piece == 0)
+    BatchState end = state;
+    end.done = sh_code;
+    if (a.end != nullptr)
     {
-        BatchState end = state;
-        end.done = sh_code;
-        a.ctl->out[job.slot0] = end;
+        // no workgroup but this one can fail the system
+        if (tid != 0 || a.st[job.system].done != kRunning) return;  // stopped before the launch, and counted then
+        a.end[job.system] = end;
+        atomicAdd(a.done_count, 1ull);
+        return;
     }
+    if (tid == 0 && job.piece == 0) a.ctl->out[job.slot0] = end;
     __syncthreads();
     if (tid == 0)
         __hip_atomic_fetch_add(&a.ctl->finished[job.slot0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -334,8 +345,8 @@ __global__ void k_team_reset(TeamControl* ctl, const TeamControl* before, unsign
 // The band of every system of short rows, kNoBand for the others: rows too long, a
 // column outside the system, or more than `largest` rows.  A wavefront takes
 // consecutive 64-row chunks and tells a system's value once per run of its chunks
-// (once per chunk, 24,752 chunks of 8 systems waited 0.55 ms for the one cache line;
-// now DDD us).
+// (once per chunk, 24,752 chunks of 8 systems met on one cache line: five iterations of
+// eight 198,000-row FP32 systems 1.02 ms, now 0.49).
 constexpr int kNoBand = 0x7fffffff;
 constexpr int kLookWaves = 2048;
 template <typename I>
@@ -406,6 +417,28 @@ const void* team_kernel(int rows_per_lane)
     return nullptr;
 }
 
+// Systems below kTinyBytes of a vector leave most lanes of a workgroup idle: more than
+// kTinyRounds of them for every CU take the kernels.  60 iterations of FP32 systems,
+// kernels / a workgroup each: 1,024 of 64 rows 1.17 / 0.87 ms, 2,048 of 128 rows 1.67 /
+// 2.20, 8,192 of 64 rows 4.6 / 8.4, 2,048 of 256 rows 2.16 / 1.56; FP64, 8,192 of 64
+// rows 4.7 / 7.2, of 128 rows 6.24 / 6.09.
+constexpr int64_t kTinyBytes = 1024;
+constexpr int64_t kTinyRounds = 4;
+
+// Rows of a system that teams take, at least.
+int64_t least_rows(const BatchTeams& b, int es, int slots)
+{
+    int64_t tiny = 0;
+    for (int64_t s = 0; s < b.systems; ++s) tiny += (b.end[s] - b.begin[s]) * es < kTinyBytes;
+    return tiny > kTinyRounds * slots ? kTinyBytes / es : 1;
+}
+
+// The tasks of one-workgroup systems, behind the looks.
+size_t team_tasks_offset(int64_t systems)
+{
+    return (sizeof(BatchLook) * static_cast<size_t>(systems) + 255) & ~size_t(255);
+}
+
 // Rows per lane that the registers hold.
 template <typename S>
 constexpr int team_rows()
@@ -433,6 +466,7 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
     const int es = static_cast<int>(sizeof(S));
     int slots = 0;
     PM_TRY(team_slots(ws, b, &slots));
+    const int64_t least = least_rows(b, es, slots);
     std::vector<int> order;
     int64_t total[3] = {0, 0, 0};  // workgroups with 1, 2, 4 rows per lane
     for (int64_t s = 0; s < b.systems; ++s)
@@ -441,7 +475,7 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         const BatchLook& l = look[static_cast<size_t>(s)];
         const int64_t piece = static_cast<int64_t>(most) * kPersistThreads;
         const int64_t team = ceil_div(n, piece);
-        if (n <= 0 || b.skip[s] || l.band == kNoBand || team > std::min(kTeamLargest, slots)) continue;
+        if (n < least || b.skip[s] || l.band == kNoBand || team > std::min(kTeamLargest, slots)) continue;
         if (team > 1 && (team_lds(es, most, l.band) > kTeamLds || piece + 2 * static_cast<int64_t>(l.band) > 65535)) continue;
         order.push_back(static_cast<int>(s));
         for (int k = 0; k < 3; ++k) total[k] += ceil_div(n, static_cast<int64_t>(kPersistThreads) << k);
@@ -468,9 +502,10 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
     const int64_t piece = static_cast<int64_t>(rows_per_lane) * kPersistThreads;
     std::stable_sort(order.begin(), order.end(),
                      [&](int l, int r) { return b.end[l] - b.begin[l] > b.end[r] - b.begin[r]; });
-    // launches of at most `slots` workgroups
+    // launches of at most `slots` workgroups, which run together
     std::vector<std::vector<TeamTask>> launches;
     std::vector<TeamTask> now;
+    const bool together = total[rows_per_lane / 2] <= slots;
     auto add = [&](int s) {
         const int64_t n = b.end[s] - b.begin[s];
         const int team = static_cast<int>(ceil_div(n, piece));
@@ -480,19 +515,32 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
             now.push_back(TeamTask{s, slot0, team, q, static_cast<int32_t>(n), look[static_cast<size_t>(s)].band, b.begin[s]});
         return true;
     };
-    for (int s : order)
+    // ... up to the last one with a system of several workgroups; the smaller systems
+    // that it has no room for wait for nobody
+    size_t at = 0;
+    for (; at < order.size(); ++at)
     {
-        if (add(s)) continue;
-        launches.push_back(std::move(now));
+        const int64_t n = b.end[order[at]] - b.begin[order[at]];
+        if ((together || n > piece || !now.empty()) && add(order[at])) continue;
+        if (!now.empty()) launches.push_back(std::move(now));
         now.clear();
-        (void)add(s);
+        if (n <= piece) break;
+        (void)add(order[at]);
     }
     if (!now.empty()) launches.push_back(std::move(now));
+    std::vector<TeamTask> alone[3];  // by 1, 2, 4 rows per lane
+    for (; at < order.size(); ++at)
+    {
+        const int s = order[at];
+        const int64_t n = b.end[s] - b.begin[s];
+        const int k = n <= kPersistThreads ? 0 : n <= 2 * kPersistThreads ? 1 : 2;
+        alone[k].push_back(TeamTask{s, 0, 1, 0, static_cast<int32_t>(n), 0, b.begin[s]});
+    }
 
     const size_t words = static_cast<size_t>(slots) * static_cast<size_t>(piece);
     const size_t plane_words = words * Exchange<S>::kWords;
     const size_t control = (sizeof(TeamControl) + 255) & ~size_t(255);
-    const size_t control_all = control * launches.size();
+    const size_t control_all = control * std::max<size_t>(launches.size(), 1);
     // the control blocks come after the words, whose places then only ever hold words
     const size_t need = 2 * plane_words * sizeof(word) + control_all;
     // (blocks in a place that earlier held words, or the other way round, are
@@ -552,6 +600,7 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         for (const TeamTask& t : launches[k]) halo = std::max(halo, t.team > 1 ? t.halo : 0);
         const size_t lds = team_lds(es, rows_per_lane, halo);
         PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        a.tasks = ctl->tasks;
         a.ctl = ctl;
         a.give_up = reinterpret_cast<PersistControl*>(ctl);
         a.tag = ws->teams_tag;
@@ -574,7 +623,26 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
                            gave_up);
         PM_HIP(hipGetLastError());
     }
-    // the launches vector is the source of the copies above
+    a.ctl = reinterpret_cast<TeamControl*>(blocks0);
+    a.give_up = reinterpret_cast<PersistControl*>(a.ctl);
+    a.x_out = static_cast<S*>(b.x);
+    a.end = b.st;
+    a.done_count = b.done_count;
+    auto* tasks = reinterpret_cast<TeamTask*>(ws->looks.as<char>() + team_tasks_offset(b.systems));
+    for (int k = 0; k < 3; ++k)
+    {
+        if (alone[k].empty()) continue;
+        PM_HIP(hipMemcpyAsync(tasks, alone[k].data(), sizeof(TeamTask) * alone[k].size(), hipMemcpyHostToDevice, stream));
+        hipLaunchKernelGGL(k_team_reset, dim3(1), dim3(kTeamSlots), 0, stream, a.ctl, nullptr, 0u);
+        a.tasks = tasks;
+        tasks += alone[k].size();
+        const void* one = team_kernel<S, I>(1 << k);
+        const size_t lds = team_lds(es, 1 << k, 0);
+        PM_HIP(hipFuncSetAttribute(one, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        void* args[] = {&a};
+        PM_HIP(hipLaunchKernel(one, dim3(static_cast<unsigned>(alone[k].size())), dim3(kPersistThreads), args, lds, stream));
+    }
+    // the vectors of tasks are the sources of the copies above
     PM_HIP(hipStreamSynchronize(stream));
     if (*gave_up != 0u)
     {
@@ -593,10 +661,12 @@ int batch_teams_look(pm_workspace* ws, const BatchTeams& b, std::vector<BatchLoo
     PM_TRY(team_slots(ws, b, &slots));
     const int64_t piece = static_cast<int64_t>(b.a->dtype == PM_F64 ? team_rows<double>() : team_rows<float>()) * kPersistThreads;
     const int64_t largest = piece * std::min(kTeamLargest, slots);
+    const int64_t least = least_rows(b, b.a->dtype == PM_F64 ? 8 : 4, slots);
     bool any = false;
-    for (int64_t s = 0; s < b.systems && !any; ++s) any = !b.skip[s] && b.end[s] > b.begin[s] && b.end[s] - b.begin[s] <= largest;
+    for (int64_t s = 0; s < b.systems && !any; ++s)
+        any = !b.skip[s] && b.end[s] - b.begin[s] >= least && b.end[s] - b.begin[s] <= largest;
     if (!any || b.chunks == 0) return PM_OK;
-    if (!persist_storage(ws->looks, sizeof(BatchLook) * static_cast<size_t>(b.systems)))
+    if (!persist_storage(ws->looks, team_tasks_offset(b.systems) + sizeof(TeamTask) * static_cast<size_t>(b.systems)))
     {
         ws->last_one_launch = -1;
         return PM_OK;

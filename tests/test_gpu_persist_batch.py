@@ -44,6 +44,8 @@ def members(kind):
                 lap(17, 241), long_rows(60, 1), diag_system(63)]
     if kind == "teams":  # halos narrower and wider than a piece
         return [lap(150, 90), box(25, 24, 23, seed=1), lap(40, 400), box(60, 50, 4, seed=2), lap(3000, 5)]
+    if kind == "alone":  # more workgroups than CUs, most of the systems one workgroup each with 1, 2 or 4 rows per lane
+        return [lap(150, 140)] * 45 + [lap(64, 64), lap(60, 68), lap(45, 45), lap(32, 32), lap(20, 20), diag_system(5)] * 20
     # more workgroups than CUs at any rows per lane: several launches
     return [lap(150, 140 + i % 7) for i in range(60)] + [box(30, 30, 30, seed=i) for i in range(6)]
 
@@ -55,7 +57,7 @@ def batch(kind, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("kind", ["edges", "teams", "launches"])
+@pytest.mark.parametrize("kind", ["edges", "teams", "launches", "alone"])
 def test_teams_match_the_per_kernel_batch(dev, monkeypatch, kind, dtype):
     h, begin, end = batch(kind, dtype)
     rel, bound = (1e-10, 1e-6) if dtype == np.float64 else (1e-5, 1e-2)
@@ -237,3 +239,26 @@ def test_systems_past_a_team(dev, monkeypatch, dtype):
         kernels = i in (0, 3, 4) or (i == 2 and dtype == np.float64)
         assert same or not kernels, i
         assert np.linalg.norm(p[2] - q[2]) <= (1e-3 if dtype == np.float32 else 1e-10) * np.linalg.norm(p[2]), i
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_many_tiny_systems_take_the_kernels(dev, monkeypatch, dtype):
+    # below 1 KB of a vector and more than four for every CU; the larger ones beside them
+    # get a workgroup each
+    lap = generators.laplacian2d_csr
+    hosts = [lap(6, 5, dtype=dtype)] * 1100 + [lap(32, 31, dtype=dtype), lap(16, 16, dtype=dtype), lap(70, 70, dtype=dtype)]
+    h, begin, end = generators.block_diagonal(hosts, dtype=dtype)
+    a = capi.to_device_csr(h, compact=True)
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=5).astype(dtype)).to(dev)
+    out = {}
+    for flag in ("0", "1"):
+        monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+        ws, x = capi.Workspace(), torch.zeros_like(b)
+        reps = capi.batch_pcg(a, begin, end, b, x, ws, relative_tolerance=1e-4, max_iterations=400)
+        torch.cuda.synchronize()
+        assert all(r.converged for r in reps) and ws.solver_one_launch == int(flag)
+        out[flag] = [r.iterations for r in reps], x.cpu().numpy()
+    assert out["0"][0][:1100] == out["1"][0][:1100]
+    assert np.array_equal(out["0"][1][:1100 * 64], out["1"][1][:1100 * 64])
+    x0, x1 = (out[f][1][int(begin[1100]):].astype(np.float64) for f in ("0", "1"))
+    assert np.linalg.norm(x0 - x1) <= 1e-1 * np.linalg.norm(x0)  # 1e-4 times a condition below 1e3
