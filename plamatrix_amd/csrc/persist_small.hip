@@ -32,6 +32,13 @@ constexpr int64_t kSmallRows = 4096;                  // four rows per lane
 // entries beyond the registers come from the L2 at about 64 bytes per clock of
 // the one CU: 32,768 entries of 16 bytes take as long as the two kernels
 constexpr int64_t kSmallEntries = 32768;
+// FP64 with four rows per lane spills (108 to 137 registers of a lane): 3 entries a row
+// on average 12.6 us per iteration in the two kernels against 10.4 here (4,000 rows,
+// scattered columns), 5 entries 13.3 against 14.0, 7 entries 13.7 against 16.9.  A
+// 5-point stencil (7.9 here at 2,116 rows, 8.0 at 4,096) takes 5.8 with a row per lane
+// (persist_csr.hip).
+constexpr int64_t kSmallSpillRows = 2048;
+constexpr int64_t kSmallSpillEntries = 4;  // a row
 constexpr int64_t kSmallSegment = 65536;              // iterations per launch
 constexpr unsigned kSmallDone = 1, kSmallUnsupported = 2;
 
@@ -315,8 +322,9 @@ bool persist_small_wanted(const PersistProblem& p)
 {
     // one row per lane and slot: the per-kernel workgroups hold at most four
     // chunks of 64 rows
+    const bool spills = p.dtype == PM_F64 && p.rows > kSmallSpillRows;
     return persist_enabled() && p.rows > 0 && p.rows <= kSmallRows && p.a->nnz <= kSmallEntries &&
-           p.count <= 4 * kSmallGroups && ceil_div(chunk_count(p.rows), static_cast<int64_t>(p.count)) <= kWavesPerBlock;
+           (!spills || p.a->nnz <= kSmallSpillEntries * p.rows) && p.count <= 4 * kSmallGroups && ceil_div(chunk_count(p.rows), static_cast<int64_t>(p.count)) <= kWavesPerBlock;
 }
 
 int persist_small_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iterations, hipStream_t stream,

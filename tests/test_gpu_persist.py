@@ -423,3 +423,43 @@ def test_hand_over_after_several_launches(dev, monkeypatch, dims):
             torch.cuda.synchronize()
             out.append(got + (x.cpu().numpy().tobytes(),))
         assert out[0] == out[1], shift
+
+
+def scattered(n, k, dtype):
+    """SPD, 2 k + 1 entries a row on average, their columns anywhere."""
+    import scipy.sparse as sp
+
+    rng = np.random.default_rng(n + k)
+    i = np.repeat(np.arange(n), k)
+    m = sp.csr_matrix((-rng.random(len(i)) - 0.1, (i, (i + 1 + rng.integers(0, n - 1, len(i))) % n)), shape=(n, n))
+    m = m + m.T
+    m = (m + sp.diags(np.asarray(abs(m).sum(axis=1)).ravel() + 0.1)).tocsr()
+    m.sort_indices()
+    return generators.CSRHost(n, n, m.indptr.astype(np.int64), m.indices.astype(np.int64), m.data.astype(dtype))
+
+
+# (matrix, whether one launch takes it): FP64 over 2,048 rows in one workgroup up to four
+# entries a row, above that with a row per lane if the columns are near
+BESIDE = [
+    (scattered(2048, 3, np.float64), 1), (scattered(2049, 3, np.float64), 0), (scattered(2049, 1, np.float64), 1),
+    (scattered(4096, 1, np.float64), 1), (scattered(4096, 3, np.float32), 1), (generators.laplacian2d_csr(2049, 1), 1),
+    (generators.laplacian2d_csr(46, 45), 1), (generators.laplacian2d_csr(64, 64), 1),
+]
+
+
+@pytest.mark.parametrize("index", range(len(BESIDE)))
+def test_one_workgroup_sizes(dev, monkeypatch, index):
+    h, one = BESIDE[index]
+    b = torch.from_numpy(generators.rhs_normal(h.rows, seed=43).astype(h.values.dtype)).to(dev)
+    rel = 1e-10 if h.values.dtype == np.float64 else 1e-5
+    for compact, solver in ((True, capi.pcg), (False, capi.cg)):
+        a = capi.to_device_csr(h, compact=compact)
+        out = {}
+        for flag in ("0", "1"):
+            monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", flag)
+            ws, x = capi.Workspace(), torch.full_like(b, 0.25)
+            rep = solver(a, b, x, ws, capi.policy(refresh_interval=20), relative_tolerance=rel, max_iterations=500)
+            torch.cuda.synchronize()
+            assert ws.solver_one_launch == (one if flag == "1" else 0)
+            out[flag] = rep.converged, rep.iterations, rep.final_residual, x.cpu().numpy().tobytes()
+        assert out["0"] == out["1"]
