@@ -28,3 +28,10 @@ def ref_lib():
     if not _oracle.ref_available():
         pytest.skip("reference CPU build (oracle/_ref) not built on this host")
     return _oracle
+
+
+@pytest.fixture(params=["1", "0"], ids=["one_launch", "kernels"])
+def persistent(request, monkeypatch):
+    """With the solves that fit in one launch, and with their kernels, which serve the
+    sizes beyond it and a launch that is refused or gives up."""
+    monkeypatch.setenv("PLAMATRIX_AMD_PERSISTENT", request.param)

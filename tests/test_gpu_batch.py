@@ -9,7 +9,7 @@ bad diagonal, zero right-hand side) are per system.
 import numpy as np
 import pytest
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("persistent")]
 
 torch = pytest.importorskip("torch")
 

@@ -11,7 +11,7 @@ layout does not fit (unsorted rows, too many diagonals) fall back to CSR.
 import numpy as np
 import pytest
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("persistent")]
 
 torch = pytest.importorskip("torch")
 
@@ -342,7 +342,8 @@ def test_restart_hands_over_identically(dev, monkeypatch, shift):
     # after its chunks in flight the solve continues in the three-kernel form
     # from the vectors the one-kernel iteration left in its first buffers,
     # which reports the breakdown (at iteration 21; the three-kernel form alone
-    # stops at 2); one and two kernels per iteration must end identically
+    # stops at 2); one and two kernels per iteration must end identically, and
+    # the one launch of test_gpu_persist.py's form like the two kernels
     import scipy.sparse as sp
 
     h = generators.laplacian2d_csr(300, dtype=np.float64)

@@ -210,6 +210,7 @@ def test_loss_and_gradient_match_oracle(dev):
         assert abs(grad[k] - ref_grad[k]) <= 1e-2 * abs(ref_grad[k]) + 1e-6, (k, grad[k], ref_grad[k])
 
 
+@pytest.mark.usefixtures("persistent")
 def test_factored_pcg_matches_oracle(dev, ws):
     h = system(10, 9, 8, seed=10, dtype=np.float64)
     a = capi.to_device_csr(h, compact=True)
@@ -272,6 +273,7 @@ def trained_factors(h):
     return a, graph
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("refresh", [0, 20])
 def test_factored_single_reduction_matches_oracle(dev, refresh):
     # A, G and G^T on the diagonal layout (76,800 rows): the factored PCG runs
@@ -302,6 +304,7 @@ def test_factored_single_reduction_matches_oracle(dev, refresh):
     assert capi.true_relres(a, b, x, w) <= 1e-9
 
 
+@pytest.mark.usefixtures("persistent")
 def test_factored_single_reduction_keeps_fp32_iterations(dev, monkeypatch):
     # FP32 with residual refreshes: the single-reduction factored iteration
     # ends within 3 % of the classic form's iteration count at the same
@@ -325,6 +328,7 @@ def test_factored_single_reduction_keeps_fp32_iterations(dev, monkeypatch):
     assert t1 <= 5e-5 and t0 <= 5e-5, (t0, t1)
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_factored_pair_kernel_is_bitwise(dev, monkeypatch, dtype):
     # G r and G^T t in one kernel (each t of the four rows holding column i
@@ -348,6 +352,7 @@ def test_factored_pair_kernel_is_bitwise(dev, monkeypatch, dtype):
     assert np.array_equal(x0, x1)
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("dims", [2, 3])
 def test_factored_single_reduction_restart_hands_over(dev, monkeypatch, dims):
     # an indefinite matrix (Laplacian minus a shift that leaves a diagonal of

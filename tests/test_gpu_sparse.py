@@ -270,6 +270,7 @@ def poisson1d(oracle, n, dtype=np.float64, scale=1.0):
     return oracle.coo_to_csr(n, n, rows, cols, np.array(vals, dtype))
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("graph", [0, 1])
 def test_adaptive_matches_cpu(dev, ws, oracle, dtype, graph):
@@ -309,6 +310,7 @@ def test_block_pcg_one_iteration(dev, ws, oracle, dtype):
     np.testing.assert_allclose(host(x), expected, atol=2e-4 if dtype == np.float32 else 1e-10)
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_zero_iterations_and_nonconvergence(dev, ws, oracle, dtype):
     # iterative_solver_test.cpp:426-461
@@ -328,6 +330,7 @@ def test_zero_iterations_and_nonconvergence(dev, ws, oracle, dtype):
     assert kinds(e) == "runtime_error"
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_workspace_resize_planned_sizes(dev, oracle, dtype):
     # iterative_solver_test.cpp:463-495
@@ -343,6 +346,7 @@ def test_workspace_resize_planned_sizes(dev, oracle, dtype):
         assert ws.capacity_rows == n
 
 
+@pytest.mark.usefixtures("persistent")
 def test_disabled_jacobi(dev, ws, oracle):
     # iterative_solver_test.cpp:497-519
     m = oracle.coo_to_csr(3, 3, [0, 1, 2], [0, 1, 2], np.array([2.0, 4.0, 8.0]))
@@ -352,6 +356,7 @@ def test_disabled_jacobi(dev, ws, oracle):
     assert not rep.converged and rep.iterations == 1 and rep.final_residual > 0
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_breakdown_leaves_solution_untouched(dev, ws, oracle, dtype):
     # iterative_solver_test.cpp:521-560
@@ -370,6 +375,7 @@ def test_breakdown_leaves_solution_untouched(dev, ws, oracle, dtype):
     assert host(x1)[0] == 0
 
 
+@pytest.mark.usefixtures("persistent")
 def test_jacobi_rejects_bad_diagonal(dev, ws, oracle):
     for vals, cols in (([1.0, 1.0], [1, 0]), ([1.0, 0.0], [0, 1])):
         m = oracle.coo_to_csr(2, 2, [0, 1], cols, np.array(vals))
@@ -399,6 +405,7 @@ def test_fixed_iterations_closed_form(dev, ws, oracle, dtype):
     assert np.all(np.abs(host(x) - expected) <= tol * expected)
 
 
+@pytest.mark.usefixtures("persistent")
 def test_c0_poisson_fp64_parity(dev, ws, oracle):
     """2-D Poisson 256^2 from shuffled COO with split duplicates: device
     COO->CSR then Jacobi-PCG to rel 1e-8 (max 2000) against the CPU solve."""
@@ -418,6 +425,7 @@ def test_c0_poisson_fp64_parity(dev, ws, oracle):
     assert abs(relres - oracle.true_relres(ref, b, gx)) <= 1e-12
 
 
+@pytest.mark.usefixtures("persistent")
 def test_solve_is_deterministic_and_graph_equals_direct(dev, ws, oracle):
     h = generators.diffusion3d_csr(24, seed=5)
     a = capi.to_device_csr(h, compact=True)
@@ -432,6 +440,7 @@ def test_solve_is_deterministic_and_graph_equals_direct(dev, ws, oracle):
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][1], out[2][1])
 
 
+@pytest.mark.usefixtures("persistent")
 def test_fp32_pcg_matches_cpu_within_1e4(dev, ws, oracle):
     h = generators.diffusion3d_csr(32, seed=12)
     b = generators.rhs_normal(h.rows, seed=13)
@@ -446,6 +455,7 @@ def test_fp32_pcg_matches_cpu_within_1e4(dev, ws, oracle):
     assert oracle.true_relres(ref, b, gx) <= 5e-6
 
 
+@pytest.mark.usefixtures("persistent")
 def test_refinement_reaches_1e8(dev, ws, oracle):
     h = generators.diffusion3d_csr(32, seed=22)
     b = generators.rhs_normal(h.rows, seed=23).astype(np.float64)
@@ -554,6 +564,7 @@ def test_spmm_diffusion3d_full_size_eight_columns(dev, ws):
         assert torch.equal(y[j], yj), j
 
 
+@pytest.mark.usefixtures("persistent")
 @pytest.mark.parametrize("dims", [(40, 40, 40), (48, 48, 48)])
 def test_single_reduction_keeps_iteration_count_on_ill_conditioned_refresh(dev, monkeypatch, dims):
     # FP32 Jacobi-PCG with a residual refresh every 50 iterations on a badly
