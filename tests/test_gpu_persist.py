@@ -463,3 +463,31 @@ def test_one_workgroup_sizes(dev, monkeypatch, index):
             assert ws.solver_one_launch == (one if flag == "1" else 0)
             out[flag] = rep.converged, rep.iterations, rep.final_residual, x.cpu().numpy().tobytes()
         assert out["0"] == out["1"]
+
+
+@pytest.mark.parametrize("forms", [("dia", "csr"), ("dia", "dia"), ("factored", "dia"), ("csr", "factored"), ("small", "dia")])
+def test_two_solves_at_once(dev, forms):
+    # two threads, each with its stream and workspace: launches of both may be queued
+    # together, and neither waits for the other's workgroups
+    import threading
+
+    runs = [form_solve(form, dev) for form in forms]
+    refs = [run(capi.Workspace()) for run in runs]
+    torch.cuda.synchronize()
+    got = [[], []]
+
+    def work(k):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            ws = capi.Workspace()
+            for _ in range(6):
+                out = runs[k](ws)
+                got[k].append((out == refs[k], ws.solver_one_launch))
+            stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert got == [[(True, 1)] * 6] * 2
