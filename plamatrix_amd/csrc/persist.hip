@@ -6,8 +6,10 @@
 // iteration, all latency; 2.1 M rows: 27.9 us for 113 MB).  Here a workgroup
 // keeps its rows for the whole solve: p, s, x, r, w and the rows' matrix values
 // live in registers (the chip's register files hold 128 MB), with a few words
-// per row in LDS for the largest systems.  Per iteration only u crosses
-// workgroups, and one reduction.
+// per row in LDS for the largest systems.  Those with 32 bytes of a vector per lane
+// (eight FP32 rows, four FP64) do not fit the 128 registers of a lane: 20 to 170 spill,
+// which bounds their iteration and still costs less than the kernels (below).  Per
+// iteration only u crosses workgroups, and one reduction.
 //
 // Work split.  The per-kernel iteration sums its dot products in `count`
 // workgroups of four wavefronts over contiguous 64-row chunks; a workgroup here
@@ -36,6 +38,19 @@
 // (767 iterations, one row per lane) 7.50 / 3.90 ms, 5.0 us per iteration, two
 // exchange latencies; 2,097,152-row FP32 3-D diffusion (753 iterations, eight
 // rows per lane) 21.2 / 15.2 ms with refinement, 18.6 us per iteration.
+//
+// us per iteration of 200-iteration solves, per-kernel / persistent, by diagonals and
+// rows per lane (U: unit diagonal, J: Jacobi):
+//   5 FP64 J   1: 262 k rows 21.3 / 8.3    2: 504 k 24.7 / 9.4    4: 1.04 M 34.2 / 12.7
+//   7 FP64 U   1: 216 k 19.7 / 8.4         2: 493 k 23.1 / 12.4   4: not in LDS
+//   7 FP64 J   1: 216 k 24.3 / 9.1         2: 493 k 28.5 / 13.5
+//   5 FP32 J   2: 303 k 14.4 / 8.3         4: 1.0 M 20.8 / 9.9    8: 1.99 M 36.6 / 12.5
+//   5 FP32 U   2: 303 k 11.8 / 7.3         4: 1.0 M 15.7 / 8.4    8: 1.99 M 27.4 / 10.3
+//   7 FP32 J   2: 493 k 19.2 / 9.8         4: 1.0 M 26.1 / 12.1   8: 1.12 M 28.9 / 20.4, 2.1 M 38.2 / 21.9
+//   7 FP32 U   2: 493 k 13.4 / 8.8         4: 1.0 M 17.7 / 10.7   8: 1.12 M 19.8 / 17.7, 2.1 M 28.0 / 20.9
+// A launch costs more before its first iteration; solves of six iterations still gain up
+// to four rows per lane (7 FP32 U 1.0 M: 356 / 327 us), with eight they are level (7 FP32
+// U 384 / 386 us at 1.12 M rows, 463 / 490 at 2.0 M; J 699 / 650).
 #include "persist.hpp"
 
 #include <algorithm>
@@ -228,7 +243,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
             const int i = base + q;
             if (h >= 2 * H || size == 0 || i < 0 || i >= rows) continue;
             word hw[X::kWords];
-            fine = fine && wait_for(a.ctl, [&] {
+            fine = fine && wait_for(&a.ctl->abort, [&] {
                        X::issue(buf, rows, i, hw);
                        return ready<S>(hw, tag);
                    });
@@ -241,7 +256,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cg_persist(PersistArgs<S> a
             if constexpr (FAR)
             {
                 if (!__all(arrived()))
-                    fine = fine && wait_for(a.ctl, [&] {
+                    fine = fine && wait_for(&a.ctl->abort, [&] {
                                issue(kb);
                                return arrived();
                            });
@@ -362,8 +377,6 @@ struct PersistShape
     size_t lds;
 };
 
-constexpr size_t kPersistLds = 160 * 1024 - 2048;  // LDS of a CU less the static part
-
 bool persist_shape(const PersistProblem& p, PersistShape* out)
 {
     const DiaLayout& d = *p.dia;
@@ -475,8 +488,7 @@ int persist_run_t(pm_workspace* ws, const PersistProblem& p, int64_t max_iterati
     a.priv = static_cast<int>(shape.shared);
     a.red = static_cast<int>(shape.red);
     a.span = shape.span;
-    // every workgroup decides for itself, or eight decide and answer the rest
-    a.leaders = shape.blocks <= 64 ? shape.blocks : kXcds;
+    a.leaders = persist_leaders(shape.blocks);
     a.refresh = p.refresh;
     a.chunk = p.chunk;
     a.grow = p.grow ? 1 : 0;

@@ -71,7 +71,6 @@ struct TeamArgs
     const BatchState* st;
     const TeamTask* tasks;
     TeamControl* ctl;
-    PersistControl* give_up;  // its abort notice alone is used: TeamControl starts with it
     word* xu;                 // [slot][row of the piece]
     word* xx;
     int plane;                // words of a half plane
@@ -166,7 +165,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_batch_team(TeamArgs<S, I> a
             const int i = first + q;
             if (h >= 2 * H || i < 0 || i >= job.rows) continue;
             word hw[X::kWords];
-            fine = wait_for(a.give_up, [&] {
+            fine = wait_for(&a.ctl->abort, [&] {
                        X::issue(buf, a.plane, words0 + i, hw);
                        return ready<S>(hw, tag);
                    }) && fine;
@@ -253,7 +252,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_batch_team(TeamArgs<S, I> a
                 {
                     const word* from = &a.ctl->part[t & 1][0][0][job.slot0 + lane];
                     word hw[kCgValues][2];
-                    fine = wait_for(a.give_up, [&] {
+                    fine = wait_for(&a.ctl->abort, [&] {
                         bool ok = true;
 #pragma unroll
                         for (int q = 0; q < kCgValues; ++q)
@@ -406,8 +405,6 @@ size_t team_lds(int es, int rows_per_lane, int halo)
     return static_cast<size_t>(es) * (static_cast<size_t>(rows_per_lane) * kPersistThreads + 2 * static_cast<size_t>(halo));
 }
 
-constexpr size_t kTeamLds = 160 * 1024 - 2048;  // LDS of a CU less the static part
-
 template <typename S, typename I>
 const void* team_kernel(int rows_per_lane)
 {
@@ -476,7 +473,7 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         const int64_t piece = static_cast<int64_t>(most) * kPersistThreads;
         const int64_t team = ceil_div(n, piece);
         if (n < least || b.skip[s] || l.band == kNoBand || team > std::min(kTeamLargest, slots)) continue;
-        if (team > 1 && (team_lds(es, most, l.band) > kTeamLds || piece + 2 * static_cast<int64_t>(l.band) > 65535)) continue;
+        if (team > 1 && (team_lds(es, most, l.band) > kPersistLds || piece + 2 * static_cast<int64_t>(l.band) > 65535)) continue;
         order.push_back(static_cast<int>(s));
         for (int k = 0; k < 3; ++k) total[k] += ceil_div(n, static_cast<int64_t>(kPersistThreads) << k);
     }
@@ -602,7 +599,6 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         a.tasks = ctl->tasks;
         a.ctl = ctl;
-        a.give_up = reinterpret_cast<PersistControl*>(ctl);
         a.tag = ws->teams_tag;
         ws->teams_tag += static_cast<uint32_t>(b.max_iterations) + 2u;
         hipLaunchKernelGGL(k_team_reset, dim3(1), dim3(kTeamSlots), 0, stream, ctl, before,
@@ -624,7 +620,6 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         PM_HIP(hipGetLastError());
     }
     a.ctl = reinterpret_cast<TeamControl*>(blocks0);
-    a.give_up = reinterpret_cast<PersistControl*>(a.ctl);
     a.x_out = static_cast<S*>(b.x);
     a.end = b.st;
     a.done_count = b.done_count;

@@ -18,6 +18,7 @@ constexpr int kRedEntries = kSolverGrid - kBlock;
 constexpr int kDecWords = 16;        // one 128-byte line per workgroup
 constexpr int kWaitSeconds = 4;
 constexpr int64_t kSegment = 8192;   // iterations per launch
+constexpr size_t kPersistLds = 160 * 1024 - 2048;  // LDS of a CU less the static part
 
 struct PersistControl
 {
@@ -105,9 +106,10 @@ __device__ __forceinline__ int physical_block(int lb, int nb)
 }
 
 // Waits for words that other workgroups write: `poll` loads them and says
-// whether all carry their tag.  The whole wavefront polls together.
+// whether all carry their tag.  The whole wavefront polls together.  `abort`: the
+// launch's notice to give up.
 template <typename Poll>
-__device__ __forceinline__ bool wait_for(PersistControl* ctl, Poll poll)
+__device__ __forceinline__ bool wait_for(unsigned* abort, Poll poll)
 {
     unsigned polls = 0;
     long long start = 0;
@@ -118,10 +120,10 @@ __device__ __forceinline__ bool wait_for(PersistControl* ctl, Poll poll)
         if ((++polls & 255u) != 0u) continue;
         const long long now = wall_clock64();
         if (start == 0) start = now;
-        if (__hip_atomic_load(&ctl->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ||
+        if (__hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ||
             now - start > kWaitSeconds * 100000000ll)
         {
-            __hip_atomic_store(&ctl->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return false;
         }
     }
@@ -178,7 +180,7 @@ __device__ __forceinline__ bool persist_decide(PersistShared<S>& sh, const Persi
             }
             word hw[NV][2];
             const word* from = &at.ctl->part[(t - 1) & 1][0][0][e];
-            fine = wait_for(at.ctl, [&] {
+            fine = wait_for(&at.ctl->abort, [&] {
                 bool ok = true;
 #pragma unroll
                 for (int v = 0; v < NV; ++v)
@@ -269,7 +271,7 @@ __device__ __forceinline__ bool persist_decide(PersistShared<S>& sh, const Persi
             // alpha, beta, code by lanes 0, 1, 2 (the other lanes repeat 2)
             const word* line = at.ctl->dec[at.bid] + (lane < 2 ? lane : 2);
             word hw[X::kWords];
-            const bool fine = wait_for(at.ctl, [&] {
+            const bool fine = wait_for(&at.ctl->abort, [&] {
                 hw[0] = load_word(line);
                 bool ok = word_ready(hw[0], tag);
                 if constexpr (X::kWords == 2)

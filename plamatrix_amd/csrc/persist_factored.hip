@@ -39,7 +39,6 @@ struct FactoredArgs
     int words;  // of one vector
     unsigned tag;
     int count, per, halo, leaders, refresh, t0, t_end, chunk, grow;
-    int span;    // local rows of a window
     int window;  // bytes of an LDS window, then the leaders' reduction after three
 };
 
@@ -166,7 +165,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cgf_persist(FactoredArgs<S>
             const int i = base + q;
             if (h >= 2 * H || size == 0 || i < 0 || i >= rows) continue;
             word hw[X::kWords];
-            fine = wait_for(a.ctl, [&] {
+            fine = wait_for(&a.ctl->abort, [&] {
                        X::issue(buf, rows, i, hw);
                        return ready<S>(hw, tag);
                    }) && fine;
@@ -176,7 +175,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_cgf_persist(FactoredArgs<S>
         if constexpr (FAR)
         {
             if (!__all(arrived()))
-                fine = wait_for(a.ctl, [&] {
+                fine = wait_for(&a.ctl->abort, [&] {
                            issue();
                            return arrived();
                        }) && fine;
@@ -281,8 +280,6 @@ struct FactoredShape
     size_t window, lds;
 };
 
-constexpr size_t kFactoredLds = 160 * 1024 - 2048;  // LDS of a CU less the static part
-
 bool factored_shape(const PersistProblem& p, FactoredShape* out)
 {
     const DiaArgs &d = p.dia->args, &l = p.dia_g->args, &u = p.dia_gt->args;
@@ -310,11 +307,11 @@ bool factored_shape(const PersistProblem& p, FactoredShape* out)
         return 3 * window(halo) + (p.count > kBlock ? sizeof(double) * 4 * kRedEntries : size_t(0));
     };
     int64_t halo = d.off[nd - 1];
-    if (halo > piece || halo > kPersistThreads / 2 || total(halo) > kFactoredLds)
+    if (halo > piece || halo > kPersistThreads / 2 || total(halo) > kPersistLds)
     {
         halo = d.off[nd - 2];
         s.far = true;
-        if (halo > piece || total(halo) > kFactoredLds) return false;
+        if (halo > piece || total(halo) > kPersistLds) return false;
     }
     s.halo = static_cast<int>(halo);
     s.window = window(halo);
@@ -373,7 +370,6 @@ int factored_run(pm_workspace* ws, const PersistProblem& p, int64_t max_iteratio
     a.refresh = p.refresh;
     a.chunk = p.chunk;
     a.grow = p.grow ? 1 : 0;
-    a.span = shape.span;
     a.window = static_cast<int>(shape.window);
     return persist_loop<S>(ws, p, a, kernel, shape.blocks, shape.lds, max_iterations, stream, outcome, next, state, 4);
 }

@@ -1063,7 +1063,7 @@ __global__ __launch_bounds__(kBlock) void k_invert_order(int64_t n, const unsign
 
 // rhs_p = -g_p + sum over the primary's cross blocks in (primary, eliminated)
 // order of W C^-1 g_e (block_schur.cpp:158-181), the products precomputed by
-// k_cross_rhs; the ordered sum loads kRhsBatch products ahead of the adds.
+// k_cross_rhs or k_transform_rhs.
 // A workgroup per primary: all its products come into LDS with coalesced loads in
 // flight together, and ps lanes add them in order.  (A thread per rhs entry kept 188
 // wavefronts waiting for batches of 64 gathers: 12.7 us for 60 primaries, 37 for
