@@ -452,6 +452,10 @@ def run_poisson(args, torch, capi, generators):
         solve()
     solve_ms, rep = _median_ms(solve, max(args.steps, 3))
     form = ws.solver_form
+    one_launch = ws.solver_one_launch == 1
+    kernels = {1: "k_cg_fused_dia", 2: "k_cg_step + k_cg_spmv", 3: "k_direction + k_spmv_den + k_update"}[form]
+    if one_launch:
+        kernels = {1: "k_cg_persist", 2: "k_cg_csr"}[form] + ", one launch per solve"
     relres = capi.true_relres(a, b, x, ws)
     it_bytes = pcg_iteration_bytes(n, nnz, value_bytes=8, index_bytes=4 if a.row_offsets32 is not None else 8,
                                    form=form)
@@ -476,11 +480,10 @@ def run_poisson(args, torch, capi, generators):
                                   "to relres 1e-8, max 2000", "rows": n, "nnz": nnz, "triplets": t_count},
                      {"bound": "hbm", "achieved": round(it_bytes / (it_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                       "unit": "GB/s", "frac": round(it_bytes / (it_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                      "traffic": None, "kernel": {1: "PCG iteration (k_cg_fused_dia)", 2: "PCG iteration (k_cg_step + k_cg_spmv)",
-                                 3: "PCG iteration (k_direction + k_spmv_den + k_update)"}[form],
+                      "traffic": None, "kernel": f"PCG iteration ({kernels})",
                       "bytes_per_launch": it_bytes, "ms_per_launch": round(it_ms, 5),
-                      "note": f"latency-bound: {it_bytes / 1e6:.1f} MB per iteration in the per-kernel form; "
-                              "one launch per solve keeps them on the CUs"},
+                      "note": f"latency-bound: {it_bytes / 1e6:.1f} MB per iteration in the per-kernel form"
+                              + ("; one launch per solve keeps them on the CUs" if one_launch else "")},
                      cpu)
     line["solve"] = {"converged": rep.converged, "iterations": rep.iterations, "true_relres": relres}
     line["coo_to_csr"] = {"ms_steady": round(conv_ms, 4), "ms_synchronous": round(sync_ms, 4),
