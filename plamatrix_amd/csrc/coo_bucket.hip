@@ -585,6 +585,8 @@ __global__ __launch_bounds__(kThreads) void k_bucket_unpack(CooBuckets b, Tables
     }
 }
 
+// `bytes`: the most that any conversion asks of the kernel (the limit belongs to the
+// process, and another thread's conversion may need more than this one).
 template <typename K>
 int allow_lds(K kernel, size_t bytes)
 {
@@ -658,8 +660,9 @@ int coo_bucket_prepare(const CooBuckets& b, const int64_t* r, const int64_t* c, 
     PM_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_bucket_columns, dim3(ceil_div(p.buckets, kWave)), dim3(kThreads), 0, stream, b, t);
     PM_HIP(hipGetLastError());
-    const size_t lds = sizeof(unsigned) * p.buckets + sizeof(unsigned short) * p.buckets * kWaves;
-    PM_TRY(allow_lds(k_bucket_partition, lds));
+    constexpr size_t per_bucket = sizeof(unsigned) + sizeof(unsigned short) * kWaves;
+    const size_t lds = per_bucket * p.buckets;
+    PM_TRY(allow_lds(k_bucket_partition, per_bucket * kBucketsMost));
     hipLaunchKernelGGL(k_bucket_partition, dim3(p.tiles), dim3(kThreads), lds, stream, b, t, bits_for(p.buckets));
     PM_HIP(hipGetLastError());
     PM_TRY(allow_lds(k_bucket_sort, sizeof(SortLds)));
@@ -677,7 +680,7 @@ int coo_bucket_finish(const CooBuckets& b, const S* v, int check_finite, int64_t
     auto* fold = k_bucket_fold<S>;
     const int room = static_cast<int>((most + 255) / 256 * 256);
     const size_t lds = (sizeof(S) + sizeof(unsigned)) * room;
-    PM_TRY(allow_lds(fold, lds));
+    PM_TRY(allow_lds(fold, (sizeof(S) + sizeof(unsigned)) * kBucketCap));
     hipLaunchKernelGGL(fold, dim3(b.plan.buckets), dim3(kThreads), lds, stream, b, tables(b),
                        b.plan.tiles == 0 ? b.words : b.keys, v, check_finite, capacity, row_offsets, cols, vals, room);
     PM_HIP(hipGetLastError());

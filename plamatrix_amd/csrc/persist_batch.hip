@@ -596,7 +596,7 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         int halo = 0;
         for (const TeamTask& t : launches[k]) halo = std::max(halo, t.team > 1 ? t.halo : 0);
         const size_t lds = team_lds(es, rows_per_lane, halo);
-        PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        PM_TRY(persist_allow_lds(kernel));
         a.tasks = ctl->tasks;
         a.ctl = ctl;
         a.tag = ws->teams_tag;
@@ -633,7 +633,7 @@ int teams_run(pm_workspace* ws, const BatchTeams& b, const std::vector<BatchLook
         tasks += alone[k].size();
         const void* one = team_kernel<S, I>(1 << k);
         const size_t lds = team_lds(es, 1 << k, 0);
-        PM_HIP(hipFuncSetAttribute(one, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        PM_TRY(persist_allow_lds(one));
         void* args[] = {&a};
         PM_HIP(hipLaunchKernel(one, dim3(static_cast<unsigned>(alone[k].size())), dim3(kPersistThreads), args, lds, stream));
     }

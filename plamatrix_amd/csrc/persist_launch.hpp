@@ -97,6 +97,14 @@ inline bool persist_refused(hipError_t err, pm_workspace* ws)
     return true;
 }
 
+// The limit of a kernel's LDS belongs to the process: always the same, whatever another
+// thread's launch of the kernel needs.
+inline int persist_allow_lds(const void* kernel)
+{
+    PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kPersistLds)));
+    return PM_OK;
+}
+
 // Launch `number` of a call.
 inline hipError_t persist_launch(const void* kernel, int blocks, void** args, size_t lds, hipStream_t stream, int64_t number)
 {
@@ -119,7 +127,7 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
                  int vectors = 2)
 {
     *outcome = kPersistAbandoned;
-    PM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    PM_TRY(persist_allow_lds(kernel));
     const size_t words = static_cast<size_t>(p.rows) * Exchange<S>::kWords;
     const size_t control = (sizeof(PersistControl) + 255) & ~size_t(255);
     const size_t need = control + static_cast<size_t>(vectors) * words * sizeof(word);

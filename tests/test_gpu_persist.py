@@ -293,7 +293,7 @@ def form_solve(form, dev):
     elif form == "small":
         h = generators.laplacian2d_csr(45, 37)
     else:
-        h = matrix(*{"dia": ("laplace", (300, 290), np.float64), "factored": ("diffusion", (41, 43, 40), np.float32)}[form])
+        h = matrix(*{"dia": ("laplace", (300, 290), np.float64), "wide": ("laplace", (1000, 70), np.float64), "factored": ("diffusion", (41, 43, 40), np.float32)}[form])
     a = capi.to_device_csr(h, compact=True)
     b = torch.from_numpy(generators.rhs_normal(a.rows, seed=41).astype(h.values.dtype)).to(dev)
     graph = None
@@ -465,10 +465,11 @@ def test_one_workgroup_sizes(dev, monkeypatch, index):
         assert out["0"] == out["1"]
 
 
-@pytest.mark.parametrize("forms", [("dia", "csr"), ("dia", "dia"), ("factored", "dia"), ("csr", "factored"), ("small", "dia")])
+@pytest.mark.parametrize("forms", [("dia", "csr"), ("dia", "dia"), ("factored", "dia"), ("csr", "factored"), ("small", "dia"), ("dia", "wide")])
 def test_two_solves_at_once(dev, forms):
     # two threads, each with its stream and workspace: launches of both may be queued
-    # together, and neither waits for the other's workgroups
+    # together, and neither waits for the other's workgroups ("dia" and "wide": one kernel
+    # with different amounts of LDS)
     import threading
 
     runs = [form_solve(form, dev) for form in forms]
