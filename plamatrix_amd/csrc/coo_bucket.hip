@@ -600,7 +600,8 @@ int allow_lds(K kernel, size_t bytes)
 // Buckets of 2^shift rows, the most that keep the mean at kBucketMean and a local
 // key in 32 bits (and kBucketRowBits): uneven rows may then be 2.7 times the mean
 // before a bucket outgrows its workgroup (the conversion then pays the partition's
-// counts and goes on in the LSD sort).  Longer rows, wider keys and more than kBucketsMost
+// counts and goes on in the LSD sort: 100,000 triplets 184 us against 154 by the sort
+// alone, 5.76 M 752 against 700).  Longer rows, wider keys and more than kBucketsMost
 // buckets stay on the LSD sort.
 //
 // Smaller conversions are cut finer, towards a bucket per CU but not below
