@@ -49,13 +49,19 @@ inline bool persist_enabled()
 // What a test asks of the launches in PLAMATRIX_AMD_PERSIST_TEST, a list of
 // name=number: the number, or `none`.  refuse=k, too_large=k: launch k of a call is
 // turned down with that error; give_up=k: its workgroups find a notice to give up;
-// storage=0: there is no memory for the exchange; segment=n: launches of n (even)
-// iterations; tag=n: the last exchange tag used.
+// storage=0: there is no memory for the exchange; segment=n: launches of n iterations
+// (even, or one less); tag=n: the last exchange tag used.
 inline int64_t persist_test(const char* name, int64_t none)
 {
     const char* env = std::getenv("PLAMATRIX_AMD_PERSIST_TEST");
     const char* at = env != nullptr ? std::strstr(env, name) : nullptr;
     return at != nullptr ? std::atoll(at + std::strlen(name)) : none;
+}
+
+// Iterations of a launch.
+inline int64_t persist_segment(int64_t most)
+{
+    return std::max<int64_t>(2, persist_test("segment=", most) & ~int64_t(1));
 }
 
 // Storage that only the one-launch forms need: without it a solve takes the kernels.
@@ -135,7 +141,7 @@ int persist_loop(pm_workspace* ws, const PersistProblem& p, Args& a, const void*
     if (!persist_storage(ws->persist, need)) return PM_OK;
     if (grown) ws->persist_tag = kLastTag;
     else ws->persist_tag = static_cast<uint32_t>(persist_test("tag=", ws->persist_tag));
-    const int64_t segment = persist_test("segment=", kSegment);
+    const int64_t segment = persist_segment(kSegment);
     a.ctl = ws->persist.as<PersistControl>();
     a.xu = reinterpret_cast<word*>(ws->persist.as<char>() + control);
     a.xx = a.xu + words;

@@ -288,7 +288,7 @@ int small_run(pm_workspace* ws, const PersistProblem& p, const I* ro, const I* c
     a.grow = p.grow ? 1 : 0;
     const void* kernel = small_kernel<S, I>(static_cast<int>(ceil_div(p.count, kSmallGroups)), p.jacobi);
     *outcome = kPersistAbandoned;
-    const int64_t segment = persist_test("segment=", kSmallSegment);
+    const int64_t segment = persist_segment(kSmallSegment);
     for (int64_t t = 0;;)
     {
         // an even number of iterations, the last one's decision included
