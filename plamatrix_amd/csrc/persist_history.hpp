@@ -50,7 +50,9 @@ struct PersistHistory
         h.tol = d.tol;
         h.gamma_prev = gamma;
         h.den_prev = d.den;
-        if (d.restart && over == 0)
+        // one thread decides while the others wait: the rare branch out of its way (0.2 %
+        // of a 767-iteration solve)
+        if (__builtin_expect(d.restart, 0) && over == 0)
         {
             const int64_t at = hand_over_iteration(t, chunk, grow, kMaxGrownChunk);
             over = at < INT32_MAX ? static_cast<int>(at) : INT32_MAX;
